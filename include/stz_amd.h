@@ -127,7 +127,11 @@ typedef struct stz_mg_config {
                                     the 64x65 level of a 1024^2 grid; levels
                                     of even width up to 128 and at most 72
                                     rows qualify); 0: the V-cycle runs to the
-                                    coarsest level, solved exactly */
+                                    coarsest level, solved exactly.  With
+                                    direct_nodes > 0 most grids need no
+                                    V-cycle at all: the top level itself is
+                                    solved directly (Fourier modes along x,
+                                    block recurrences along y, FP64) */
     int32_t predict_unit;        /* 0: after a failed test run k more cycles
                                     (k = 1, 2, 3, ...) before the next, as
                                     tgmg.in.cc:282-292 (default); 1: one more
@@ -140,9 +144,13 @@ typedef struct stz_mg_config {
 /* Result of the last projection solve. */
 typedef struct stz_solve_info {
     int32_t status;              /* STZ_OK / STZ_ERR_NOT_CONVERGED / STZ_ERR_NAN */
-    int32_t cycles;              /* V-cycles counted as tgmg_predict does */
-    int32_t total_cycles;        /* V-cycles actually run (incl. extra) */
-    int32_t refinements;         /* FP64 residual evaluations (mixed mode) */
+    int32_t cycles;              /* V-cycles counted as tgmg_predict does; of a
+                                    direct solve, corrections after its first
+                                    test (0 as a rule) */
+    int32_t total_cycles;        /* V-cycles actually run (incl. extra), or
+                                    direct solves */
+    int32_t refinements;         /* FP64 residual evaluations (mixed mode,
+                                    V-cycles) */
     double residual;             /* mean-square residual (tgmg.hh:146) */
     double tolerance;            /* threshold it was compared against */
 } stz_solve_info;

@@ -31,6 +31,7 @@ struct EnsState {
     int resid;                 // 1 if the slot's cycle is followed by a residual evaluation
     int cycles_run, solves, vcount;
     int status;        // STZ_OK, STZ_ERR_NOT_CONVERGED, STZ_ERR_NAN
+    int direct;        // 1: the member's solves go through mg_fourier.hip
 };
 
 // predictor settings shared by all members (tgmg_config.hh:26-45)
@@ -86,6 +87,17 @@ template <typename T> struct DirectEntry {
     double *D;     // the level's mode inverses, twiddles and mode scratch (FP64)
     const T *b;
     T *z;
+};
+
+// one member's direct solve (mg_fourier.hip) and the residual test after it
+struct FourierEntry {
+    int member, gx;
+    FourierArgs a;
+    const double *src;
+    double *z;
+    double *r;          // FP64 residual, the source of a correction
+    LevelArgs<double> L;
+    double *partial;
 };
 
 // workgroup-partial sums of one member's residual
@@ -147,6 +159,19 @@ int direct_inverse_workgroups(int M, int Nn);
 template <typename T> int batch_set_lds_limit(size_t bytes);
 // fp64: |r|^2 partials of the top level, blocks as mg_resid_norm
 int batch_resid_norm(const RefineEntry *E, const int *map, int ne, int total, const EnsState *S, hipStream_t st);
+
+// direct solves: the row launches of members of one row variant (M any of
+// theirs), the mode launch of members of one column variant; the residual
+// (`store`: of the members about to correct, kept) and its norm
+int fourier_row_workgroups(int N);
+int fourier_row_variant(int M);
+int fourier_mode_variant(int N);
+size_t fourier_row_lds(int M);
+int batch_fourier_rows(bool inverse, int M, size_t lds, const FourierEntry *E, const int *map, int total,
+                       const EnsState *S, hipStream_t st);
+int batch_fourier_modes(int N, const FourierEntry *E, const int *map, int total, const EnsState *S, hipStream_t st);
+int batch_resid_test(bool store, int sparse, const FourierEntry *E, const int *map, int total, const EnsState *S,
+                     hipStream_t st);
 
 // the per-member V-cycle count (mg.hip): mode 0 starts a solve, mode 1
 // follows a cycle slot, mode 2 marks corrected members

@@ -65,6 +65,19 @@ template <typename T> struct VCyclePlan {
     size_t dlds = 0;
 };
 
+// the launches of the members that solve directly: row and mode launches by
+// kernel variant (`size`: M or N of a member), and the residual test of all
+struct FourierLaunch {
+    int size = 0;
+    size_t lds = 0;
+    DevTable<FourierEntry> t;
+};
+struct FourierPlan {
+    std::vector<FourierLaunch> rows, modes;
+    DevTable<FourierEntry> test;
+    int sparse = 0;
+};
+
 }  // namespace
 
 struct stz_ensemble {
@@ -87,6 +100,7 @@ struct stz_ensemble {
     int top_sparse = 0;
     VCyclePlan<double> plan64;
     VCyclePlan<float> plan32;
+    FourierPlan fplan;
     EnsPredict pred{};
     // state: device array and a pinned host copy
     EnsState *dst = nullptr, *hst = nullptr;
@@ -113,6 +127,7 @@ struct stz_ensemble {
         bufs.clear();
         plan64 = VCyclePlan<double>();
         plan32 = VCyclePlan<float>();
+        fplan = FourierPlan();
         tuned[0] = tuned[1] = 0;
         built = false;
     }
@@ -202,6 +217,8 @@ int build_plan(stz_ensemble *e, VCyclePlan<T> &P, DevMG<T> stz_sim::*mgp, bool t
     for (int k = 0; k < e->nmem(); k++) {
         stz_sim *s = e->mem[k];
         DevMG<T> &mg = s->*mgp;
+        const bool direct_solve = fourier_active(s);
+        if (!direct_solve && (rc = mg_ensure_direct(s))) return rc;
         CoarseArgs<T> A = mg.args;
         A.nu1 = e->cfg.nu1;
         A.nu2 = e->cfg.nu2;
@@ -213,6 +230,7 @@ int build_plan(stz_ensemble *e, VCyclePlan<T> &P, DevMG<T> stz_sim::*mgp, bool t
             set_error("%s", msg);
             return rc;
         }
+        if (direct_solve) continue;
         for (const TileRec<T> &r : recs) {
             const int lk = r.phase == 0 ? r.level : -r.level;  // up: deeper levels first
             groups[Pos(r.phase, lk, r.index)].push_back({r, k});
@@ -318,6 +336,54 @@ int build_plan(stz_ensemble *e, VCyclePlan<T> &P, DevMG<T> stz_sim::*mgp, bool t
     return batch_set_lds_limit<T>(lds);
 }
 
+// the launches of the members that solve directly
+int build_fourier(stz_ensemble *e) {
+    FourierPlan &P = e->fplan;
+    std::map<int, std::vector<FourierEntry>> rows, modes;
+    std::vector<FourierEntry> all;
+    std::vector<int> wtest;
+    int rc;
+    for (int k = 0; k < e->nmem(); k++) {
+        stz_sim *s = e->mem[k];
+        if (!fourier_active(s)) continue;
+        FourierEntry f;
+        std::memset(&f, 0, sizeof f);
+        f.member = k;
+        f.a = s->fa;
+        f.src = s->src;
+        f.z = s->vel;
+        f.r = s->mg64.args.lv[0].z2;
+        f.L = s->top64();
+        f.gx = (f.L.m + 63) / 64;
+        f.partial = s->partial;
+        rows[fourier_row_variant(f.a.M)].push_back(f);
+        modes[fourier_mode_variant(f.a.N)].push_back(f);
+        all.push_back(f);
+        wtest.push_back(mg_refine_blocks(f.L));
+        P.sparse = f.L.sparse;  // fourier_setup takes the top-level pattern only
+    }
+    for (auto &g : rows) {
+        FourierLaunch l;
+        l.size = g.second[0].a.M;
+        std::vector<int> w;
+        for (auto &f : g.second) {
+            w.push_back(fourier_row_workgroups(f.a.N));
+            l.lds = std::max(l.lds, fourier_row_lds(f.a.M));
+        }
+        if ((rc = make_table(e, g.second, w, l.t))) return rc;
+        P.rows.push_back(l);
+    }
+    for (auto &g : modes) {
+        FourierLaunch l;
+        l.size = g.second[0].a.N;
+        std::vector<int> w;
+        for (auto &f : g.second) w.push_back(f.a.M / 2 + 1);
+        if ((rc = make_table(e, g.second, w, l.t))) return rc;
+        P.modes.push_back(l);
+    }
+    return make_table(e, all, wtest, P.test);
+}
+
 int build_tables(stz_ensemble *e, double dt) {
     e->free_tables();
     int rc;
@@ -388,6 +454,11 @@ int build_tables(stz_ensemble *e, double dt) {
         NormEntry ne;
         ne.member = k;
         ne.partial = s->partial;
+        if (fourier_active(s)) {
+            ne.np = mg_refine_blocks(t);
+            norms.push_back(ne);
+            continue;
+        }
         if (e->precision == STZ_PREC_MIXED) {
             // mg_refine's grid: 64 x 16 tiles
             re.gx = (t.m + 63) / 64;
@@ -431,6 +502,7 @@ int build_tables(stz_ensemble *e, double dt) {
         if (!rc) {
             if (e->precision == STZ_PREC_MIXED) rc = build_plan<float>(e, e->plan32, &stz_sim::mg32, true);
             else rc = build_plan<double>(e, e->plan64, &stz_sim::mg64, false);
+            if (!rc) rc = build_fourier(e);
         }
         for (int k = 0; k < N; k++)
             if (hipMemcpyAsync(e->mem[k]->vel, keep + off[k], (off[k + 1] - off[k]) * sizeof(double),
@@ -478,9 +550,27 @@ template <typename T> int launch_vcycle(stz_ensemble *e, const VCyclePlan<T> &P)
     return STZ_OK;
 }
 
+// the direct solves of a slot: the residual of members past their first
+// test, the solve, the test
+int launch_fourier(stz_ensemble *e) {
+    const FourierPlan &P = e->fplan;
+    const DevTable<FourierEntry> &T = P.test;
+    hipStream_t st = e->stream;
+    int rc;
+    if ((rc = batch_resid_test(true, P.sparse, T.E, T.map, T.total, e->dst, st))) return rc;
+    for (const FourierLaunch &l : P.rows)
+        if ((rc = batch_fourier_rows(false, l.size, l.lds, l.t.E, l.t.map, l.t.total, e->dst, st))) return rc;
+    for (const FourierLaunch &l : P.modes)
+        if ((rc = batch_fourier_modes(l.size, l.t.E, l.t.map, l.t.total, e->dst, st))) return rc;
+    for (const FourierLaunch &l : P.rows)
+        if ((rc = batch_fourier_rows(true, l.size, l.lds, l.t.E, l.t.map, l.t.total, e->dst, st))) return rc;
+    return batch_resid_test(false, P.sparse, T.E, T.map, T.total, e->dst, st);
+}
+
 int launch_slot(stz_ensemble *e) {
     int rc;
     hipStream_t st = e->stream;
+    if ((rc = launch_fourier(e))) return rc;
     const DevTable<RefineEntry> &R = e->refs;
     if (e->precision == STZ_PREC_MIXED) {
         // vel += e is applied by the top level's last smoothing launch
@@ -581,8 +671,9 @@ bool in_progress(const EnsState &s) { return s.phase == ENS_FIRST || s.phase == 
 // cycles the predictor of a member will run if its first test passes
 int planned_slots(const stz_ensemble *e) {
     int most = 0;
-    for (int k = 0; k < e->nmem(); k++) most = std::max(most, e->mem[k]->lim / e->pred.mult);
-    return most + e->pred.extra;
+    for (int k = 0; k < e->nmem(); k++)
+        most = std::max(most, fourier_active(e->mem[k]) ? 1 : e->mem[k]->lim / e->pred.mult + e->pred.extra);
+    return most;
 }
 
 }  // namespace
@@ -711,6 +802,7 @@ int stz_ensemble_step_quasistatic(stz_ensemble *e, double dt, int nsteps) {
         h.solves = s->solves;
         h.vcount = s->vcount;
         h.phase = ENS_CORRECTED;
+        h.direct = fourier_active(s) ? 1 : 0;
     }
     STZ_HIP(hipMemcpyAsync(e->dst, e->hst, N * sizeof(EnsState), hipMemcpyHostToDevice, e->stream));
     int status = STZ_OK;
@@ -753,7 +845,7 @@ int stz_ensemble_step_quasistatic(stz_ensemble *e, double dt, int nsteps) {
             s->last.status = h.status;
             s->last.cycles = h.n;
             s->last.total_cycles = h.cycles_run;
-            s->last.refinements = e->precision == STZ_PREC_MIXED ? h.cycles_run : 0;
+            s->last.refinements = e->precision == STZ_PREC_MIXED && !h.direct ? h.cycles_run : 0;
             s->last.residual = h.acc;
             s->last.tolerance = h.tol;
             if (h.status != STZ_OK && status == STZ_OK) {

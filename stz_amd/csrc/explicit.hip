@@ -612,8 +612,13 @@ __device__ __forceinline__ static void correct_body(const SimConst &c, const Fie
     PL(f.s, i, j) = s;
     PL(f.tau, i, j) = t;
 }
+// gate: launched ahead of the host's reading of a convergence test, the
+// correction runs only if the test's sum of squares passes it on the device
+// too (denom nodes, threshold tol)
 __global__ void __launch_bounds__(256) correct_kernel(SimConst c, FieldPtrs f, const double *vel, double dt,
-                                                      double bvel, double bpos) {
+                                                      double bvel, double bpos, const double *gate, double denom,
+                                                      double tol) {
+    if (gate && !(*gate / denom < tol)) return;
     int bx, by;
     xcd_band_tile(bx, by);
     correct_body(c, f, vel, dt, bvel, bpos, bx, by);
@@ -718,9 +723,9 @@ int launch_source(const SimConst &c, const FieldPtrs &f, double dt, double xbc, 
 }
 
 int launch_correct(const SimConst &c, const FieldPtrs &f, const double *vel, double dt, double bvel, double bpos,
-                   hipStream_t st) {
+                   hipStream_t st, const double *gate, double denom, double tol) {
     dim3 b(64, 4);
-    hipLaunchKernelGGL(correct_kernel, grid2(c.m, c.n, b), b, 0, st, c, f, vel, dt, bvel, bpos);
+    hipLaunchKernelGGL(correct_kernel, grid2(c.m, c.n, b), b, 0, st, c, f, vel, dt, bvel, bpos, gate, denom, tol);
     STZ_HIP(hipGetLastError());
     return STZ_OK;
 }

@@ -70,6 +70,24 @@ bool direct_inverse(const double *S, int M, int Nn, std::vector<double> &D);
 // within the launches' fixed register and LDS tiles)
 bool direct_fits(int M, int Nn);
 
+// mg_fourier.hip: direct solve of the top level's operator, FP64.  M nodes
+// per row, N interior rows; tw the M roots of unity and tab the modes'
+// constants (fourier_setup fills both, in this order), S the spectrum
+struct FourierArgs {
+    int M, N, nst;
+    int radix[16];
+    double cxx, cyy, cxy;  // a wall node's weight in the row next to it: u, v, and u-v through the corners
+    double wix, wiy;       // inverse diagonal of the wall rows
+    const double *tw, *tab;
+    double *S;
+};
+// whether the launches cover M nodes per row and n node rows
+bool fourier_fits(int M, int n);
+size_t fourier_spectrum_elems(int M, int N);
+bool fourier_setup(const double *s40, const double *w40, int M, int N, FourierArgs &a, std::vector<double> &T);
+int fourier_set_lds_limit(const FourierArgs &a);
+int mg_fourier_solve(const FourierArgs &a, const double *src, double *z, bool add, hipStream_t st);
+
 // LDS layout for levels lc..L-1; returns the number of elements of T
 template <typename T> int coarse_layout(CoarseArgs<T> &A);
 // host: the constant part of the layout, to be uploaded as A.pack.  S[l] are
@@ -95,7 +113,8 @@ template <typename T> int mg_set_lds_limit(size_t bytes);
 int mg_resid64_to32(const LevelArgs<double> &L, float *b32, float *z32, double *partial, double *out,
                     hipStream_t st);
 int mg_correct64(double *z, const float *e, int count, hipStream_t st);
-int mg_sum_partials(const double *partial, int np, double *out, hipStream_t st);
+// out2: a second place for the sum, or null
+int mg_sum_partials(const double *partial, int np, double *out, hipStream_t st, double *out2 = nullptr);
 template <typename T> int mg_fill_zero(T *p, size_t count, hipStream_t st);
 
 // tiled path (mg_tiled.hip)
@@ -123,5 +142,9 @@ template <typename T> int mg_smooth_level(LevelArgs<T> &L, int sweeps, hipStream
 // (out == nullptr: partials only)
 int mg_refine(const LevelArgs<double> &L, float *b32, double *partial, double *out, hipStream_t st);
 int mg_refine_blocks(const LevelArgs<double> &L);
+// |b - A z|^2 of the FP64 top level summed to *out and *out2; with r, the
+// residual itself is stored there too
+int mg_resid_test(const LevelArgs<double> &L, double *r, double *partial, double *out, double *out2,
+                  hipStream_t st);
 
 }  // namespace stz

@@ -110,9 +110,13 @@ __device__ __forceinline__ static double sum_partials_body(const double *partial
     return (ws[0] + ws[1]) + (ws[2] + ws[3]);  // valid in thread 0
 }
 
-__global__ void __launch_bounds__(256) sum_partials_kernel(const double *partial, int np, double *out) {
+__global__ void __launch_bounds__(256) sum_partials_kernel(const double *partial, int np, double *out,
+                                                           double *out2) {
     const double v = sum_partials_body(partial, np);
-    if (threadIdx.x == 0) *out = v;
+    if (threadIdx.x == 0) {
+        *out = v;
+        if (out2) *out2 = v;
+    }
 }
 
 // mixed precision: FP64 residual of the top level -> FP32 source of the
@@ -780,7 +784,7 @@ template <typename T> int mg_coarse(const CoarseArgs<T> &A, hipStream_t st) {
 template <typename T> int mg_resid_norm(const LevelArgs<T> &L, double *partial, double *out, hipStream_t st) {
     const int nb = (L.m * L.n + 255) / 256;
     hipLaunchKernelGGL(resid_norm_kernel<T>, dim3(nb), dim3(256), 0, st, L, partial);
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, nb, out);
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, nb, out, (double *)nullptr);
     STZ_HIP(hipGetLastError());
     return STZ_OK;
 }
@@ -789,7 +793,7 @@ int mg_resid64_to32(const LevelArgs<double> &L, float *b32, float *z32, double *
                     hipStream_t st) {
     const int nb = (L.m * L.n + 255) / 256;
     hipLaunchKernelGGL(resid64_to32_kernel, dim3(nb), dim3(256), 0, st, L, b32, z32, partial);
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, nb, out);
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, nb, out, (double *)nullptr);
     STZ_HIP(hipGetLastError());
     return STZ_OK;
 }
@@ -802,8 +806,8 @@ template <typename T> int mg_fill_zero(T *p, size_t count, hipStream_t st) {
 template int mg_fill_zero<double>(double *, size_t, hipStream_t);
 template int mg_fill_zero<float>(float *, size_t, hipStream_t);
 
-int mg_sum_partials(const double *partial, int np, double *out, hipStream_t st) {
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, np, out);
+int mg_sum_partials(const double *partial, int np, double *out, hipStream_t st, double *out2) {
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, np, out, out2);
     STZ_HIP(hipGetLastError());
     return STZ_OK;
 }
@@ -960,6 +964,32 @@ __device__ static void ens_resolve(EnsState &st, double acc, const EnsPredict &P
     }
 }
 
+// the same for a member that solves directly (mg_fourier.hip): the first
+// test follows the solve, and every failed test asks for one correction
+// (fourier_solve in sim.hip)
+__device__ static void ens_resolve_direct(EnsState &st, double acc, const EnsPredict &P) {
+    st.acc = acc;
+    if (st.phase == ENS_FIRST ? acc < st.tol : !(acc >= st.tol)) {
+        if (st.phase == ENS_FIRST && st.lim > 0) st.lim -= 1 + st.lim / P.decay;
+    } else {
+        st.lim += P.mult;
+        if (st.lim > P.max_thresh) {
+            st.phase = ENS_FAILED;
+            st.status = STZ_ERR_NOT_CONVERGED;
+            st.active = 0;
+            return;
+        }
+        st.n++;
+        st.phase = ENS_LOOP;
+        return;
+    }
+    st.phase = ENS_DONE;
+    st.active = 0;
+    st.solves++;
+    st.vcount += st.n;
+    st.status = isnan(acc) ? STZ_ERR_NAN : STZ_OK;
+}
+
 // one workgroup per member: mode 0 starts the solve from the residual of the
 // step's first evaluation, mode 1 counts the slot's cycle of every member
 // that ran it and tests its residual, mode 2 marks members corrected
@@ -972,8 +1002,23 @@ __global__ void __launch_bounds__(256) control_batch_kernel(EnsState *S, const N
         return;
     }
     if (mode == 1 && !st.active) return;
+    if (st.direct && mode == 0) {
+        if (threadIdx.x == 0) {
+            st.n = st.k = st.remaining = st.cycles_run = 0;
+            st.phase = ENS_FIRST;
+            st.status = STZ_OK;
+            st.active = 1;
+            st.resid = 0;
+        }
+        return;
+    }
     const double sum = sum_partials_body(x.partial, x.np);
     if (threadIdx.x != 0) return;
+    if (st.direct) {
+        st.cycles_run++;
+        ens_resolve_direct(st, sum / st.denom, P);
+        return;
+    }
     if (mode == 0) {
         st.n = st.lim / P.mult;
         st.k = 0;

@@ -1,0 +1,824 @@
+// mg_fourier.hip -- direct solve of the projection's top-level operator.
+//
+// qs_multi's operator (qs_multi.hh:30-50, qs_multi.cc:31-54) does not depend
+// on x, which is periodic, and away from the two wall rows not on y either.
+// A discrete Fourier transform along x therefore leaves, for each mode
+// k = 0..M/2, a block tridiagonal Toeplitz system over the N = n - 1 interior
+// rows whose 2x2 blocks are real once the transverse velocity is written
+// v = i v':
+//     Cd w_{j-1} + B w_j + Cu w_{j+1} = f_j,   w = (u, v'),  Cd = Cu^T.
+// With D the limit of the elimination D -> B - Cd D^{-1} Cu the system factors
+// as T = L U + E1 P E1^T, L and U bidiagonal with constant blocks and
+// P = B - D acting on the first row only, so one solve is a forward and a
+// backward recurrence with constant coefficients F = -Cd D^{-1} and
+// E = -D^{-1} Cu = F^T, and the first row's rank-two term:
+//     g_j = f_j + F g_{j-1},  y_j = D^{-1} g_j + E y_{j+1}   (y = M^{-1} f)
+//     w_1 = (I + G P)^{-1} y_1,  w = M^{-1}(f - E1 P w_1),   G = (M^{-1})_11.
+// Constant coefficients make both recurrences scans: each lane of a mode's
+// workgroup runs P rows, and the carries combine through F^P, F^2P, F^4P, ...
+// Per mode the host forms D, F, the powers and P (I + G P)^{-1} in extended
+// precision (the limit by cyclic reduction, which converges quadratically;
+// mode 0 in closed form: D = -Cu, F = I).  In FP64 the result is at the
+// rounding floor: the residual is 1e-16 of the source on every size from 8^2
+// to 1024^2, so one application replaces all V-cycles of a solve.
+//
+// Three launches:
+//   forward   R rows per workgroup: u + i v of a row as one complex signal,
+//             an in-LDS Stockham transform, the two real signals' modes
+//             separated on the way out
+//   modes     one workgroup per mode, the column in LDS
+//   inverse   R rows per workgroup, back to (u, v)
+// The spectrum is kept mode-major, S[k][j] of 32 bytes (u, v' complex), so
+// the mode launch reads and writes whole columns and a row workgroup touches
+// R * 32 contiguous bytes per mode.
+#include <hip/hip_runtime.h>
+
+#include <cmath>
+#include <type_traits>
+#include <vector>
+
+#include "batch.h"
+#include "device.h"
+#include "mg.h"
+#include "mg_node.h"
+
+namespace stz {
+
+// ---------------------------------------------------------------------------
+// the row transform
+// ---------------------------------------------------------------------------
+constexpr int kRowThreads = 256;
+constexpr int kRows = 2;           // rows per workgroup of the row launches
+
+struct alignas(16) cplx { double x, y; };
+
+__device__ __forceinline__ static cplx operator+(const cplx &a, const cplx &b) { return {a.x + b.x, a.y + b.y}; }
+__device__ __forceinline__ static cplx operator-(const cplx &a, const cplx &b) { return {a.x - b.x, a.y - b.y}; }
+__device__ __forceinline__ static cplx cmul(const cplx &a, const cplx &b) {
+    return {fmav(a.x, b.x, -(a.y * b.y)), fmav(a.x, b.y, a.y * b.x)};
+}
+__device__ __forceinline__ static cplx mul_mi(const cplx &a) { return {a.y, -a.x}; }  // -i a
+
+// LDS position of element i: one 16-byte slot in nine is skipped, so that
+// the transform's strided writes (strides 4, 8) spread over the banks
+__host__ __device__ constexpr int fpad(int i) { return i + (i >> 3); }
+
+// forward DFTs of R values in place (e^{-2 pi i / R})
+template <int R> __device__ __forceinline__ static void dft(cplx (&x)[R]);
+template <> __device__ __forceinline__ void dft<2>(cplx (&x)[2]) {
+    const cplx a = x[0], b = x[1];
+    x[0] = a + b;
+    x[1] = a - b;
+}
+template <> __device__ __forceinline__ void dft<3>(cplx (&x)[3]) {
+    const double s = 0.86602540378443864676;  // sqrt(3)/2
+    const cplx t = x[1] + x[2], d = x[1] - x[2], a = x[0];
+    const cplx c = {fmav(-0.5, t.x, a.x), fmav(-0.5, t.y, a.y)};
+    x[0] = a + t;
+    x[1] = {fmav(s, d.y, c.x), fmav(-s, d.x, c.y)};
+    x[2] = {fmav(-s, d.y, c.x), fmav(s, d.x, c.y)};
+}
+template <> __device__ __forceinline__ void dft<4>(cplx (&x)[4]) {
+    const cplx a = x[0] + x[2], b = x[0] - x[2], c = x[1] + x[3], d = mul_mi(x[1] - x[3]);
+    x[0] = a + c;
+    x[1] = b + d;
+    x[2] = a - c;
+    x[3] = b - d;
+}
+template <> __device__ __forceinline__ void dft<5>(cplx (&x)[5]) {
+    const double c1 = 0.30901699437494742410, c2 = -0.80901699437494742410;  // cos 2 pi/5, 4 pi/5
+    const double s1 = 0.95105651629515357212, s2 = 0.58778525229247312917;   // sin
+    const cplx a = x[0], p = x[1] + x[4], q = x[2] + x[3], m = x[1] - x[4], n = x[2] - x[3];
+    const cplx u = {fmav(c2, q.x, fmav(c1, p.x, a.x)), fmav(c2, q.y, fmav(c1, p.y, a.y))};
+    const cplx v = {fmav(c1, q.x, fmav(c2, p.x, a.x)), fmav(c1, q.y, fmav(c2, p.y, a.y))};
+    const cplx f = {fmav(s1, m.x, s2 * n.x), fmav(s1, m.y, s2 * n.y)};
+    const cplx g = {fmav(s2, m.x, -(s1 * n.x)), fmav(s2, m.y, -(s1 * n.y))};
+    x[0] = a + p + q;
+    x[1] = {u.x + f.y, u.y - f.x};
+    x[4] = {u.x - f.y, u.y + f.x};
+    x[2] = {v.x + g.y, v.y - g.x};
+    x[3] = {v.x - g.y, v.y + g.x};
+}
+template <> __device__ __forceinline__ void dft<8>(cplx (&x)[8]) {
+    const double h = 0.70710678118654752440;
+    cplx e[4] = {x[0], x[2], x[4], x[6]}, o[4] = {x[1], x[3], x[5], x[7]};
+    dft<4>(e);
+    dft<4>(o);
+    const cplx o1 = {h * (o[1].x + o[1].y), h * (o[1].y - o[1].x)};
+    const cplx o2 = mul_mi(o[2]);
+    const cplx o3 = {h * (o[3].y - o[3].x), -h * (o[3].x + o[3].y)};
+    x[0] = e[0] + o[0];
+    x[4] = e[0] - o[0];
+    x[1] = e[1] + o1;
+    x[5] = e[1] - o1;
+    x[2] = e[2] + o2;
+    x[6] = e[2] - o2;
+    x[3] = e[3] + o3;
+    x[7] = e[3] - o3;
+}
+
+// One Stockham stage of radix RX for kRows rows of M values in `buf`, in
+// place: L is the product of the radices before it.  Every butterfly of a
+// thread is in registers between the two barriers, which is why M is a
+// compile-time constant here.
+template <int M, int RX, int L>
+__device__ __forceinline__ static void stage_fixed(cplx *buf, const cplx *__restrict__ tw) {
+    constexpr int NBF = kRows * (M / RX), NT = kRowThreads, Q = (NBF + NT - 1) / NT;
+    cplx x[Q][RX];
+#pragma unroll
+    for (int b = 0; b < Q; b++) {
+        const int t = threadIdx.x + NT * b;
+        if (NBF % NT == 0 || t < NBF) {
+            const int row = t / (M / RX), idx = t % (M / RX);
+#pragma unroll
+            for (int q = 0; q < RX; q++) x[b][q] = buf[row * fpad(M) + fpad(idx + q * (M / RX))];
+            if (L > 1) {
+                const int k = idx % L;
+#pragma unroll
+                for (int q = 1; q < RX; q++) x[b][q] = cmul(x[b][q], tw[k * q * (M / (L * RX))]);
+            }
+            dft<RX>(x[b]);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int b = 0; b < Q; b++) {
+        const int t = threadIdx.x + NT * b;
+        if (NBF % NT == 0 || t < NBF) {
+            const int row = t / (M / RX), idx = t % (M / RX);
+            const int o = (idx / L) * (L * RX) + idx % L;
+#pragma unroll
+            for (int q = 0; q < RX; q++) buf[row * fpad(M) + fpad(o + q * L)] = x[b][q];
+        }
+    }
+    __syncthreads();
+}
+
+// the stages of a power-of-two length: radix 8 while that leaves a multiple
+// of 4, then radix 4 and at most one radix 2
+template <int M, int L> __device__ __forceinline__ static void stages_fixed(cplx *buf, const cplx *tw) {
+    constexpr int left = M / L;
+    if constexpr (left > 1) {
+        constexpr int RX = left % 8 == 0 && left != 16 ? 8 : (left % 4 == 0 ? 4 : 2);
+        stage_fixed<M, RX, L>(buf, tw);
+        stages_fixed<M, L * RX>(buf, tw);
+    }
+}
+
+// any length: one stage from `in` to `out`, radix RX (0: the run-time radix
+// r as a plain sum per output, for the primes without a butterfly above)
+template <int RX>
+__device__ __forceinline__ static void stage_any(const cplx *in, cplx *out, const cplx *__restrict__ tw, int M,
+                                                 int L, int r) {
+    const int P = fpad(M);
+    if constexpr (RX > 0) {
+        const int nb = M / RX, step = M / (L * RX);
+        for (int t = threadIdx.x; t < kRows * nb; t += kRowThreads) {
+            const int row = t / nb, idx = t - row * nb, k = idx % L;
+            cplx x[RX];
+#pragma unroll
+            for (int q = 0; q < RX; q++) x[q] = in[row * P + fpad(idx + q * nb)];
+            if (L > 1)
+#pragma unroll
+                for (int q = 1; q < RX; q++) x[q] = cmul(x[q], tw[k * q * step]);
+            dft<RX>(x);
+            const int o = (idx - k) * RX + k;
+#pragma unroll
+            for (int q = 0; q < RX; q++) out[row * P + fpad(o + q * L)] = x[q];
+        }
+    } else {
+        const int nb = M / r, step = M / (L * r);
+        for (int t = threadIdx.x; t < kRows * M; t += kRowThreads) {
+            const int row = t / M, e = t - row * M, q = e / nb, idx = e - q * nb, k = idx % L;
+            // sum_p in[idx + p nb] w^{p (k step + q nb)}
+            const int inc = (k * step + q * nb) % M;
+            cplx s = in[row * P + fpad(idx)];
+            int w = 0;
+            for (int p = 1; p < r; p++) {
+                w += inc;
+                if (w >= M) w -= M;
+                s = s + cmul(in[row * P + fpad(idx + p * nb)], tw[w]);
+            }
+            out[row * P + fpad((idx - k) * r + k + q * L)] = s;
+        }
+    }
+}
+
+// transform the kRows rows in LDS; returns where the result is
+template <int MT>
+__device__ __forceinline__ static cplx *transform_rows(const FourierArgs &a, cplx *buf) {
+    const cplx *tw = reinterpret_cast<const cplx *>(a.tw);
+    if constexpr (MT > 0) {
+        stages_fixed<MT, 1>(buf, tw);
+        return buf;
+    } else {
+        cplx *in = buf, *out = buf + kRows * fpad(a.M);
+        int L = 1;
+        for (int s = 0; s < a.nst; s++) {
+            const int r = a.radix[s];
+            if (r == 4) stage_any<4>(in, out, tw, a.M, L, r);
+            else if (r == 2) stage_any<2>(in, out, tw, a.M, L, r);
+            else if (r == 3) stage_any<3>(in, out, tw, a.M, L, r);
+            else if (r == 5) stage_any<5>(in, out, tw, a.M, L, r);
+            else stage_any<0>(in, out, tw, a.M, L, r);
+            __syncthreads();
+            cplx *t = in;
+            in = out;
+            out = t;
+            L *= r;
+        }
+        return in;
+    }
+}
+
+// the solved value of wall node (i, row 0 or n): its row holds the diagonal only
+__device__ __forceinline__ static cplx wall_node(const FourierArgs &a, const cplx *src, int i, int j) {
+    const cplx s = src[(size_t)i + (size_t)a.M * j];
+    return {a.wix * s.x, a.wiy * s.y};
+}
+
+// forward launch body: interior rows 1 + kRows * blk .., the two rows next to
+// the walls with the wall velocity's part moved to the right-hand side
+template <int MT>
+__device__ __forceinline__ static void fourier_forward_body(const FourierArgs &a, const double *__restrict__ src2,
+                                                            int blk) {
+    extern __shared__ __align__(16) unsigned char fourier_smem[];
+    cplx *buf = reinterpret_cast<cplx *>(fourier_smem);
+    const int M = MT > 0 ? MT : a.M, N = a.N, K = M / 2 + 1;
+    const cplx *src = reinterpret_cast<const cplx *>(src2);
+    const int j0 = 1 + kRows * blk;
+    for (int t = threadIdx.x; t < kRows * M; t += kRowThreads) {
+        const int row = t / M, i = t - row * M, j = j0 + row;
+        cplx v = {0, 0};
+        if (j <= N) {
+            v = src[(size_t)i + (size_t)M * j];
+            if (j == 1 || j == N) {
+                const int il = i == 0 ? M - 1 : i - 1, ir = i == M - 1 ? 0 : i + 1;
+                if (j == 1) {
+                    const cplx c = wall_node(a, src, i, 0), l = wall_node(a, src, il, 0), r = wall_node(a, src, ir, 0);
+                    v.x -= a.cxx * c.x + a.cxy * (l.y - r.y);
+                    v.y -= a.cyy * c.y + a.cxy * (l.x - r.x);
+                }
+                if (j == N) {
+                    const cplx c = wall_node(a, src, i, N + 1), l = wall_node(a, src, il, N + 1),
+                               r = wall_node(a, src, ir, N + 1);
+                    v.x -= a.cxx * c.x + a.cxy * (r.y - l.y);
+                    v.y -= a.cyy * c.y + a.cxy * (r.x - l.x);
+                }
+            }
+        }
+        buf[row * fpad(M) + fpad(i)] = v;
+    }
+    __syncthreads();
+    const cplx *c = transform_rows<MT>(a, buf);
+    // twice the modes of u and of v' = -i v from those of u + i v
+    double2 *S = reinterpret_cast<double2 *>(a.S);
+    for (int t = threadIdx.x; t < kRows * K; t += kRowThreads) {
+        const int row = t % kRows, k = t / kRows, j = j0 - 1 + row;
+        if (j >= N) continue;
+        const cplx p = c[row * fpad(M) + fpad(k)], q = c[row * fpad(M) + fpad(k == 0 ? 0 : M - k)];
+        double2 *o = S + 2 * ((size_t)k * N + j);
+        o[0] = make_double2(p.x + q.x, p.y - q.y);
+        o[1] = make_double2(q.x - p.x, -p.y - q.y);
+    }
+}
+
+// inverse launch body: the modes of kRows interior rows back to (u, v),
+// stored (or added); the first workgroup also writes the wall rows
+template <int MT>
+__device__ __forceinline__ static void fourier_inverse_body(const FourierArgs &a, const double *__restrict__ src2,
+                                                            double *__restrict__ z2, bool add, int blk) {
+    extern __shared__ __align__(16) unsigned char fourier_smem[];
+    cplx *buf = reinterpret_cast<cplx *>(fourier_smem);
+    const int M = MT > 0 ? MT : a.M, N = a.N, K = M / 2 + 1;
+    const int j0 = 1 + kRows * blk;
+    const double2 *S = reinterpret_cast<const double2 *>(a.S);
+    cplx *z = reinterpret_cast<cplx *>(z2);
+    // conjugates of the modes of u + i v, so that the forward transform is
+    // the conjugate of the inverse one
+    for (int t = threadIdx.x; t < kRows * K; t += kRowThreads) {
+        const int row = t % kRows, k = t / kRows, j = j0 - 1 + row;
+        double2 u = make_double2(0, 0), w = u;
+        if (j < N) {
+            const double2 *s = S + 2 * ((size_t)k * N + j);
+            u = s[0];
+            w = s[1];
+        }
+        buf[row * fpad(M) + fpad(k)] = {u.x - w.x, w.y - u.y};
+        if (k > 0 && 2 * k < M) buf[row * fpad(M) + fpad(M - k)] = {u.x + w.x, u.y + w.y};
+    }
+    __syncthreads();
+    const cplx *c = transform_rows<MT>(a, buf);
+    const double sc = 0.5 / M;
+    for (int t = threadIdx.x; t < kRows * M; t += kRowThreads) {
+        const int row = t / M, i = t - row * M, j = j0 + row;
+        if (j > N) continue;
+        const cplx v = c[row * fpad(M) + fpad(i)];
+        cplx *o = z + (size_t)i + (size_t)M * j;
+        if (add) *o = {fmav(sc, v.x, o->x), fmav(-sc, v.y, o->y)};
+        else *o = {sc * v.x, -sc * v.y};
+    }
+    if (blk == 0) {
+        const cplx *src = reinterpret_cast<const cplx *>(src2);
+        for (int t = threadIdx.x; t < 2 * M; t += kRowThreads) {
+            const int i = t % M, j = t < M ? 0 : N + 1;
+            const cplx w = wall_node(a, src, i, j);
+            cplx *o = z + (size_t)i + (size_t)M * j;
+            if (add) *o = *o + w;
+            else *o = w;
+        }
+    }
+}
+
+// ---------------------------------------------------------------------------
+// the mode solve
+// ---------------------------------------------------------------------------
+// per-mode table: F, D^{-1}, -P (I + G P)^{-1}, then F^P 2^s for s = 0..6
+// (row-major 2x2 blocks)
+constexpr int kModePow = 7;
+constexpr int kModeTab = 4 * (3 + kModePow);
+
+struct v4 { double ux, uy, wx, wy; };  // (u, v') of a row, complex
+
+// r = A x + r with A row-major 2x2 acting on (u, v')
+__device__ __forceinline__ static void mad2(const double *A, const v4 &x, v4 &r) {
+    r.ux = fmav(A[1], x.wx, fmav(A[0], x.ux, r.ux));
+    r.uy = fmav(A[1], x.wy, fmav(A[0], x.uy, r.uy));
+    r.wx = fmav(A[3], x.wx, fmav(A[2], x.ux, r.wx));
+    r.wy = fmav(A[3], x.wy, fmav(A[2], x.uy, r.wy));
+}
+__device__ __forceinline__ static void mad2t(const double *A, const v4 &x, v4 &r) {  // transpose
+    r.ux = fmav(A[2], x.wx, fmav(A[0], x.ux, r.ux));
+    r.uy = fmav(A[2], x.wy, fmav(A[0], x.uy, r.uy));
+    r.wx = fmav(A[3], x.wx, fmav(A[1], x.ux, r.wx));
+    r.wy = fmav(A[3], x.wy, fmav(A[1], x.uy, r.wy));
+}
+__device__ __forceinline__ static v4 mul2(const double *A, const v4 &x) {
+    v4 r = {0, 0, 0, 0};
+    mad2(A, x, r);
+    return r;
+}
+template <bool UP> __device__ __forceinline__ static v4 lane_shift(const v4 &x, int d) {
+    // the value d lanes below (UP) or above; zero past the wave's end
+    const int lane = threadIdx.x & 63;
+    v4 r;
+    if (UP) {
+        r = {__shfl_up(x.ux, d, 64), __shfl_up(x.uy, d, 64), __shfl_up(x.wx, d, 64), __shfl_up(x.wy, d, 64)};
+        if (lane < d) r = {0, 0, 0, 0};
+    } else {
+        r = {__shfl_down(x.ux, d, 64), __shfl_down(x.uy, d, 64), __shfl_down(x.wx, d, 64),
+             __shfl_down(x.wy, d, 64)};
+        if (lane + d >= 64) r = {0, 0, 0, 0};
+    }
+    return r;
+}
+
+// carry into each lane of a recurrence whose lanes' own results are `t`:
+// the inclusive scan of t with the factor F^P per lane (or its transpose,
+// backwards), shifted by one lane; W waves combined through `xw` in LDS
+template <int W, bool UP>
+__device__ __forceinline__ static v4 scan_carry(const double *pw, v4 t, v4 *xw) {
+#pragma unroll
+    for (int s = 0; s < 6; s++) {
+        const v4 n = lane_shift<UP>(t, 1 << s);
+        if (UP) mad2(pw + 4 * s, n, t);
+        else mad2t(pw + 4 * s, n, t);
+    }
+    v4 c = lane_shift<UP>(t, 1);
+    if constexpr (W > 1) {
+        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        __syncthreads();
+        if (lane == (UP ? 63 : 0)) xw[wave] = t;
+        __syncthreads();
+        // the waves before (after) this one, combined in their order
+        v4 in = {0, 0, 0, 0};
+#pragma unroll
+        for (int q = 0; q < W - 1; q++) {
+            const int w = UP ? q : W - 1 - q;
+            if (UP ? w < wave : w > wave) {
+                v4 r = xw[w];
+                if (UP) mad2(pw + 4 * 6, in, r);
+                else mad2t(pw + 4 * 6, in, r);
+                in = r;
+            }
+        }
+        // times F^{P lane}: the powers of this lane's bits
+        const int d = UP ? lane : 63 - lane;
+#pragma unroll
+        for (int s = 0; s < 6; s++)
+            if ((d >> s) & 1) {
+                v4 r = {0, 0, 0, 0};
+                if (UP) mad2(pw + 4 * s, in, r);
+                else mad2t(pw + 4 * s, in, r);
+                in = r;
+            }
+        c = {c.ux + in.ux, c.uy + in.uy, c.wx + in.wx, c.wy + in.wy};
+    }
+    return c;
+}
+
+// LDS column of a mode: row j of P rows per thread at slot 2 j + (j / P), in
+// 16-byte units: a thread's rows are contiguous and threads start one slot
+// apart in the banks
+template <int P> __host__ __device__ constexpr int mode_slot(int j) { return 2 * j + j / P; }
+
+template <int W, int P>
+__device__ __forceinline__ static void fourier_mode_body(const FourierArgs &a, int k) {
+    extern __shared__ __align__(16) unsigned char fourier_smem[];
+    constexpr int NT = 64 * W, ROWS = NT * P;
+    double2 *col = reinterpret_cast<double2 *>(fourier_smem);
+    __shared__ v4 xw[W];
+    __shared__ v4 first;
+    const int N = a.N, tid = threadIdx.x;
+    const double *tab = a.tab + (size_t)kModeTab * k;
+    const double *F = tab, *Di = tab + 4, *C = tab + 8, *pw = tab + 12;
+    double2 *S = reinterpret_cast<double2 *>(a.S) + (size_t)2 * k * N;
+    // the column, coalesced, all of a thread's loads in flight
+    double2 in[2 * P];
+#pragma unroll
+    for (int q = 0; q < 2 * P; q++) {
+        const int t = tid + NT * q;
+        in[q] = S[t < 2 * N ? t : 0];
+    }
+#pragma unroll
+    for (int q = 0; q < 2 * P; q++) {
+        const int t = tid + NT * q;
+        col[mode_slot<P>(t >> 1) + (t & 1)] = t < 2 * N ? in[q] : make_double2(0, 0);
+    }
+    __syncthreads();
+    v4 g[P];
+    const int r0 = tid * P;
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+        const double2 u = col[mode_slot<P>(r0) + 2 * p], w = col[mode_slot<P>(r0) + 2 * p + 1];
+        g[p] = {u.x, u.y, w.x, w.y};
+    }
+    static_assert(ROWS > 0, "rows");
+    // forward: g_j = f_j + F g_{j-1}
+#pragma unroll
+    for (int p = 1; p < P; p++) mad2(F, g[p - 1], g[p]);
+    v4 c = scan_carry<W, true>(pw, g[P - 1], xw);
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+        c = mul2(F, c);
+        g[p] = {g[p].ux + c.ux, g[p].uy + c.uy, g[p].wx + c.wx, g[p].wy + c.wy};
+        if (r0 + p >= N) g[p] = {0, 0, 0, 0};
+    }
+    // backward for the first row only: y_1
+    v4 y = mul2(Di, g[P - 1]);
+#pragma unroll
+    for (int p = P - 2; p >= 0; p--) {
+        v4 t = mul2(Di, g[p]);
+        mad2t(F, y, t);
+        y = t;
+    }
+    v4 t0 = scan_carry<W, false>(pw, y, xw);
+    if (tid == 0) {
+        // y_1 = this thread's own part + E^P times the carry from the next
+        mad2t(pw, t0, y);
+        first = mul2(C, y);  // -P w_1
+    }
+    __syncthreads();
+    // g_j += F^{j-1} (-P w_1)
+    v4 h = first;
+#pragma unroll
+    for (int s = 0; s < 6; s++)
+        if ((tid >> s) & 1) h = mul2(pw + 4 * s, h);
+    if constexpr (W > 1)
+        for (int w = 0; w < (tid >> 6); w++) h = mul2(pw + 4 * 6, h);
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+        if (r0 + p < N) g[p] = {g[p].ux + h.ux, g[p].uy + h.uy, g[p].wx + h.wx, g[p].wy + h.wy};
+        h = mul2(F, h);
+    }
+    // backward: w_j = D^{-1} g_j + E w_{j+1}
+    g[P - 1] = mul2(Di, g[P - 1]);
+#pragma unroll
+    for (int p = P - 2; p >= 0; p--) {
+        v4 t = mul2(Di, g[p]);
+        mad2t(F, g[p + 1], t);
+        g[p] = t;
+    }
+    c = scan_carry<W, false>(pw, g[0], xw);
+#pragma unroll
+    for (int p = P - 1; p >= 0; p--) {
+        v4 t = {0, 0, 0, 0};
+        mad2t(F, c, t);
+        c = t;
+        g[p] = {g[p].ux + c.ux, g[p].uy + c.uy, g[p].wx + c.wx, g[p].wy + c.wy};
+    }
+#pragma unroll
+    for (int p = 0; p < P; p++) {
+        col[mode_slot<P>(r0) + 2 * p] = make_double2(g[p].ux, g[p].uy);
+        col[mode_slot<P>(r0) + 2 * p + 1] = make_double2(g[p].wx, g[p].wy);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 2 * P; q++) {
+        const int t = tid + NT * q;
+        if (t < 2 * N) S[t] = col[mode_slot<P>(t >> 1) + (t & 1)];
+    }
+}
+
+// ---------------------------------------------------------------------------
+// kernels
+// ---------------------------------------------------------------------------
+template <int MT>
+__global__ void __launch_bounds__(kRowThreads) fourier_forward_kernel(FourierArgs a, const double *src) {
+    fourier_forward_body<MT>(a, src, blockIdx.x);
+}
+template <int MT>
+__global__ void __launch_bounds__(kRowThreads) fourier_inverse_kernel(FourierArgs a, const double *src, double *z,
+                                                                      bool add) {
+    fourier_inverse_body<MT>(a, src, z, add, blockIdx.x);
+}
+template <int W, int P> __global__ void __launch_bounds__(64 * W) fourier_mode_kernel(FourierArgs a) {
+    fourier_mode_body<W, P>(a, blockIdx.x);
+}
+
+// the same over the members of an ensemble (batch.h) that solve this way;
+// members whose slot flag is clear return at once, and those past their first
+// test solve for the residual and add
+template <int MT>
+__global__ void __launch_bounds__(kRowThreads) fourier_forward_batch_kernel(const FourierEntry *E, const int *map,
+                                                                            const EnsState *St) {
+    const int2 el = batch_slot(map, blockIdx.x);
+    const FourierEntry &x = E[el.x];
+    if (!St[x.member].active) return;
+    const FourierArgs a = x.a;
+    fourier_forward_body<MT>(a, St[x.member].phase == ENS_LOOP ? x.r : x.src, el.y);
+}
+template <int MT>
+__global__ void __launch_bounds__(kRowThreads) fourier_inverse_batch_kernel(const FourierEntry *E, const int *map,
+                                                                            const EnsState *St) {
+    const int2 el = batch_slot(map, blockIdx.x);
+    const FourierEntry &x = E[el.x];
+    if (!St[x.member].active) return;
+    const FourierArgs a = x.a;
+    const bool add = St[x.member].phase == ENS_LOOP;
+    fourier_inverse_body<MT>(a, add ? x.r : x.src, x.z, add, el.y);
+}
+template <int W, int P>
+__global__ void __launch_bounds__(64 * W) fourier_mode_batch_kernel(const FourierEntry *E, const int *map,
+                                                                    const EnsState *St) {
+    const int2 el = batch_slot(map, blockIdx.x);
+    const FourierEntry &x = E[el.x];
+    if (!St[x.member].active) return;
+    const FourierArgs a = x.a;
+    fourier_mode_body<W, P>(a, el.y);
+}
+
+// ---------------------------------------------------------------------------
+// launchers
+// ---------------------------------------------------------------------------
+// lengths with the in-place transform of compile-time length
+static bool fixed_length(int M) { return M == 128 || M == 256 || M == 512 || M == 1024 || M == 2048 || M == 4096; }
+
+size_t fourier_row_lds(int M) { return (size_t)(fixed_length(M) ? 1 : 2) * kRows * fpad(M) * sizeof(cplx); }
+
+// rows per thread and waves per mode: eight rows a thread, fewer where one
+// wave then covers the column
+static int mode_rows(int N) { return N <= 128 ? 2 : (N <= 256 ? 4 : 8); }
+static int mode_waves(int N) { return N <= 512 ? 1 : (N <= 1024 ? 2 : (N <= 2048 ? 4 : 8)); }
+size_t fourier_mode_lds(int N) {
+    const int rows = 64 * mode_waves(N) * mode_rows(N);
+    return (size_t)(2 * rows + rows / mode_rows(N)) * 16;
+}
+
+bool fourier_fits(int M, int n) {
+    const int N = n - 2;  // n node rows, walls included
+    return M >= 4 && M <= 4096 && N >= 1 && N <= 4096 && fourier_row_lds(M) <= 152 * 1024;
+}
+
+// f(integral_constant) of the row kernels' compile-time length (0: any)
+template <typename F> static int with_length(int M, F f) {
+    switch (fixed_length(M) ? M : 0) {
+    case 128: return f(std::integral_constant<int, 128>());
+    case 256: return f(std::integral_constant<int, 256>());
+    case 512: return f(std::integral_constant<int, 512>());
+    case 1024: return f(std::integral_constant<int, 1024>());
+    case 2048: return f(std::integral_constant<int, 2048>());
+    case 4096: return f(std::integral_constant<int, 4096>());
+    default: return f(std::integral_constant<int, 0>());
+    }
+}
+// f(waves, rows per thread) of the mode kernel for N interior rows
+template <typename F> static int with_column(int N, F f) {
+    typedef std::integral_constant<int, 8> eight;
+    const int W = mode_waves(N), P = mode_rows(N);
+    if (W == 1 && P == 2) return f(std::integral_constant<int, 1>(), std::integral_constant<int, 2>());
+    if (W == 1 && P == 4) return f(std::integral_constant<int, 1>(), std::integral_constant<int, 4>());
+    if (W == 1) return f(std::integral_constant<int, 1>(), eight());
+    if (W == 2) return f(std::integral_constant<int, 2>(), eight());
+    if (W == 4) return f(std::integral_constant<int, 4>(), eight());
+    return f(eight(), eight());
+}
+
+template <typename K> static int allow_lds(K kernel, size_t bytes) {
+    if (bytes <= 64 * 1024) return STZ_OK;
+    STZ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)bytes));
+    return STZ_OK;
+}
+
+// raise the LDS limit of the kernels a grid uses (once per operator set-up)
+int fourier_set_lds_limit(const FourierArgs &a) {
+    const size_t rl = fourier_row_lds(a.M), ml = fourier_mode_lds(a.N);
+    const int e = with_length(a.M, [&](auto mt) {
+        constexpr int MT = decltype(mt)::value;
+        int r;
+        if ((r = allow_lds(fourier_forward_kernel<MT>, rl)) || (r = allow_lds(fourier_inverse_kernel<MT>, rl)) ||
+            (r = allow_lds(fourier_forward_batch_kernel<MT>, rl)))
+            return r;
+        return allow_lds(fourier_inverse_batch_kernel<MT>, rl);
+    });
+    if (e) return e;
+    return with_column(a.N, [&](auto w, auto p) {
+        constexpr int W = decltype(w)::value, P = decltype(p)::value;
+        const int r = allow_lds(fourier_mode_kernel<W, P>, ml);
+        return r ? r : allow_lds(fourier_mode_batch_kernel<W, P>, ml);
+    });
+}
+
+int fourier_row_workgroups(int N) { return (N + kRows - 1) / kRows; }
+int fourier_row_variant(int M) { return fixed_length(M) ? M : 0; }
+int fourier_mode_variant(int N) { return 16 * mode_waves(N) + mode_rows(N); }
+
+// z = A^{-1} src, or (add) z += A^{-1} src
+int mg_fourier_solve(const FourierArgs &a, const double *src, double *z, bool add, hipStream_t st) {
+    const dim3 g(fourier_row_workgroups(a.N)), b(kRowThreads);
+    const size_t rl = fourier_row_lds(a.M), ml = fourier_mode_lds(a.N);
+    with_length(a.M, [&](auto mt) {
+        hipLaunchKernelGGL((fourier_forward_kernel<decltype(mt)::value>), g, b, rl, st, a, src);
+        return 0;
+    });
+    with_column(a.N, [&](auto w, auto p) {
+        constexpr int W = decltype(w)::value, P = decltype(p)::value;
+        hipLaunchKernelGGL((fourier_mode_kernel<W, P>), dim3(a.M / 2 + 1), dim3(64 * W), ml, st, a);
+        return 0;
+    });
+    with_length(a.M, [&](auto mt) {
+        hipLaunchKernelGGL((fourier_inverse_kernel<decltype(mt)::value>), g, b, rl, st, a, src, z, add);
+        return 0;
+    });
+    STZ_HIP(hipGetLastError());
+    return STZ_OK;
+}
+
+int batch_fourier_rows(bool inverse, int M, size_t lds, const FourierEntry *E, const int *map, int total,
+                       const EnsState *St, hipStream_t st) {
+    if (total == 0) return STZ_OK;
+    with_length(M, [&](auto mt) {
+        constexpr int MT = decltype(mt)::value;
+        if (inverse)
+            hipLaunchKernelGGL((fourier_inverse_batch_kernel<MT>), dim3(total), dim3(kRowThreads), lds, st, E, map, St);
+        else
+            hipLaunchKernelGGL((fourier_forward_batch_kernel<MT>), dim3(total), dim3(kRowThreads), lds, st, E, map, St);
+        return 0;
+    });
+    STZ_HIP(hipGetLastError());
+    return STZ_OK;
+}
+
+int batch_fourier_modes(int N, const FourierEntry *E, const int *map, int total, const EnsState *St,
+                        hipStream_t st) {
+    if (total == 0) return STZ_OK;
+    const size_t ml = fourier_mode_lds(N);
+    with_column(N, [&](auto w, auto p) {
+        constexpr int W = decltype(w)::value, P = decltype(p)::value;
+        hipLaunchKernelGGL((fourier_mode_batch_kernel<W, P>), dim3(total), dim3(64 * W), ml, st, E, map, St);
+        return 0;
+    });
+    STZ_HIP(hipGetLastError());
+    return STZ_OK;
+}
+
+// ---------------------------------------------------------------------------
+// host set-up
+// ---------------------------------------------------------------------------
+namespace {
+typedef long double real;
+struct m2 { real a, b, c, d; };
+m2 operator*(const m2 &x, const m2 &y) {
+    return {x.a * y.a + x.b * y.c, x.a * y.b + x.b * y.d, x.c * y.a + x.d * y.c, x.c * y.b + x.d * y.d};
+}
+m2 operator+(const m2 &x, const m2 &y) { return {x.a + y.a, x.b + y.b, x.c + y.c, x.d + y.d}; }
+m2 operator-(const m2 &x, const m2 &y) { return {x.a - y.a, x.b - y.b, x.c - y.c, x.d - y.d}; }
+m2 neg(const m2 &x) { return {-x.a, -x.b, -x.c, -x.d}; }
+m2 tr(const m2 &x) { return {x.a, x.c, x.b, x.d}; }
+m2 inv(const m2 &x) {
+    const real r = 1 / (x.a * x.d - x.b * x.c);
+    return {x.d * r, -x.b * r, -x.c * r, x.a * r};
+}
+real big(const m2 &x) { return std::fmax(std::fmax(std::fabs(x.a), std::fabs(x.b)), std::fmax(std::fabs(x.c), std::fabs(x.d))); }
+}  // namespace
+
+size_t fourier_spectrum_elems(int M, int N) { return (size_t)4 * (M / 2 + 1) * N; }
+size_t fourier_table_elems(int M) { return (size_t)2 * M + (size_t)kModeTab * (M / 2 + 1); }
+
+// The constants of the solve for M x (N + 2) nodes with the interior stencil
+// s40 and the wall rows' stencil w40 (sim.hip, top_row_stencil): T receives
+// the M roots of unity e^{-2 pi i m / M} and the mode tables.  Returns false
+// if the operator does not have the form above or a mode is singular.
+bool fourier_setup(const double *s40, const double *w40, int M, int N, FourierArgs &a, std::vector<double> &T) {
+    a.M = M;
+    a.N = N;
+    a.nst = 0;
+    int left = M;
+    for (int r : {4, 2, 3, 5})
+        while (left % r == 0) {
+            a.radix[a.nst++] = r;
+            left /= r;
+        }
+    for (int r = 7; left > 1; r += 2)
+        while (left % r == 0) {
+            a.radix[a.nst++] = r;
+            left /= r;
+        }
+    // the pattern of qs_multi's operator: edges diagonal, corners +-q off the
+    // diagonal, walls diagonal
+    const real xx = s40[12], xy = s40[15], yx = s40[4], yy = s40[7], q = s40[1];
+    if (!sparse_pattern(s40) || s40[20] != s40[12] || s40[23] != s40[15] || s40[28] != s40[4] ||
+        s40[31] != s40[7] || s40[2] != s40[1] || s40[9] != -s40[1] || s40[10] != -s40[1] || s40[25] != -s40[1] ||
+        s40[26] != -s40[1] || s40[33] != s40[1] || s40[34] != s40[1])
+        return false;
+    for (int k = 0; k < 36; k++)
+        if (w40[k] != 0 && k != 16 && k != 19) return false;
+    a.cxx = s40[4];
+    a.cyy = s40[7];
+    a.cxy = s40[1];
+    a.wix = w40[36];
+    a.wiy = w40[39];
+    T.assign(fourier_table_elems(M), 0.0);
+    const real pi = 3.14159265358979323846264338327950288L;
+    for (int m = 0; m < M; m++) {
+        // octant symmetry is not needed: sine and cosine in extended
+        // precision are correctly rounded to double all but always
+        const real th = 2 * pi * m / M;
+        T[2 * m] = (double)std::cos(th);
+        T[2 * m + 1] = (double)-std::sin(th);
+    }
+    const int P = mode_rows(N);
+    const real e0 = (real)s40[16] + 2 * xx + 2 * yx, e1 = (real)s40[19] + 2 * xy + 2 * yy;  // row sums: rounding
+    for (int k = 0; k <= M / 2; k++) {
+        const real th = pi * k / M, sh = std::sin(th) * std::sin(th);
+        const real sn = 2 * k == M ? 0 : 2 * q * std::sin(2 * th);
+        // cc + 2 cos(theta) edge = (row sum) - 2 edge_y - 4 sin^2(theta/2) edge_x;
+        // the row sum is zero but for rounding, which the residual keeps
+        const m2 B = {e0 - 2 * yx - 4 * sh * xx, 0, 0, e1 - 2 * yy - 4 * sh * xy};
+        const m2 Cu = {yx, -sn, sn, yy}, Cd = tr(Cu);
+        m2 D;
+        if (k == 0) {
+            D = {-yx, 0, 0, -yy};
+        } else {
+            m2 b = B, u = Cu, d = Cd;
+            D = B;
+            for (int it = 0; it < 64; it++) {
+                const m2 s = inv(b), us = u * s, ds = d * s, step = ds * u;
+                D = D - step;
+                b = b - us * d - step;
+                u = neg(us * u);
+                d = neg(ds * d);
+                if (big(step) <= 1e-22L * big(D)) break;
+            }
+        }
+        const m2 Di = inv(D), F = neg(Cd * Di);
+        // G = (M^{-1})_11 = sum_{m < N} (F^T)^m D^{-1} F^m, by doubling over N's bits
+        m2 G = Di, Fn = F;
+        int bit = 0;
+        while ((2 << bit) <= N) bit++;
+        for (bit--; bit >= 0; bit--) {
+            G = G + tr(Fn) * G * Fn;
+            Fn = Fn * Fn;
+            if ((N >> bit) & 1) {
+                G = Di + tr(F) * G * F;
+                Fn = Fn * F;
+            }
+        }
+        // P keeps the row-sum rounding out (mode 0: P = -Cu exactly)
+        const m2 Pm = k == 0 ? m2{-yx, 0, 0, -yy} : B - D;
+        const m2 one = {1, 0, 0, 1};
+        const m2 Cm = neg(Pm * inv(one + G * Pm));
+        double *t = T.data() + 2 * (size_t)M + (size_t)kModeTab * k;
+        auto put = [](double *o, const m2 &x) {
+            o[0] = (double)x.a;
+            o[1] = (double)x.b;
+            o[2] = (double)x.c;
+            o[3] = (double)x.d;
+        };
+        put(t, F);
+        put(t + 4, Di);
+        put(t + 8, Cm);
+        m2 Fp = F;
+        for (int p = 1; p < P; p++) Fp = Fp * F;
+        for (int s = 0; s < kModePow; s++) {
+            put(t + 12 + 4 * s, Fp);
+            Fp = Fp * Fp;
+        }
+        for (int r = 0; r < kModeTab; r++)
+            if (!std::isfinite(t[r])) return false;
+    }
+    return true;
+}
+
+}  // namespace stz

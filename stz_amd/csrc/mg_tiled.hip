@@ -26,6 +26,7 @@
 // The colour order inside a sweep, (0,0),(1,0),(0,1),(1,1) in (i%2, j%2), is
 // the one the per-colour kernels of mg.hip use, so both paths apply the same
 // smoother.
+#include <type_traits>
 #include <utility>
 
 #include "batch.h"
@@ -456,9 +457,11 @@ __global__ void __launch_bounds__(256) restrict_tile_kernel(LevelArgs<T> F, Leve
     }
 }
 
-// FP64 residual of the top level (64x16 tiles) -> FP32 source, |r|^2 partials
-template <bool SP>
-__device__ __forceinline__ static void refine_body(const LevelArgs<double> &L, float *b32, double *partial,
+// FP64 residual of the top level (64x16 tiles) -> |r|^2 partials and, unless
+// OUT is void, the residual in OUT (the FP32 source of the correction
+// equation, or the FP64 one)
+template <bool SP, typename OUT>
+__device__ __forceinline__ static void refine_body(const LevelArgs<double> &L, OUT *rout, double *partial,
                                                    int bx, int by, int gx) {
     constexpr int TX = 64, TY = 16, ZX = TX + 2, ZY = TY + 2, NT = 256;
     __shared__ vec2s<double> zs[ZY * ZX];
@@ -503,8 +506,10 @@ __device__ __forceinline__ static void refine_body(const LevelArgs<double> &L, f
             offdiag9_any<SP, double>(si, zd[-1], zd[0], zd[1], zc[-1], zc[1], zu[-1], zu[0], zu[1], ax, ay);
             resid_value_any<SP, double>(si, L.b[k], L.b[k + 1], ax, ay, z0, rx, ry);
         }
-        b32[k] = (float)rx;
-        b32[k + 1] = (float)ry;
+        if constexpr (!std::is_void<OUT>::value) {
+            rout[k] = (OUT)rx;
+            rout[k + 1] = (OUT)ry;
+        }
         acc += rx * rx + ry * ry;
     }
 #pragma unroll
@@ -516,7 +521,11 @@ __device__ __forceinline__ static void refine_body(const LevelArgs<double> &L, f
 
 template <bool SP>
 __global__ void __launch_bounds__(256) refine_kernel(LevelArgs<double> L, float *b32, double *partial) {
-    refine_body<SP>(L, b32, partial, blockIdx.x, blockIdx.y, gridDim.x);
+    refine_body<SP, float>(L, b32, partial, blockIdx.x, blockIdx.y, gridDim.x);
+}
+template <bool SP, typename OUT>
+__global__ void __launch_bounds__(256) resid_test_kernel(LevelArgs<double> L, OUT *r, double *partial) {
+    refine_body<SP, OUT>(L, r, partial, blockIdx.x, blockIdx.y, gridDim.x);
 }
 
 template <bool SP>
@@ -528,7 +537,21 @@ __global__ void __launch_bounds__(256) refine_batch_kernel(const RefineEntry *E,
     if (St && !St[x.member].resid) return;
     const LevelArgs<double> L = x.L;
     const int gx = x.gx;
-    refine_body<SP>(L, x.b32, x.partial, l % gx, l / gx, gx);
+    refine_body<SP, float>(L, x.b32, x.partial, l % gx, l / gx, gx);
+}
+
+// the residual test of the members that solve directly; OUT double: the
+// residual of those about to correct
+template <bool SP, typename OUT>
+__global__ void __launch_bounds__(256) resid_test_batch_kernel(const FourierEntry *E, const int *map,
+                                                               const EnsState *St) {
+    const int2 el = batch_slot(map, blockIdx.x);
+    const FourierEntry &x = E[el.x];
+    const EnsState &s = St[x.member];
+    if (!s.active || (!std::is_void<OUT>::value && s.phase != ENS_LOOP)) return;
+    const LevelArgs<double> L = x.L;
+    const int gx = x.gx, l = el.y;
+    refine_body<SP, OUT>(L, (OUT *)x.r, x.partial, l % gx, l / gx, gx);
 }
 
 // ---------------------------------------------------------------------------
@@ -723,6 +746,21 @@ int mg_refine(const LevelArgs<double> &L, float *b32, double *partial, double *o
     return out ? mg_sum_partials(partial, (int)(g.x * g.y), out, st) : STZ_OK;
 }
 
+template <typename OUT>
+static void launch_resid_test(const LevelArgs<double> &L, OUT *r, double *partial, hipStream_t st) {
+    const dim3 g((L.m + 63) / 64, (L.n + 15) / 16);
+    if (L.sparse) hipLaunchKernelGGL((resid_test_kernel<true, OUT>), g, dim3(256), 0, st, L, r, partial);
+    else hipLaunchKernelGGL((resid_test_kernel<false, OUT>), g, dim3(256), 0, st, L, r, partial);
+}
+
+int mg_resid_test(const LevelArgs<double> &L, double *r, double *partial, double *out, double *out2,
+                  hipStream_t st) {
+    if (r) launch_resid_test<double>(L, r, partial, st);
+    else launch_resid_test<void>(L, nullptr, partial, st);
+    STZ_HIP(hipGetLastError());
+    return mg_sum_partials(partial, mg_refine_blocks(L), out, st, out2);
+}
+
 template bool wall_ok<double>(const LevelArgs<double> &);
 template bool wall_ok<float>(const LevelArgs<float> &);
 template bool tiled_ok<double>(const LevelArgs<double> &);
@@ -791,6 +829,18 @@ int batch_refine(const RefineEntry *E, const int *map, int ne, int total, int sp
     if (ne == 0) return STZ_OK;
     if (sparse) hipLaunchKernelGGL(refine_batch_kernel<true>, dim3(total), dim3(256), 0, st, E, map, ne, St);
     else hipLaunchKernelGGL(refine_batch_kernel<false>, dim3(total), dim3(256), 0, st, E, map, ne, St);
+    STZ_HIP(hipGetLastError());
+    return STZ_OK;
+}
+
+int batch_resid_test(bool store, int sparse, const FourierEntry *E, const int *map, int total, const EnsState *St,
+                     hipStream_t st) {
+    if (total == 0) return STZ_OK;
+    const dim3 g(total), b(256);
+    if (store && sparse) hipLaunchKernelGGL((resid_test_batch_kernel<true, double>), g, b, 0, st, E, map, St);
+    else if (store) hipLaunchKernelGGL((resid_test_batch_kernel<false, double>), g, b, 0, st, E, map, St);
+    else if (sparse) hipLaunchKernelGGL((resid_test_batch_kernel<true, void>), g, b, 0, st, E, map, St);
+    else hipLaunchKernelGGL((resid_test_batch_kernel<false, void>), g, b, 0, st, E, map, St);
     STZ_HIP(hipGetLastError());
     return STZ_OK;
 }

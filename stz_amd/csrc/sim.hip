@@ -382,24 +382,81 @@ template <typename T> static int set_direct(DevMG<T> &mg, int ld, const std::vec
 // the finest level l in 1..lc with at most cfg.direct_nodes nodes, an
 // x-invariant operator and a shape the direct launches cover (direct_fits)
 // is solved exactly; the V-cycle stops there (both hierarchies)
-static int set_direct_level(stz_sim *s) {
-    int ld = -1;
+static int direct_level(const stz_sim *s) {
     const int lc = s->mg64.args.lc;
     for (int l = 1; l <= lc && l < (int)s->hl.size() && s->cfg.direct_nodes > 0; l++) {
         const HostLevel &H = s->hl[l];
-        if (H.xinv && (long long)H.m * H.n <= s->cfg.direct_nodes && direct_fits(H.m, H.n)) {
-            ld = l;
-            break;
-        }
+        if (H.xinv && (long long)H.m * H.n <= s->cfg.direct_nodes && direct_fits(H.m, H.n)) return l;
     }
+    return -1;
+}
+
+// pick the level; its mode inverses (a Gauss-Jordan per mode on the host) are
+// formed by mg_ensure_direct, when a V-cycle runs
+static void set_direct_level(stz_sim *s) {
+    const int ld = direct_level(s);
+    s->mg64.args.ld = ld;
+    s->mg64.args.Gd = nullptr;
+    if (s->precision == STZ_PREC_MIXED) {
+        s->mg32.args.ld = ld;
+        s->mg32.args.Gd = nullptr;
+    }
+    s->direct_pending = ld >= 0;
+}
+
+int mg_ensure_direct(stz_sim *s) {
+    if (!s->direct_pending) return STZ_OK;
+    const int ld = s->mg64.args.ld;
     std::vector<double> G;
-    if (ld >= 0 && !direct_inverse(s->hl[ld].S.data(), s->hl[ld].m, s->hl[ld].n, G)) {
+    if (!direct_inverse(s->hl[ld].S.data(), s->hl[ld].m, s->hl[ld].n, G)) {
         set_error("multigrid level %d (%d x %d) is singular", ld, s->hl[ld].m, s->hl[ld].n);
         return STZ_ERR_STATE;
     }
     int e;
     if ((e = set_direct(s->mg64, ld, G))) return e;
     if (s->precision == STZ_PREC_MIXED && (e = set_direct(s->mg32, ld, G))) return e;
+    s->direct_pending = false;
+    return STZ_OK;
+}
+
+// whether the V-cycle of this grid runs on tiled launches throughout
+static bool all_tiled(const stz_sim *s) {
+    const CoarseArgs<double> &A = s->mg64.args;
+    for (int l = 0; l < bottom_level(A); l++)
+        if (l == 0 ? !tiled_ok(s->top64()) : !tiled_ok(A.lv[l])) return false;
+    return true;
+}
+
+// Grids the direct solver (mg_fourier.hip) takes over from V-cycles (see also
+// fourier_active):
+//   - any grid with a level the tiled launches do not cover, where a V-cycle
+//     is a launch per colour and level: 240 x 191 at the default settings
+//     2.4 ms a step with V-cycles, 0.067 ms with it;
+//   - tiled grids of more than direct_nodes nodes (FP64 form) or four times
+//     that (mixed form).  It is faster there too (128^2 FP64 0.36 -> 0.043 ms
+//     a step, 1024^2 mixed in elastic loading 0.33 -> 0.12, 1024^2 FP64 in
+//     plastic flow 1.27 -> 0.14); the grids below the line keep the V-cycle
+//     and with it the adaptive cycle counts by which a batch of small members
+//     plans its launches;
+// unless direct_nodes = 0 asks for V-cycles down to the coarsest level
+// (`kernels` chooses the kernels of V-cycles only).
+static int set_fourier(stz_sim *s) {
+    s->fourier = false;
+    const int M = s->c.m, n = s->c.n + 1;
+    if (s->cfg.direct_nodes <= 0 || !fourier_fits(M, n)) return STZ_OK;
+    const long long least = (long long)s->cfg.direct_nodes * (s->precision == STZ_PREC_MIXED ? 4 : 1);
+    if (all_tiled(s) && (long long)M * n <= least) return STZ_OK;
+    std::vector<double> T;
+    if (!fourier_setup(s->hl[0].at(0, 1), s->hl[0].at(0, 0), M, n - 2, s->fa, T)) return STZ_OK;
+    if (!s->ftab) STZ_HIP(hipMalloc(&s->ftab, T.size() * sizeof(double)));
+    if (!s->fspec) STZ_HIP(hipMalloc(&s->fspec, fourier_spectrum_elems(M, n - 2) * sizeof(double)));
+    STZ_HIP(hipMemcpy(s->ftab, T.data(), T.size() * sizeof(double), hipMemcpyHostToDevice));
+    s->fa.tw = s->ftab;
+    s->fa.tab = s->ftab + 2 * (size_t)M;
+    s->fa.S = s->fspec;
+    int e;
+    if ((e = fourier_set_lds_limit(s->fa))) return e;
+    s->fourier = true;
     return STZ_OK;
 }
 
@@ -437,7 +494,9 @@ int mg_build(stz_sim *s, double viscdt) {
     }
     if ((e = set_level_stencils(s, s->mg64, Sx, binv))) return e;
     if (s->precision == STZ_PREC_MIXED && (e = set_level_stencils(s, s->mg32, Sx, binv))) return e;
-    return set_direct_level(s);
+    set_direct_level(s);
+    if ((e = set_fourier(s))) return e;
+    return fourier_active(s) ? STZ_OK : mg_ensure_direct(s);
 }
 
 // mixed form: FP64 residual of the top level -> FP32 source of the next
@@ -469,6 +528,7 @@ static int top_home(stz_sim *s) {
 // and a fresh FP64 residual (the next cycle's source)
 static int one_cycle(stz_sim *s, bool need_resid, bool need_norm = true) {
     int e;
+    if ((e = mg_ensure_direct(s))) return e;
     const bool tiled = s->cfg.kernels == 0;
     if (s->precision == STZ_PREC_FP64) {
         CoarseArgs<double> &A = s->mg64.args;
@@ -523,6 +583,63 @@ static int read_test(stz_sim *s, double *acc) {
     return STZ_OK;
 }
 
+// A solve through mg_fourier.hip: the direct solve, the residual test of
+// every solve, and for a test that fails one correction (residual, direct
+// solve, added) per further test.  The predictor moves as in a V-cycle solve
+// whose first test comes before any counted cycle and that adds one cycle
+// per failed test; there is no extra cycle, since what it adds to an iterate
+// stopped at its threshold the direct solve's rounding floor already has.
+// `ahead` is enqueued after the first test, before the host waits for it: the
+// caller's next launch, which tests the same norm on the device (s->gate) and
+// does nothing where the test fails; *ran says whether it took effect.
+template <typename F> static int fourier_solve(stz_sim *s, F ahead, bool *ran) {
+    int e;
+    const stz_mg_config &g = s->cfg;
+    const double tol = s->acc_base * g.tol_mult;
+    const int max_thresh = g.predict_mult * g.predict_max_iters;
+    *ran = false;
+    std::memset(&s->last, 0, sizeof s->last);
+    s->last.tolerance = tol;
+    double acc;
+    int n = 0;
+    double *scratch = s->mg64.args.lv[0].z2;
+    if ((e = mg_fourier_solve(s->fa, s->src, s->vel, false, s->stream))) return e;
+    if ((e = mg_resid_test(s->top64(), nullptr, s->partial, s->dnorm, s->gate, s->stream))) return e;
+    STZ_HIP(hipEventRecord(s->norm_ev, s->stream));
+    if ((e = ahead())) return e;
+    s->last.total_cycles = 1;
+    if ((e = read_test(s, &acc))) return e;
+    if (acc < tol) {
+        *ran = true;
+        if (s->lim > 0) s->lim -= 1 + s->lim / g.predict_decay;
+    } else {
+        do {
+            s->lim += g.predict_mult;
+            if (s->lim > max_thresh) {
+                s->last.status = STZ_ERR_NOT_CONVERGED;
+                s->last.cycles = n;
+                s->last.residual = acc;
+                set_error("multigrid: residual %g not below %g after %d corrections", acc, tol, n);
+                return STZ_ERR_NOT_CONVERGED;
+            }
+            n++;
+            if ((e = mg_resid_test(s->top64(), scratch, s->partial, s->dnorm, s->gate, s->stream))) return e;
+            if ((e = mg_fourier_solve(s->fa, scratch, s->vel, true, s->stream))) return e;
+            if ((e = mg_resid_test(s->top64(), nullptr, s->partial, s->dnorm, s->gate, s->stream))) return e;
+            STZ_HIP(hipEventRecord(s->norm_ev, s->stream));
+            s->last.total_cycles++;
+            if ((e = read_test(s, &acc))) return e;
+        } while (acc >= tol);
+    }
+    s->solves++;
+    s->vcount += n;
+    s->last.cycles = n;
+    s->last.residual = acc;
+    s->last.status = std::isnan(acc) ? STZ_ERR_NAN : STZ_OK;
+    if (s->last.status != STZ_OK) set_error("multigrid: NaN residual");
+    return s->last.status;
+}
+
 // tgmg::solve(type=4, tgmg_predict&) (tgmg.in.cc:266-301).  Every test is
 // followed by at least one more cycle: the extra cycle when it passes, the
 // first of the next k when it fails.  So with extra_cycles >= 1 that cycle is
@@ -531,6 +648,10 @@ static int read_test(stz_sim *s, double *acc) {
 // plain schedule, so the result is the same bit for bit.
 static int mg_solve_impl(stz_sim *s) {
     int e;
+    if (fourier_active(s)) {
+        bool ran;
+        return fourier_solve(s, [] { return (int)STZ_OK; }, &ran);
+    }
     const stz_mg_config &g = s->cfg;
     const double tol = s->acc_base * g.tol_mult;
     const int max_thresh = g.predict_mult * g.predict_max_iters;
@@ -629,7 +750,18 @@ static int projection_impl(stz_sim *s, double dt) {
     const double cxx = s->hl[0].S[40 + 16];  // interior centre block, x row
     const double xbc = s->c.bcs * cxx;
     if ((e = launch_source(s->c, s->cur, dt, xbc, bdry_vel(s), s->src, s->stream))) return e;
-    if ((e = mg_solve_impl(s))) return e;
+    if (fourier_active(s)) {
+        bool ran;
+        const double denom = (double)s->c.m * (s->c.n + 1), tol = s->acc_base * s->cfg.tol_mult;
+        if ((e = fourier_solve(s, [&] {
+                return launch_correct(s->c, s->cur, s->vel, dt, bdry_vel(s), bdry_pos(s), s->stream, s->gate, denom,
+                                      tol);
+            }, &ran)))
+            return e;
+        if (ran) return STZ_OK;
+    } else if ((e = mg_solve_impl(s))) {
+        return e;
+    }
     return launch_correct(s->c, s->cur, s->vel, dt, bdry_vel(s), bdry_pos(s), s->stream);
 }
 
@@ -703,6 +835,7 @@ int stz_sim_create(const stz_sim_params *p, int precision, stz_sim **out) {
     s->src = s->vel + 2 * nodes;
     if (hipMalloc(&s->dec, (size_t)c.m * c.n * sizeof(uint32_t)) != hipSuccess) return fail(STZ_ERR_HIP);
     (void)hipMemset(s->dec, 0, (size_t)c.m * c.n * sizeof(uint32_t));
+    if (hipMalloc(&s->gate, sizeof(double)) != hipSuccess) return fail(STZ_ERR_HIP);
     s->nblocks_norm = (int)std::max<size_t>((nodes + 255) / 256,
                                             (size_t)((c.m + 63) / 64) * ((c.n + 1 + 15) / 16));
     {
@@ -741,6 +874,9 @@ int stz_sim_destroy(stz_sim *s) {
     if (s->vel) (void)hipFree(s->vel);
     if (s->dec) (void)hipFree(s->dec);
     if (s->rep) (void)hipFree(s->rep);
+    if (s->ftab) (void)hipFree(s->ftab);
+    if (s->fspec) (void)hipFree(s->fspec);
+    if (s->gate) (void)hipFree(s->gate);
     if (s->partial) (void)hipFree(s->partial);
     if (s->hnorm) (void)hipHostFree(s->hnorm);
     if (s->norm_ev) (void)hipEventDestroy(s->norm_ev);
@@ -1037,6 +1173,7 @@ int stz_mg_vcycle_launch(stz_sim *s, int level, int mode, int count) {
     if (s->cfg.kernels != 0) { set_error("the per-colour kernels have no tiled launches"); return STZ_ERR_ARG; }
     if (count < 0) { set_error("negative count"); return STZ_ERR_ARG; }
     int e;
+    if ((e = mg_ensure_direct(s))) return e;
     for (int k = 0; k < count; k++) {
         if (s->precision == STZ_PREC_MIXED) {
             CoarseArgs<float> &A = s->mg32.args;
@@ -1057,6 +1194,7 @@ int stz_mg_fmg_pre(stz_sim *s) {
     CHECK_SIM(s);
     if (s->viscdt_prev < 0) { set_error("stz_mg_setup has not been called"); return STZ_ERR_STATE; }
     int e;
+    if ((e = mg_ensure_direct(s))) return e;
     if ((e = top_home(s))) return e;
     CoarseArgs<double> &A = s->mg64.args;
     A.nu1 = s->cfg.nu1;

@@ -77,6 +77,12 @@ struct stz_sim {
     double viscdt_prev = -1;
     stz::DevMG<double> mg64;
     stz::DevMG<float> mg32;
+    // direct solve of the top level (mg_fourier.hip), where the grid takes it
+    bool fourier = false;
+    stz::FourierArgs fa{};
+    double *ftab = nullptr, *fspec = nullptr;
+    bool direct_pending = false;       // the direct level's inverses are not formed yet
+    double *gate = nullptr;            // device copy of a convergence test's norm
     double *partial = nullptr, *dnorm = nullptr, *hnorm = nullptr;
     hipEvent_t norm_ev = nullptr;  // marks the end of a convergence test's norm
     int nblocks_norm = 0;
@@ -110,3 +116,17 @@ void top_row_stencil(const SimConst &c, double viscdt, bool wall, double *s40);
 // (re)build the operators for viscosity/dt = viscdt (qs_multi::init,
 // qs_multi.cc:31-54): host Galerkin hierarchy, uploads; no-op when unchanged
 int mg_build(stz_sim *s, double viscdt);
+// the direct coarse level's mode inverses, formed when a V-cycle first needs
+// them (mg_build leaves them out where solves go through mg_fourier.hip)
+int mg_ensure_direct(stz_sim *s);
+// Whether the simulation's solves go through mg_fourier.hip.  Small grids
+// whose predictor follows the threshold closely (predict_decay well below the
+// reference's 32) keep their V-cycles: such solves stop within a cycle or two
+// of the threshold, and up to about 180^2 that stopping error is 1e-6 to 2e-5
+// of an elastic run's transverse velocity, so the direct solve's result, exact
+// to 1e-12, would differ visibly from the run the caller tuned.  (Elsewhere
+// the two agree to 1e-6: at the default predictor to 2e-6 on any grid.)
+inline bool fourier_active(const stz_sim *s) {
+    const bool small = (long long)s->c.m * (s->c.n + 1) <= 32768;
+    return s->fourier && !(small && s->cfg.predict_decay < 8);
+}
