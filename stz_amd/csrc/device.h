@@ -55,6 +55,8 @@ int launch_source(const SimConst &c, const FieldPtrs &f, double dt, double xbc, 
 int launch_correct(const SimConst &c, const FieldPtrs &f, const double *vel, double dt, double bvel,
                    double bpos, hipStream_t st, const double *gate = nullptr, double denom = 1, double tol = 0);
 int launch_boundaries(const SimConst &c, const FieldPtrs &f, double bvel, double bpos, hipStream_t st);
+int launch_direct_finish(const SimConst &c, const FieldPtrs &f, const double *un, const double *vn, double bvel,
+                         double bpos, hipStream_t st);
 int launch_init_fields(const SimConst &c, const FieldPtrs &f, int chi_case, double chi0, double chi1,
                        hipStream_t st);
 

@@ -15,6 +15,8 @@
 // reference wherever no transcendental function is involved (the ENO, upwind
 // and yield decisions in particular); exp/tanh/cosh differ from glibc by at
 // most a few ulp.
+#include <algorithm>
+
 #include "batch.h"
 #include "device.h"
 #include "stz_law.h"
@@ -304,85 +306,89 @@ __global__ void __launch_bounds__(256) advect_replay_kernel(SimConst c, FieldPtr
 // plus the velocity update (ENO2 advection of u,v, the stress-divergence
 // force net_force(..,-hx,-hy,..) and viscosity), the compressive terms of
 // the stress update, and constant chi diffusion inside the cell update.
-// New u,v go to un,vn (rows 1..n-1; the caller copies them back), all other
-// new fields to the plane set w.
+// New u,v go to un,vn (rows 1..n-1; direct_finish_kernel copies them back),
+// all other new fields to the plane set w.
 // ---------------------------------------------------------------------------
 __global__ void __launch_bounds__(256) direct_kernel(SimConst c, FieldPtrs o, FieldPtrs w, double *un, double *vn,
                                                      double dt) {
     const int m = c.m, n = c.n;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    const int j = blockIdx.y * blockDim.y + threadIdx.y;
+    int bx, by;
+    xcd_band_tile(bx, by);
+    const int tx = threadIdx.x, ty = threadIdx.y;
+    const int i = bx * kAdvTileX + tx, j = by * kAdvTileY + ty;
+    // the same nine planes and halo as the advection, staged the same way
+    __shared__ double tile[kAdvPlanes * kAdvRows * kAdvCols];
+    stage_advect_tile(o, m, n, bx * kAdvTileX, by * kAdvTileY, tile);
     if (i >= m || j >= n) return;
+#define RD(k, dx, dy) tile[((k) * kAdvRows + ty + 2 + (dy)) * kAdvCols + tx + 2 + (dx)]
     const double third = 1. / 3;
     const double hx = 0.5 * c.xsp * dt, hy = 0.5 * c.ysp * dt, lx = c.lx;
     const double hxxv = 2 * c.xsp * hx * c.viscosity, hyyv = 2 * c.ysp * hy * c.viscosity, hcv = 2 * (hxxv + hyyv);
     const double hxxcd = 2 * c.xsp * hx * c.chi_diff, hyycd = 2 * c.ysp * hy * c.chi_diff,
                  hccd = 2 * (hxxcd + hyycd);
-    const int il = i == 0 ? m - 1 : i - 1, ir = i == m - 1 ? 0 : i + 1;
-    const int ill = i <= 1 ? i + m - 2 : i - 2, irr = i >= m - 2 ? i + 2 - m : i + 2;
     uint32_t br;
     double uc, vc, ux, vx, uy, vy, two_omega, dtmp;
 
     if (j > 0) {
         double Xx, Xy, Yx, Yy, fx, fy;
-        uc = PL(o.u, i, j);
-        vc = PL(o.v, i, j);
-        const double X0 = PL(o.X, i, j), Y0 = PL(o.Y, i, j);
+        uc = RD(kU, 0, 0);
+        vc = RD(kV, 0, 0);
+        const double X0 = RD(kX, 0, 0), Y0 = RD(kY, 0, 0);
         // rmv_eno2 / rmv_one_sided, shear_sim.cc:203-219, 588-625
         if (uc > 0) {
-            ux = hx * eno2(PL(o.u, ir, j), uc, PL(o.u, il, j), PL(o.u, ill, j), br);
-            vx = hx * eno2(PL(o.v, ir, j), vc, PL(o.v, il, j), PL(o.v, ill, j), br);
-            Xx = hx * eno2(PL(o.X, ir, j) + (i == m - 1 ? lx : 0), X0, PL(o.X, il, j) + (i == 0 ? -lx : 0),
-                           PL(o.X, ill, j) + (i <= 1 ? -lx : 0), br);
-            Yx = hx * eno2(PL(o.Y, ir, j), Y0, PL(o.Y, il, j), PL(o.Y, ill, j), br);
+            ux = hx * eno2(RD(kU, 1, 0), uc, RD(kU, -1, 0), RD(kU, -2, 0), br);
+            vx = hx * eno2(RD(kV, 1, 0), vc, RD(kV, -1, 0), RD(kV, -2, 0), br);
+            Xx = hx * eno2(RD(kX, 1, 0) + (i == m - 1 ? lx : 0), X0, RD(kX, -1, 0) + (i == 0 ? -lx : 0),
+                           RD(kX, -2, 0) + (i <= 1 ? -lx : 0), br);
+            Yx = hx * eno2(RD(kY, 1, 0), Y0, RD(kY, -1, 0), RD(kY, -2, 0), br);
         } else {
-            ux = -hx * eno2(PL(o.u, il, j), uc, PL(o.u, ir, j), PL(o.u, irr, j), br);
-            vx = -hx * eno2(PL(o.v, il, j), vc, PL(o.v, ir, j), PL(o.v, irr, j), br);
-            Xx = -hx * eno2(PL(o.X, il, j) + (i == 0 ? -lx : 0), X0, PL(o.X, ir, j) + (i == m - 1 ? lx : 0),
-                            PL(o.X, irr, j) + (i >= m - 2 ? lx : 0), br);
-            Yx = -hx * eno2(PL(o.Y, il, j), Y0, PL(o.Y, ir, j), PL(o.Y, irr, j), br);
+            ux = -hx * eno2(RD(kU, -1, 0), uc, RD(kU, 1, 0), RD(kU, 2, 0), br);
+            vx = -hx * eno2(RD(kV, -1, 0), vc, RD(kV, 1, 0), RD(kV, 2, 0), br);
+            Xx = -hx * eno2(RD(kX, -1, 0) + (i == 0 ? -lx : 0), X0, RD(kX, 1, 0) + (i == m - 1 ? lx : 0),
+                            RD(kX, 2, 0) + (i >= m - 2 ? lx : 0), br);
+            Yx = -hx * eno2(RD(kY, -1, 0), Y0, RD(kY, 1, 0), RD(kY, 2, 0), br);
         }
         if (vc > 0) {
             if (j > 1) {
-                uy = hy * eno2(PL(o.u, i, j + 1), uc, PL(o.u, i, j - 1), PL(o.u, i, j - 2), br);
-                vy = hy * eno2(PL(o.v, i, j + 1), vc, PL(o.v, i, j - 1), PL(o.v, i, j - 2), br);
-                Xy = hy * eno2(PL(o.X, i, j + 1), X0, PL(o.X, i, j - 1), PL(o.X, i, j - 2), br);
-                Yy = hy * eno2(PL(o.Y, i, j + 1), Y0, PL(o.Y, i, j - 1), PL(o.Y, i, j - 2), br);
+                uy = hy * eno2(RD(kU, 0, 1), uc, RD(kU, 0, -1), RD(kU, 0, -2), br);
+                vy = hy * eno2(RD(kV, 0, 1), vc, RD(kV, 0, -1), RD(kV, 0, -2), br);
+                Xy = hy * eno2(RD(kX, 0, 1), X0, RD(kX, 0, -1), RD(kX, 0, -2), br);
+                Yy = hy * eno2(RD(kY, 0, 1), Y0, RD(kY, 0, -1), RD(kY, 0, -2), br);
             } else {
-                uy = 2 * hy * (uc - PL(o.u, i, j - 1));
-                vy = 2 * hy * (vc - PL(o.v, i, j - 1));
+                uy = 2 * hy * (uc - RD(kU, 0, -1));
+                vy = 2 * hy * (vc - RD(kV, 0, -1));
                 const double hs = hy * 2;
-                Xy = hs * (X0 - PL(o.X, i, j - 1));
-                Yy = hs * (Y0 - PL(o.Y, i, j - 1));
+                Xy = hs * (X0 - RD(kX, 0, -1));
+                Yy = hs * (Y0 - RD(kY, 0, -1));
             }
         } else {
             if (j < n - 1) {
-                uy = -hy * eno2(PL(o.u, i, j - 1), uc, PL(o.u, i, j + 1), PL(o.u, i, j + 2), br);
-                vy = -hy * eno2(PL(o.v, i, j - 1), vc, PL(o.v, i, j + 1), PL(o.v, i, j + 2), br);
-                Xy = -hy * eno2(PL(o.X, i, j - 1), X0, PL(o.X, i, j + 1), PL(o.X, i, j + 2), br);
-                Yy = -hy * eno2(PL(o.Y, i, j - 1), Y0, PL(o.Y, i, j + 1), PL(o.Y, i, j + 2), br);
+                uy = -hy * eno2(RD(kU, 0, -1), uc, RD(kU, 0, 1), RD(kU, 0, 2), br);
+                vy = -hy * eno2(RD(kV, 0, -1), vc, RD(kV, 0, 1), RD(kV, 0, 2), br);
+                Xy = -hy * eno2(RD(kX, 0, -1), X0, RD(kX, 0, 1), RD(kX, 0, 2), br);
+                Yy = -hy * eno2(RD(kY, 0, -1), Y0, RD(kY, 0, 1), RD(kY, 0, 2), br);
             } else {
-                uy = 2 * -hy * (uc - PL(o.u, i, j + 1));
-                vy = 2 * -hy * (vc - PL(o.v, i, j + 1));
+                uy = 2 * -hy * (uc - RD(kU, 0, 1));
+                vy = 2 * -hy * (vc - RD(kV, 0, 1));
                 const double hs = -hy * 2;
-                Xy = hs * (X0 - PL(o.X, i, j + 1));
-                Yy = hs * (Y0 - PL(o.Y, i, j + 1));
+                Xy = hs * (X0 - RD(kX, 0, 1));
+                Yy = hs * (Y0 - RD(kY, 0, 1));
             }
         }
         // net_force(fx,fy,-hx,-hy,flp,fp), shear_sim.cc:222, 447-453
         {
             const double xf = -hx, yf = -hy;
-            const double p0 = PL(o.p, il, j - 1), p1 = PL(o.p, i, j - 1), p2 = PL(o.p, il, j), p3 = PL(o.p, i, j);
-            const double q0 = PL(o.q, il, j - 1), q1 = PL(o.q, i, j - 1), q2 = PL(o.q, il, j), q3 = PL(o.q, i, j);
-            const double s0 = PL(o.s, il, j - 1), s1 = PL(o.s, i, j - 1), s2 = PL(o.s, il, j), s3 = PL(o.s, i, j);
-            const double t0 = PL(o.tau, il, j - 1), t1 = PL(o.tau, i, j - 1), t2 = PL(o.tau, il, j),
-                         t3 = PL(o.tau, i, j);
+            const double p0 = RD(kP, -1, -1), p1 = RD(kP, 0, -1), p2 = RD(kP, -1, 0), p3 = RD(kP, 0, 0);
+            const double q0 = RD(kQ, -1, -1), q1 = RD(kQ, 0, -1), q2 = RD(kQ, -1, 0), q3 = RD(kQ, 0, 0);
+            const double s0 = RD(kS, -1, -1), s1 = RD(kS, 0, -1), s2 = RD(kS, -1, 0), s3 = RD(kS, 0, 0);
+            const double t0 = RD(kTau, -1, -1), t1 = RD(kTau, 0, -1), t2 = RD(kTau, -1, 0),
+                         t3 = RD(kTau, 0, 0);
             fx = (-p0 + p1 - p2 + p3 - q0 + q1 - q2 + q3 + s0 - s1 + s2 - s3) * xf + (t0 + t1 - t2 - t3) * yf;
             fy = (t0 - t1 + t2 - t3) * xf + (-p0 - p1 + p2 + p3 - q0 - q1 + q2 + q3 - s0 - s1 + s2 + s3) * yf;
         }
-        const double uvisc = hxxv * (PL(o.u, ir, j) + PL(o.u, il, j)) + hyyv * (PL(o.u, i, j + 1) + PL(o.u, i, j - 1)) -
+        const double uvisc = hxxv * (RD(kU, 1, 0) + RD(kU, -1, 0)) + hyyv * (RD(kU, 0, 1) + RD(kU, 0, -1)) -
                              hcv * uc;
-        const double vvisc = hxxv * (PL(o.v, ir, j) + PL(o.v, il, j)) + hyyv * (PL(o.v, i, j + 1) + PL(o.v, i, j - 1)) -
+        const double vvisc = hxxv * (RD(kV, 1, 0) + RD(kV, -1, 0)) + hyyv * (RD(kV, 0, 1) + RD(kV, 0, -1)) -
                              hcv * vc;
         // update() (fields.hh:56-60): u += cu, v += cv, X += cX, Y += cY
         PL(un, i, j) = uc + (-uc * ux - vc * uy + c.mu_inv * (fx + uvisc));
@@ -391,30 +397,30 @@ __global__ void __launch_bounds__(256) direct_kernel(SimConst c, FieldPtrs o, Fi
         PL(w.Y, i, j) = Y0 + (-uc * Yx - vc * Yy);
     } else {
         // row 0 keeps u, v, X, Y until set_boundaries; ghost row -1 carried over
-        PL(w.X, i, 0) = PL(o.X, i, 0);
-        PL(w.Y, i, 0) = PL(o.Y, i, 0);
-        PL(w.X, i, -1) = PL(o.X, i, -1);
-        PL(w.Y, i, -1) = PL(o.Y, i, -1);
-        PL(w.p, i, -1) = PL(o.p, i, -1);
-        PL(w.q, i, -1) = PL(o.q, i, -1);
-        PL(w.s, i, -1) = PL(o.s, i, -1);
-        PL(w.tau, i, -1) = PL(o.tau, i, -1);
-        PL(w.chi, i, -1) = PL(o.chi, i, -1);
+        PL(w.X, i, 0) = RD(kX, 0, 0);
+        PL(w.Y, i, 0) = RD(kY, 0, 0);
+        PL(w.X, i, -1) = RD(kX, 0, -1);
+        PL(w.Y, i, -1) = RD(kY, 0, -1);
+        PL(w.p, i, -1) = RD(kP, 0, -1);
+        PL(w.q, i, -1) = RD(kQ, 0, -1);
+        PL(w.s, i, -1) = RD(kS, 0, -1);
+        PL(w.tau, i, -1) = RD(kTau, 0, -1);
+        PL(w.chi, i, -1) = RD(kChi, 0, -1);
     }
     if (j == n - 1) {
-        PL(w.X, i, n) = PL(o.X, i, n);
-        PL(w.Y, i, n) = PL(o.Y, i, n);
-        PL(w.p, i, n) = PL(o.p, i, n);
-        PL(w.q, i, n) = PL(o.q, i, n);
-        PL(w.s, i, n) = PL(o.s, i, n);
-        PL(w.tau, i, n) = PL(o.tau, i, n);
-        PL(w.chi, i, n) = PL(o.chi, i, n);
+        PL(w.X, i, n) = RD(kX, 0, 1);
+        PL(w.Y, i, n) = RD(kY, 0, 1);
+        PL(w.p, i, n) = RD(kP, 0, 1);
+        PL(w.q, i, n) = RD(kQ, 0, 1);
+        PL(w.s, i, n) = RD(kS, 0, 1);
+        PL(w.tau, i, n) = RD(kTau, 0, 1);
+        PL(w.chi, i, n) = RD(kChi, 0, 1);
     }
 
     // deformation rate, staggered velocity and spin, shear_sim.cc:240-247
     {
-        const double u00 = PL(o.u, i, j), u10 = PL(o.u, ir, j), u01 = PL(o.u, i, j + 1), u11 = PL(o.u, ir, j + 1);
-        const double v00 = PL(o.v, i, j), v10 = PL(o.v, ir, j), v01 = PL(o.v, i, j + 1), v11 = PL(o.v, ir, j + 1);
+        const double u00 = RD(kU, 0, 0), u10 = RD(kU, 1, 0), u01 = RD(kU, 0, 1), u11 = RD(kU, 1, 1);
+        const double v00 = RD(kV, 0, 0), v10 = RD(kV, 1, 0), v01 = RD(kV, 0, 1), v11 = RD(kV, 1, 1);
         uc = 0.25 * (u00 + u10 + u01 + u11);
         vc = 0.25 * (v00 + v10 + v01 + v11);
         ux = hx * (-u00 + u10 - u01 + u11);
@@ -425,42 +431,41 @@ __global__ void __launch_bounds__(256) direct_kernel(SimConst c, FieldPtrs o, Fi
     }
 
     // ENO derivatives of p,q,s,tau,chi, shear_sim.cc:250-252
-    const double *F[5] = {o.p, o.q, o.s, o.tau, o.chi};
     double f0[5], f1[5], f2[5];
 #pragma unroll
-    for (int k = 0; k < 5; k++) f0[k] = PL(F[k], i, j);
+    for (int k = 0; k < 5; k++) f0[k] = RD(kP + k, 0, 0);
     if (uc > 0) {
 #pragma unroll
-        for (int k = 0; k < 5; k++) f1[k] = hx * eno2(PL(F[k], ir, j), f0[k], PL(F[k], il, j), PL(F[k], ill, j), br);
+        for (int k = 0; k < 5; k++) f1[k] = hx * eno2(RD(kP + k, 1, 0), f0[k], RD(kP + k, -1, 0), RD(kP + k, -2, 0), br);
     } else {
 #pragma unroll
-        for (int k = 0; k < 5; k++) f1[k] = -hx * eno2(PL(F[k], il, j), f0[k], PL(F[k], ir, j), PL(F[k], irr, j), br);
+        for (int k = 0; k < 5; k++) f1[k] = -hx * eno2(RD(kP + k, -1, 0), f0[k], RD(kP + k, 1, 0), RD(kP + k, 2, 0), br);
     }
     if (vc > 0) {
         if (j > 0) {
 #pragma unroll
             for (int k = 0; k < 5; k++)
-                f2[k] = hy * eno2(PL(F[k], i, j + 1), f0[k], PL(F[k], i, j - 1), PL(F[k], i, j - 2), br);
+                f2[k] = hy * eno2(RD(kP + k, 0, 1), f0[k], RD(kP + k, 0, -1), RD(kP + k, 0, -2), br);
         } else {
             const double hs = hy * 2;
 #pragma unroll
-            for (int k = 0; k < 5; k++) f2[k] = hs * (f0[k] - PL(F[k], i, j - 1));
+            for (int k = 0; k < 5; k++) f2[k] = hs * (f0[k] - RD(kP + k, 0, -1));
         }
     } else {
         if (j < n - 1) {
 #pragma unroll
             for (int k = 0; k < 5; k++)
-                f2[k] = -hy * eno2(PL(F[k], i, j - 1), f0[k], PL(F[k], i, j + 1), PL(F[k], i, j + 2), br);
+                f2[k] = -hy * eno2(RD(kP + k, 0, -1), f0[k], RD(kP + k, 0, 1), RD(kP + k, 0, 2), br);
         } else {
             const double hs = -hy * 2;
 #pragma unroll
-            for (int k = 0; k < 5; k++) f2[k] = hs * (f0[k] - PL(F[k], i, j + 1));
+            for (int k = 0; k < 5; k++) f2[k] = hs * (f0[k] - RD(kP + k, 0, 1));
         }
     }
 
     // chi with its constant diffusion, then plasticity, shear_sim.cc:256-257
-    double cchi = f0[4] - uc * f1[4] - vc * f2[4] + hxxcd * (PL(o.chi, ir, j) + PL(o.chi, il, j)) +
-                  hyycd * (PL(o.chi, i, j + 1) + PL(o.chi, i, j - 1)) - hccd * f0[4];
+    double cchi = f0[4] - uc * f1[4] - vc * f2[4] + hxxcd * (RD(kChi, 1, 0) + RD(kChi, -1, 0)) +
+                  hyycd * (RD(kChi, 0, 1) + RD(kChi, 0, -1)) - hccd * f0[4];
     const double sbar = sqrt(3 * f0[1] * f0[1] + f0[2] * f0[2] + f0[3] * f0[3]);
     double ddev;
     int trips;
@@ -475,6 +480,7 @@ __global__ void __launch_bounds__(256) direct_kernel(SimConst c, FieldPtrs o, Fi
     PL(w.q, i, j) = f0[1] + (-uc * f1[1] - vc * f2[1] - c.mu * third * (ux + vy) - dtmp * f0[1]);
     PL(w.s, i, j) = f0[2] + (-uc * f1[2] - vc * f2[2] + two_omega * f0[3] + c.mu * (ux - vy) - dtmp * f0[2]);
     PL(w.tau, i, j) = f0[3] + (-uc * f1[3] - vc * f2[3] - two_omega * f0[2] + c.mu * (vx + uy) - dtmp * f0[3]);
+#undef RD
 }
 
 // chi_diffusion, shear_sim.cc:364-386: w.chi holds the post-plastic chi
@@ -624,11 +630,10 @@ __global__ void __launch_bounds__(256) correct_kernel(SimConst c, FieldPtrs f, c
     correct_body(c, f, vel, dt, bvel, bpos, bx, by);
 }
 
-// set_boundaries on its own, shear_sim.cc:552-581
-__global__ void boundaries_kernel(SimConst c, FieldPtrs f, double bvel, double bpos) {
+// set_boundaries of column i, shear_sim.cc:552-581
+__device__ __forceinline__ static void boundaries_column(const SimConst &c, const FieldPtrs &f, double bvel,
+                                                         double bpos, int i) {
     const int m = c.m, n = c.n;
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= m) return;
     PL(f.u, i, 0) = -bvel;
     PL(f.v, i, 0) = 0;
     PL(f.X, i, 0) = c.ax + i * c.dx + bpos;
@@ -642,6 +647,25 @@ __global__ void boundaries_kernel(SimConst c, FieldPtrs f, double bvel, double b
     PL(f.Y, i, n) = c.by;
 #pragma unroll
     for (int k = 0; k < 5; k++) PL(F[k], i, n) = 2 * PL(F[k], i, n - 1) - PL(F[k], i, n - 2);
+}
+__global__ void boundaries_kernel(SimConst c, FieldPtrs f, double bvel, double bpos) {
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= c.m) return;
+    boundaries_column(c, f, bvel, bpos, i);
+}
+
+// the end of a direct step: the new u, v of rows 1..n-1 back into their
+// planes, and the boundaries (which write only rows the copy leaves alone)
+__global__ void __launch_bounds__(256) direct_finish_kernel(SimConst c, FieldPtrs f, const double *un,
+                                                            const double *vn, double bvel, double bpos) {
+    const int m = c.m, n = c.n;
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, nt = gridDim.x * blockDim.x;
+    if (t < m) boundaries_column(c, f, bvel, bpos, t);
+    const int count = m * (n - 1);
+    for (int k = t; k < count; k += nt) {
+        f.u[2 * m + k] = un[2 * m + k];
+        f.v[2 * m + k] = vn[2 * m + k];
+    }
 }
 
 // shear_sim.cc:60-114
@@ -732,6 +756,14 @@ int launch_correct(const SimConst &c, const FieldPtrs &f, const double *vel, dou
 
 int launch_boundaries(const SimConst &c, const FieldPtrs &f, double bvel, double bpos, hipStream_t st) {
     hipLaunchKernelGGL(boundaries_kernel, dim3((c.m + 255) / 256), dim3(256), 0, st, c, f, bvel, bpos);
+    STZ_HIP(hipGetLastError());
+    return STZ_OK;
+}
+
+int launch_direct_finish(const SimConst &c, const FieldPtrs &f, const double *un, const double *vn, double bvel,
+                         double bpos, hipStream_t st) {
+    const int blocks = std::min(std::max((c.m + 255) / 256, (int)(((long long)c.m * c.n + 1023) / 1024)), 2048);
+    hipLaunchKernelGGL(direct_finish_kernel, dim3(blocks), dim3(256), 0, st, c, f, un, vn, bvel, bpos);
     STZ_HIP(hipGetLastError());
     return STZ_OK;
 }

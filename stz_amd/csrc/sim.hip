@@ -1228,7 +1228,6 @@ int stz_sim_step_forward(stz_sim *s, double dt, int nsteps) {
     CHECK_SIM(s);
     if (nsteps < 0) { set_error("nsteps < 0"); return STZ_ERR_ARG; }
     const SimConst &c = s->c;
-    const size_t row = (size_t)c.m;
     int e;
     for (int k = 0; k < nsteps; k++) {
         s->time += dt;  // shear_sim.cc:192
@@ -1236,12 +1235,7 @@ int stz_sim_step_forward(stz_sim *s, double dt, int nsteps) {
         if (c.chi_diff != 0 || c.chi_len != 0)
             if ((e = launch_chi_diffusion(c, s->cur, s->alt, dt, s->stream))) return e;
         std::swap(s->cur, s->alt);
-        // new u, v of rows 1..n-1 (plane rows 2..n)
-        STZ_HIP(hipMemcpyAsync(s->cur.u + 2 * row, s->un + 2 * row, (c.n - 1) * row * sizeof(double),
-                               hipMemcpyDeviceToDevice, s->stream));
-        STZ_HIP(hipMemcpyAsync(s->cur.v + 2 * row, s->vn + 2 * row, (c.n - 1) * row * sizeof(double),
-                               hipMemcpyDeviceToDevice, s->stream));
-        if ((e = launch_boundaries(c, s->cur, bdry_vel(s), bdry_pos(s), s->stream))) return e;
+        if ((e = launch_direct_finish(c, s->cur, s->un, s->vn, bdry_vel(s), bdry_pos(s), s->stream))) return e;
     }
     STZ_HIP(hipStreamSynchronize(s->stream));
     return STZ_OK;

@@ -37,6 +37,18 @@ __host__ __device__ static S dpl_common_t(const stz_model_params &mp, const S &s
     return Dpl;
 }
 
+// whether the linear athermal law takes its exponential form at y = Omega
+// eps0 sbar / theta (on the device; the host evaluation keeps the C library's
+// hyperbolic tangent)
+template <class S> __host__ __device__ static inline bool large_rate(const S &y) {
+#ifdef __HIP_DEVICE_COMPILE__
+    return !(y < 10.0);
+#else
+    (void)y;
+    return false;
+#endif
+}
+
 // yield: -1 evaluates the athermal laws' yield test sbar < 1; 0 or 1 takes
 // the recorded branch (below or at/above yield) instead, whatever sbar is
 template <class S>
@@ -71,6 +83,27 @@ __host__ __device__ static S dplastic_t(const stz_model_params &mp, double theta
         S tmp, sC, sT;
         dchi2 = S(0);
         if (below) { dchi1 = S(0); return S(0); }
+        const S y = Oe * sbar * thetainv;
+        if (mp.t_model == -1 && large_rate(y)) {
+            // cosh(y) = e^y (1 + e^{-2y}) / 2 and tanh(y) = 1 - 2 e^{-2y} /
+            // (1 + e^{-2y}) at y >= 10, where e^{-2y} <= 2.1e-9: its rounding
+            // and the series' next term are below 1e-17 of either.  From
+            // 19.1 on e^{-2y} is under half a unit in the last place of both
+            // and neither sees it.  One or two exponentials in place of two
+            // and a hyperbolic tangent, which is the longest piece of a
+            // substep (a cell far above yield takes hundreds in series).
+            sC = 0.5 * exp((Oe * sbar - mp.Delta) * thetainv);
+            sT = S(1);
+            if (y < 19.1) {
+                const S q = exp(-y), q2 = q * q;
+                sC = sC + sC * q2;
+                sT = 1 - 2 * q2 * (1 - q2);
+            }
+            S bfac = exp(-1 / chi), Dpl = bfac * sC * (sT - s0 / sbar) / mp.tau0,
+              Gamma = 2 * mp.tau0 * Dpl * sbar / (s0 * bfac);
+            dchi1 = bfac * Gamma / (mp.tau0 * c0);
+            return Dpl;
+        }
         if (mp.t_model == -1 || mp.Delta >= Oe * sbar)
             sC = 0.5 * (exp((Oe * sbar - mp.Delta) * thetainv) + exp((-Oe * sbar - mp.Delta) * thetainv));
         else switch (mp.t_model) {
