@@ -105,7 +105,7 @@ struct stz_ensemble {
     // state: device array and a pinned host copy
     EnsState *dst = nullptr, *hst = nullptr;
     // graphs
-    hipGraphExec_t g_tail[2] = {nullptr, nullptr}, g_slot = nullptr;
+    hipGraphExec_t g_tail[2] = {nullptr, nullptr}, g_slot[2] = {nullptr, nullptr};
     std::map<std::pair<int, int>, hipGraphExec_t> g_step;  // whole step by (parity, planned slots)
     int64_t stats[4] = {0, 0, 0, 0};
     int tuned[2] = {0, 0};        // launch positions that kept 32x16 / 64x34 tiles
@@ -114,10 +114,9 @@ struct stz_ensemble {
     void free_graphs() {
         for (int p = 0; p < 2; p++) {
             if (g_tail[p]) (void)hipGraphExecDestroy(g_tail[p]);
-            g_tail[p] = nullptr;
+            if (g_slot[p]) (void)hipGraphExecDestroy(g_slot[p]);
+            g_tail[p] = g_slot[p] = nullptr;
         }
-        if (g_slot) (void)hipGraphExecDestroy(g_slot);
-        g_slot = nullptr;
         for (auto &g : g_step) (void)hipGraphExecDestroy(g.second);
         g_step.clear();
     }
@@ -550,14 +549,14 @@ template <typename T> int launch_vcycle(stz_ensemble *e, const VCyclePlan<T> &P)
     return STZ_OK;
 }
 
-// the direct solves of a slot: the residual of members past their first
-// test, the solve, the test
-int launch_fourier(stz_ensemble *e) {
+// the direct solves of a slot and their test; with `again`, members past
+// their first test solve for their residual
+int launch_fourier(stz_ensemble *e, bool again) {
     const FourierPlan &P = e->fplan;
     const DevTable<FourierEntry> &T = P.test;
     hipStream_t st = e->stream;
     int rc;
-    if ((rc = batch_resid_test(true, P.sparse, T.E, T.map, T.total, e->dst, st))) return rc;
+    if (again && (rc = batch_resid_test(true, P.sparse, T.E, T.map, T.total, e->dst, st))) return rc;
     for (const FourierLaunch &l : P.rows)
         if ((rc = batch_fourier_rows(false, l.size, l.lds, l.t.E, l.t.map, l.t.total, e->dst, st))) return rc;
     for (const FourierLaunch &l : P.modes)
@@ -567,10 +566,16 @@ int launch_fourier(stz_ensemble *e) {
     return batch_resid_test(false, P.sparse, T.E, T.map, T.total, e->dst, st);
 }
 
-int launch_slot(stz_ensemble *e) {
+// What a slot does for the members that solve directly: the solve of the
+// first slot, nothing in the planned ones after it (they are done, and the
+// empty launches cost some 50 us a slot over 48 members), a correction in a
+// slot beyond the plan where one of them has failed its test.
+enum { SLOT_FIRST, SLOT_CYCLE, SLOT_AGAIN };
+
+int launch_slot(stz_ensemble *e, int kind) {
     int rc;
     hipStream_t st = e->stream;
-    if ((rc = launch_fourier(e))) return rc;
+    if (kind != SLOT_CYCLE && (rc = launch_fourier(e, kind == SLOT_AGAIN))) return rc;
     const DevTable<RefineEntry> &R = e->refs;
     if (e->precision == STZ_PREC_MIXED) {
         // vel += e is applied by the top level's last smoothing launch
@@ -614,12 +619,16 @@ template <typename F> int capture(stz_ensemble *e, hipGraphExec_t *out, F fn) {
     return STZ_OK;
 }
 
-int run_slot(stz_ensemble *e) {
+// a slot beyond the planned ones; `again`: a member that solves directly
+// has failed its test
+int run_slot(stz_ensemble *e, bool again) {
+    const int kind = again ? SLOT_AGAIN : SLOT_CYCLE;
     e->stats[1]++;
-    if (!e->use_graphs) return launch_slot(e);
+    if (!e->use_graphs) return launch_slot(e, kind);
     int rc;
-    if (!e->g_slot && (rc = capture(e, &e->g_slot, [&] { return launch_slot(e); }))) return rc;
-    STZ_HIP(hipGraphLaunch(e->g_slot, e->stream));
+    hipGraphExec_t &g = e->g_slot[again ? 1 : 0];
+    if (!g && (rc = capture(e, &g, [&] { return launch_slot(e, kind); }))) return rc;
+    STZ_HIP(hipGraphLaunch(g, e->stream));
     return STZ_OK;
 }
 
@@ -630,7 +639,7 @@ int run_step(stz_ensemble *e, int parity, int slots, double dt) {
     if (!e->use_graphs) {
         if ((rc = launch_head(e, parity, dt))) return rc;
         for (int q = 0; q < slots; q++)
-            if ((rc = launch_slot(e))) return rc;
+            if ((rc = launch_slot(e, q == 0 ? SLOT_FIRST : SLOT_CYCLE))) return rc;
         return launch_tail(e, parity, dt);
     }
     const std::pair<int, int> key(parity, slots);
@@ -641,7 +650,7 @@ int run_step(stz_ensemble *e, int parity, int slots, double dt) {
             int r;
             if ((r = launch_head(e, parity, dt))) return r;
             for (int q = 0; q < slots; q++)
-                if ((r = launch_slot(e))) return r;
+                if ((r = launch_slot(e, q == 0 ? SLOT_FIRST : SLOT_CYCLE))) return r;
             return launch_tail(e, parity, dt);
         });
         if (rc) return rc;
@@ -821,12 +830,15 @@ int stz_ensemble_step_quasistatic(stz_ensemble *e, double dt, int nsteps) {
         if ((rc = sync_state(e))) return abort_step(rc);
         // members whose predictor asked for more cycles than planned
         for (;;) {
-            bool more = false;
-            for (int k = 0; k < N; k++) more |= in_progress(e->hst[k]);
+            bool more = false, again = false;
+            for (int k = 0; k < N; k++) {
+                more |= in_progress(e->hst[k]);
+                again |= in_progress(e->hst[k]) && e->hst[k].direct;
+            }
             if (!more) break;
             for (int q = 0; q < 2; q++) {
                 e->stats[2]++;
-                if ((rc = run_slot(e))) return abort_step(rc);
+                if ((rc = run_slot(e, again))) return abort_step(rc);
             }
             if ((rc = run_tail(e, p, dt))) return abort_step(rc);
             if ((rc = sync_state(e))) return abort_step(rc);
