@@ -42,6 +42,17 @@ struct SimConst {
     double thetainv;
 };
 
+// net_force (shear_sim.cc:447-453) at a node from p, q, s, tau of the cells
+// (i-1,j-1), (i,j-1), (i-1,j), (i,j), in the reference's order
+__device__ __forceinline__ static void node_force(double p0, double p1, double p2, double p3, double q0, double q1,
+                                                  double q2, double q3, double s0, double s1, double s2, double s3,
+                                                  double t0, double t1, double t2, double t3, double xfac,
+                                                  double yfac, double &fx, double &fy) {
+#pragma clang fp contract(off)
+    fx = (-p0 + p1 - p2 + p3 - q0 + q1 - q2 + q3 + s0 - s1 + s2 - s3) * xfac + (t0 + t1 - t2 - t3) * yfac;
+    fy = (t0 - t1 + t2 - t3) * xfac + (-p0 - p1 + p2 + p3 - q0 - q1 + q2 + q3 - s0 - s1 + s2 + s3) * yfac;
+}
+
 // launchers (explicit.hip)
 // rep: a decision record to replay (one uint32 per cell), or null to evaluate
 int launch_advect(const SimConst &c, const FieldPtrs &old_f, const FieldPtrs &new_f, double dt,

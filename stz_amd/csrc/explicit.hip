@@ -539,8 +539,7 @@ __device__ __forceinline__ static void source_body(const SimConst &c, const Fiel
         const double s0 = PL(f.s, il, j - 1), s1 = PL(f.s, i, j - 1), s2 = PL(f.s, il, j), s3 = PL(f.s, i, j);
         const double t0 = PL(f.tau, il, j - 1), t1 = PL(f.tau, i, j - 1), t2 = PL(f.tau, il, j),
                      t3 = PL(f.tau, i, j);
-        fx = (-p0 + p1 - p2 + p3 - q0 + q1 - q2 + q3 + s0 - s1 + s2 - s3) * xfac + (t0 + t1 - t2 - t3) * yfac;
-        fy = (t0 - t1 + t2 - t3) * xfac + (-p0 - p1 + p2 + p3 - q0 - q1 + q2 + q3 - s0 - s1 + s2 + s3) * yfac;
+        node_force(p0, p1, p2, p3, q0, q1, q2, q3, s0, s1, s2, s3, t0, t1, t2, t3, xfac, yfac, fx, fy);
     }
     const int ij = i + m * j;
     src[2 * ij] = fx;

@@ -71,10 +71,11 @@ bool direct_inverse(const double *S, int M, int Nn, std::vector<double> &D);
 bool direct_fits(int M, int Nn);
 
 // mg_fourier.hip: direct solve of the top level's operator, FP64.  M nodes
-// per row, N interior rows; tw the M roots of unity and tab the modes'
-// constants (fourier_setup fills both, in this order), S the spectrum
+// per row, N interior rows (NP with padding); tw the transform's tables (4 M
+// doubles) and tab the modes' constants (fourier_setup fills both, in this
+// order), S the spectrum
 struct FourierArgs {
-    int M, N, nst;
+    int M, N, NP, nst;
     int radix[16];
     double cxx, cyy, cxy;  // a wall node's weight in the row next to it: u, v, and u-v through the corners
     double wix, wiy;       // inverse diagonal of the wall rows
@@ -86,7 +87,14 @@ bool fourier_fits(int M, int n);
 size_t fourier_spectrum_elems(int M, int N);
 bool fourier_setup(const double *s40, const double *w40, int M, int N, FourierArgs &a, std::vector<double> &T);
 int fourier_set_lds_limit(const FourierArgs &a);
-int mg_fourier_solve(const FourierArgs &a, const double *src, double *z, bool add, hipStream_t st);
+// what the projection's source is formed from (source_kernel, explicit.hip):
+// the planes of p, q, s, tau, the factors of the differences, and the wall
+// rows' value bcs cxx u_wall
+struct SourceArgs {
+    const double *f[4];
+    double xfac, yfac, wall;
+};
+int mg_fourier_solve(const FourierArgs &a, const SourceArgs *f, double *src, double *z, bool add, hipStream_t st);
 
 // LDS layout for levels lc..L-1; returns the number of elements of T
 template <typename T> int coarse_layout(CoarseArgs<T> &A);

@@ -23,14 +23,14 @@
 // to 1024^2, so one application replaces all V-cycles of a solve.
 //
 // Three launches:
-//   forward   R rows per workgroup: u + i v of a row as one complex signal,
-//             an in-LDS Stockham transform, the two real signals' modes
-//             separated on the way out
+//   forward   R rows per workgroup: u + i v of a row as one complex signal
+//             (in a step the source is formed here), an in-LDS Stockham
+//             transform, the two real signals' modes separated on the way out
 //   modes     one workgroup per mode, the column in LDS
 //   inverse   R rows per workgroup, back to (u, v)
-// The spectrum is kept mode-major, S[k][j] of 32 bytes (u, v' complex), so
-// the mode launch reads and writes whole columns and a row workgroup touches
-// R * 32 contiguous bytes per mode.
+// The spectrum is kept mode-major, S[k][j] of 32 bytes (u, v' complex), a
+// column padded to four rows, so the mode launch reads and writes whole
+// columns and a row workgroup touches R * 32 contiguous bytes per mode.
 #include <hip/hip_runtime.h>
 
 #include <cmath>
@@ -47,8 +47,10 @@ namespace stz {
 // ---------------------------------------------------------------------------
 // the row transform
 // ---------------------------------------------------------------------------
-constexpr int kRowThreads = 256;
-constexpr int kRows = 2;           // rows per workgroup of the row launches
+// rows per workgroup R with 128 threads each: four where that leaves a
+// workgroup per CU (their 128-byte pieces of the spectrum are whole cache
+// lines), else two.  A row's result does not depend on R.
+constexpr int kRowThreads = 128;
 
 struct alignas(16) cplx { double x, y; };
 
@@ -117,13 +119,40 @@ template <> __device__ __forceinline__ void dft<8>(cplx (&x)[8]) {
     x[7] = e[3] - o3;
 }
 
-// One Stockham stage of radix RX for kRows rows of M values in `buf`, in
-// place: L is the product of the radices before it.  Every butterfly of a
-// thread is in registers between the two barriers, which is why M is a
-// compile-time constant here.
-template <int M, int RX, int L>
-__device__ __forceinline__ static void stage_fixed(cplx *buf, const cplx *__restrict__ tw) {
-    constexpr int NBF = kRows * (M / RX), NT = kRowThreads, Q = (NBF + NT - 1) / NT;
+// Twiddles of a stage after radices of product L: entry (q - 1) L + k of the
+// stage's part of the table, which starts at L - 1 (the parts of the stages
+// before it), so a wave's loads of one q are consecutive.
+template <int RX, int L, int Q> struct Twiddles { cplx w[Q][RX > 1 ? RX - 1 : 1]; };
+
+// radix of the stage after a product of L, for the lengths known at compile
+// time: 8 while that leaves a multiple of 4, then 4 and at most one 2
+__host__ __device__ constexpr int fixed_radix(int left) {
+    return left % 8 == 0 && left != 16 ? 8 : (left % 4 == 0 ? 4 : (left > 1 ? 2 : 1));
+}
+
+template <int M, int R, int RX, int L>
+__device__ __forceinline__ static auto load_twiddles(const cplx *__restrict__ tw) {
+    constexpr int NT = kRowThreads * R, NBF = R * (M / RX), Q = (NBF + NT - 1) / NT;
+    Twiddles<RX, L, Q> t;
+    if constexpr (RX > 1) {
+#pragma unroll
+        for (int b = 0; b < Q; b++) {
+            const int k = ((threadIdx.x + NT * b) % (M / RX)) % L;
+#pragma unroll
+            for (int q = 1; q < RX; q++) t.w[b][q - 1] = tw[L - 1 + (q - 1) * L + k];
+        }
+    }
+    return t;
+}
+
+// One Stockham stage for R rows of M values in `buf`, in place, and those
+// after it.  Every butterfly of a thread is in registers between the two
+// barriers, which is why M is a compile-time constant here; the next stage's
+// twiddles are loaded before them.
+template <int M, int R, int RX, int L, int Q>
+__device__ __forceinline__ static void stages_fixed(cplx *buf, const cplx *__restrict__ tw,
+                                                    const Twiddles<RX, L, Q> &w) {
+    constexpr int NT = kRowThreads * R, NBF = R * (M / RX);
     cplx x[Q][RX];
 #pragma unroll
     for (int b = 0; b < Q; b++) {
@@ -132,14 +161,14 @@ __device__ __forceinline__ static void stage_fixed(cplx *buf, const cplx *__rest
             const int row = t / (M / RX), idx = t % (M / RX);
 #pragma unroll
             for (int q = 0; q < RX; q++) x[b][q] = buf[row * fpad(M) + fpad(idx + q * (M / RX))];
-            if (L > 1) {
-                const int k = idx % L;
+            if (L > 1)
 #pragma unroll
-                for (int q = 1; q < RX; q++) x[b][q] = cmul(x[b][q], tw[k * q * (M / (L * RX))]);
-            }
+                for (int q = 1; q < RX; q++) x[b][q] = cmul(x[b][q], w.w[b][q - 1]);
             dft<RX>(x[b]);
         }
     }
+    constexpr int LN = L * RX, RN = fixed_radix(M / LN);
+    const auto next = load_twiddles<M, R, RN, LN>(tw);
     __syncthreads();
 #pragma unroll
     for (int b = 0; b < Q; b++) {
@@ -152,35 +181,27 @@ __device__ __forceinline__ static void stage_fixed(cplx *buf, const cplx *__rest
         }
     }
     __syncthreads();
-}
-
-// the stages of a power-of-two length: radix 8 while that leaves a multiple
-// of 4, then radix 4 and at most one radix 2
-template <int M, int L> __device__ __forceinline__ static void stages_fixed(cplx *buf, const cplx *tw) {
-    constexpr int left = M / L;
-    if constexpr (left > 1) {
-        constexpr int RX = left % 8 == 0 && left != 16 ? 8 : (left % 4 == 0 ? 4 : 2);
-        stage_fixed<M, RX, L>(buf, tw);
-        stages_fixed<M, L * RX>(buf, tw);
-    }
+    if constexpr (RN > 1) stages_fixed<M, R>(buf, tw, next);
 }
 
 // any length: one stage from `in` to `out`, radix RX (0: the run-time radix
-// r as a plain sum per output, for the primes without a butterfly above)
-template <int RX>
-__device__ __forceinline__ static void stage_any(const cplx *in, cplx *out, const cplx *__restrict__ tw, int M,
-                                                 int L, int r) {
+// r as a plain sum per output with the roots of unity `root`, for the primes
+// without a butterfly above)
+template <int RX, int R>
+__device__ __forceinline__ static void stage_any(const cplx *in, cplx *out, const cplx *__restrict__ tw,
+                                                 const cplx *__restrict__ root, int M, int L, int r) {
+    constexpr int NT = kRowThreads * R;
     const int P = fpad(M);
     if constexpr (RX > 0) {
-        const int nb = M / RX, step = M / (L * RX);
-        for (int t = threadIdx.x; t < kRows * nb; t += kRowThreads) {
+        const int nb = M / RX;
+        for (int t = threadIdx.x; t < R * nb; t += NT) {
             const int row = t / nb, idx = t - row * nb, k = idx % L;
             cplx x[RX];
 #pragma unroll
             for (int q = 0; q < RX; q++) x[q] = in[row * P + fpad(idx + q * nb)];
             if (L > 1)
 #pragma unroll
-                for (int q = 1; q < RX; q++) x[q] = cmul(x[q], tw[k * q * step]);
+                for (int q = 1; q < RX; q++) x[q] = cmul(x[q], tw[L - 1 + (q - 1) * L + k]);
             dft<RX>(x);
             const int o = (idx - k) * RX + k;
 #pragma unroll
@@ -188,7 +209,7 @@ __device__ __forceinline__ static void stage_any(const cplx *in, cplx *out, cons
         }
     } else {
         const int nb = M / r, step = M / (L * r);
-        for (int t = threadIdx.x; t < kRows * M; t += kRowThreads) {
+        for (int t = threadIdx.x; t < R * M; t += NT) {
             const int row = t / M, e = t - row * M, q = e / nb, idx = e - q * nb, k = idx % L;
             // sum_p in[idx + p nb] w^{p (k step + q nb)}
             const int inc = (k * step + q * nb) % M;
@@ -197,30 +218,31 @@ __device__ __forceinline__ static void stage_any(const cplx *in, cplx *out, cons
             for (int p = 1; p < r; p++) {
                 w += inc;
                 if (w >= M) w -= M;
-                s = s + cmul(in[row * P + fpad(idx + p * nb)], tw[w]);
+                s = s + cmul(in[row * P + fpad(idx + p * nb)], root[w]);
             }
             out[row * P + fpad((idx - k) * r + k + q * L)] = s;
         }
     }
 }
 
-// transform the kRows rows in LDS; returns where the result is
-template <int MT>
+// transform the R rows in LDS; returns where the result is
+template <int MT, int R>
 __device__ __forceinline__ static cplx *transform_rows(const FourierArgs &a, cplx *buf) {
     const cplx *tw = reinterpret_cast<const cplx *>(a.tw);
     if constexpr (MT > 0) {
-        stages_fixed<MT, 1>(buf, tw);
+        stages_fixed<MT, R>(buf, tw, load_twiddles<MT, R, fixed_radix(MT), 1>(tw));
         return buf;
     } else {
-        cplx *in = buf, *out = buf + kRows * fpad(a.M);
+        const cplx *root = tw + a.M;
+        cplx *in = buf, *out = buf + R * fpad(a.M);
         int L = 1;
         for (int s = 0; s < a.nst; s++) {
             const int r = a.radix[s];
-            if (r == 4) stage_any<4>(in, out, tw, a.M, L, r);
-            else if (r == 2) stage_any<2>(in, out, tw, a.M, L, r);
-            else if (r == 3) stage_any<3>(in, out, tw, a.M, L, r);
-            else if (r == 5) stage_any<5>(in, out, tw, a.M, L, r);
-            else stage_any<0>(in, out, tw, a.M, L, r);
+            if (r == 4) stage_any<4, R>(in, out, tw, root, a.M, L, r);
+            else if (r == 2) stage_any<2, R>(in, out, tw, root, a.M, L, r);
+            else if (r == 3) stage_any<3, R>(in, out, tw, root, a.M, L, r);
+            else if (r == 5) stage_any<5, R>(in, out, tw, root, a.M, L, r);
+            else stage_any<0, R>(in, out, tw, root, a.M, L, r);
             __syncthreads();
             cplx *t = in;
             in = out;
@@ -237,70 +259,137 @@ __device__ __forceinline__ static cplx wall_node(const FourierArgs &a, const cpl
     return {a.wix * s.x, a.wiy * s.y};
 }
 
-// forward launch body: interior rows 1 + kRows * blk .., the two rows next to
-// the walls with the wall velocity's part moved to the right-hand side
-template <int MT>
-__device__ __forceinline__ static void fourier_forward_body(const FourierArgs &a, const double *__restrict__ src2,
-                                                            int blk) {
-    extern __shared__ __align__(16) unsigned char fourier_smem[];
-    cplx *buf = reinterpret_cast<cplx *>(fourier_smem);
+// the wall velocity's part of the row next to it, moved to the right-hand
+// side: c, l, r the wall node below (above) and its neighbours, sg 1 (-1)
+__device__ __forceinline__ static cplx less_wall(const FourierArgs &a, const cplx &v, const cplx &c, const cplx &l,
+                                                 const cplx &r, double sg) {
+    return {v.x - fmav(a.cxx, c.x, sg * (a.cxy * (l.y - r.y))), v.y - fmav(a.cyy, c.y, sg * (a.cxy * (l.x - r.x)))};
+}
+
+// transform the R rows in `buf` (interior rows j0 ..) and store their modes:
+// twice those of u and of v' = -i v, from those of u + i v
+template <int MT, int R>
+__device__ __forceinline__ static void store_modes(const FourierArgs &a, cplx *buf, int j0) {
+    constexpr int NT = kRowThreads * R;
     const int M = MT > 0 ? MT : a.M, N = a.N, K = M / 2 + 1;
-    const cplx *src = reinterpret_cast<const cplx *>(src2);
-    const int j0 = 1 + kRows * blk;
-    for (int t = threadIdx.x; t < kRows * M; t += kRowThreads) {
-        const int row = t / M, i = t - row * M, j = j0 + row;
-        cplx v = {0, 0};
-        if (j <= N) {
-            v = src[(size_t)i + (size_t)M * j];
-            if (j == 1 || j == N) {
-                const int il = i == 0 ? M - 1 : i - 1, ir = i == M - 1 ? 0 : i + 1;
-                if (j == 1) {
-                    const cplx c = wall_node(a, src, i, 0), l = wall_node(a, src, il, 0), r = wall_node(a, src, ir, 0);
-                    v.x -= a.cxx * c.x + a.cxy * (l.y - r.y);
-                    v.y -= a.cyy * c.y + a.cxy * (l.x - r.x);
-                }
-                if (j == N) {
-                    const cplx c = wall_node(a, src, i, N + 1), l = wall_node(a, src, il, N + 1),
-                               r = wall_node(a, src, ir, N + 1);
-                    v.x -= a.cxx * c.x + a.cxy * (r.y - l.y);
-                    v.y -= a.cyy * c.y + a.cxy * (r.x - l.x);
-                }
-            }
-        }
-        buf[row * fpad(M) + fpad(i)] = v;
-    }
-    __syncthreads();
-    const cplx *c = transform_rows<MT>(a, buf);
-    // twice the modes of u and of v' = -i v from those of u + i v
+    const cplx *c = transform_rows<MT, R>(a, buf);
     double2 *S = reinterpret_cast<double2 *>(a.S);
-    for (int t = threadIdx.x; t < kRows * K; t += kRowThreads) {
-        const int row = t % kRows, k = t / kRows, j = j0 - 1 + row;
+    for (int t = threadIdx.x; t < R * K; t += NT) {
+        const int row = t % R, k = t / R, j = j0 - 1 + row;
         if (j >= N) continue;
         const cplx p = c[row * fpad(M) + fpad(k)], q = c[row * fpad(M) + fpad(k == 0 ? 0 : M - k)];
-        double2 *o = S + 2 * ((size_t)k * N + j);
+        double2 *o = S + 2 * ((size_t)k * a.NP + j);
         o[0] = make_double2(p.x + q.x, p.y - q.y);
         o[1] = make_double2(q.x - p.x, -p.y - q.y);
     }
 }
 
-// inverse launch body: the modes of kRows interior rows back to (u, v),
+// forward launch body: interior rows 1 + R * blk .. of the source
+template <int MT, int R>
+__device__ __forceinline__ static void fourier_forward_body(const FourierArgs &a, const double *__restrict__ src2,
+                                                            int blk) {
+    extern __shared__ __align__(16) unsigned char fourier_smem[];
+    constexpr int NT = kRowThreads * R;
+    cplx *buf = reinterpret_cast<cplx *>(fourier_smem);
+    const int M = MT > 0 ? MT : a.M, N = a.N;
+    const cplx *src = reinterpret_cast<const cplx *>(src2);
+    const int j0 = 1 + R * blk;
+    for (int t = threadIdx.x; t < R * M; t += NT) {
+        const int row = t / M, i = t - row * M, j = j0 + row;
+        cplx v = {0, 0};
+        if (j <= N) {
+            v = src[(size_t)i + (size_t)M * j];
+            const int il = i == 0 ? M - 1 : i - 1, ir = i == M - 1 ? 0 : i + 1;
+            if (j == 1)
+                v = less_wall(a, v, wall_node(a, src, i, 0), wall_node(a, src, il, 0), wall_node(a, src, ir, 0), 1);
+            if (j == N)
+                v = less_wall(a, v, wall_node(a, src, i, N + 1), wall_node(a, src, il, N + 1),
+                              wall_node(a, src, ir, N + 1), -1);
+        }
+        buf[row * fpad(M) + fpad(i)] = v;
+    }
+    __syncthreads();
+    store_modes<MT, R>(a, buf, j0);
+}
+
+// the same with the source formed here (shear_sim.cc:399-409, node_force)
+// and written on the way, which saves reading it back: a thread runs down a
+// column, so each stress is loaded once for the two rows it enters
+template <int MT, int R>
+__device__ __forceinline__ static void fourier_source_body(const FourierArgs &a, const SourceArgs &f,
+                                                           double *__restrict__ src2, int blk) {
+    extern __shared__ __align__(16) unsigned char fourier_smem[];
+    constexpr int NT = kRowThreads * R;
+    cplx *buf = reinterpret_cast<cplx *>(fourier_smem);
+    const int M = MT > 0 ? MT : a.M, N = a.N;
+    cplx *src = reinterpret_cast<cplx *>(src2);
+    const int j0 = 1 + R * blk;
+    const cplx low = {-f.wall, 0}, high = {f.wall, 0};
+    for (int i = threadIdx.x; i < M; i += NT) {
+        const int il = i == 0 ? M - 1 : i - 1;
+        // cell rows j - 1 (plane row j) and j
+        double p[4][R + 1], q[4][2];
+#pragma unroll
+        for (int row = 0; row <= R; row++) {
+            const size_t o = (size_t)M * min(j0 + row, N + 1);
+#pragma unroll
+            for (int k = 0; k < 4; k++) p[k][row] = f.f[k][o + i];
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) q[k][1] = f.f[k][(size_t)M * j0 + il];
+#pragma unroll
+        for (int row = 0; row < R; row++) {
+            const int j = j0 + row;
+#pragma unroll
+            for (int k = 0; k < 4; k++) {
+                q[k][0] = q[k][1];
+                q[k][1] = f.f[k][(size_t)M * min(j + 1, N + 1) + il];
+            }
+            cplx v = {0, 0};
+            if (j <= N) {
+                node_force(q[0][0], p[0][row], q[0][1], p[0][row + 1], q[1][0], p[1][row], q[1][1], p[1][row + 1],
+                           q[2][0], p[2][row], q[2][1], p[2][row + 1], q[3][0], p[3][row], q[3][1], p[3][row + 1],
+                           f.xfac, f.yfac, v.x, v.y);
+                src[(size_t)i + (size_t)M * j] = v;
+                if (j == 1) {
+                    const cplx w = {a.wix * low.x, a.wiy * low.y};
+                    v = less_wall(a, v, w, w, w, 1);
+                }
+                if (j == N) {
+                    const cplx w = {a.wix * high.x, a.wiy * high.y};
+                    v = less_wall(a, v, w, w, w, -1);
+                }
+            }
+            buf[row * fpad(M) + fpad(i)] = v;
+        }
+        if (blk == 0) {
+            src[i] = low;
+            src[(size_t)i + (size_t)M * (N + 1)] = high;
+        }
+    }
+    __syncthreads();
+    store_modes<MT, R>(a, buf, j0);
+}
+
+// inverse launch body: the modes of R interior rows back to (u, v),
 // stored (or added); the first workgroup also writes the wall rows
-template <int MT>
+template <int MT, int R>
 __device__ __forceinline__ static void fourier_inverse_body(const FourierArgs &a, const double *__restrict__ src2,
                                                             double *__restrict__ z2, bool add, int blk) {
+    constexpr int NT = kRowThreads * R;
     extern __shared__ __align__(16) unsigned char fourier_smem[];
     cplx *buf = reinterpret_cast<cplx *>(fourier_smem);
     const int M = MT > 0 ? MT : a.M, N = a.N, K = M / 2 + 1;
-    const int j0 = 1 + kRows * blk;
+    const int j0 = 1 + R * blk;
     const double2 *S = reinterpret_cast<const double2 *>(a.S);
     cplx *z = reinterpret_cast<cplx *>(z2);
     // conjugates of the modes of u + i v, so that the forward transform is
     // the conjugate of the inverse one
-    for (int t = threadIdx.x; t < kRows * K; t += kRowThreads) {
-        const int row = t % kRows, k = t / kRows, j = j0 - 1 + row;
+    for (int t = threadIdx.x; t < R * K; t += NT) {
+        const int row = t % R, k = t / R, j = j0 - 1 + row;
         double2 u = make_double2(0, 0), w = u;
         if (j < N) {
-            const double2 *s = S + 2 * ((size_t)k * N + j);
+            const double2 *s = S + 2 * ((size_t)k * a.NP + j);
             u = s[0];
             w = s[1];
         }
@@ -308,9 +397,9 @@ __device__ __forceinline__ static void fourier_inverse_body(const FourierArgs &a
         if (k > 0 && 2 * k < M) buf[row * fpad(M) + fpad(M - k)] = {u.x + w.x, u.y + w.y};
     }
     __syncthreads();
-    const cplx *c = transform_rows<MT>(a, buf);
+    const cplx *c = transform_rows<MT, R>(a, buf);
     const double sc = 0.5 / M;
-    for (int t = threadIdx.x; t < kRows * M; t += kRowThreads) {
+    for (int t = threadIdx.x; t < R * M; t += NT) {
         const int row = t / M, i = t - row * M, j = j0 + row;
         if (j > N) continue;
         const cplx v = c[row * fpad(M) + fpad(i)];
@@ -320,7 +409,7 @@ __device__ __forceinline__ static void fourier_inverse_body(const FourierArgs &a
     }
     if (blk == 0) {
         const cplx *src = reinterpret_cast<const cplx *>(src2);
-        for (int t = threadIdx.x; t < 2 * M; t += kRowThreads) {
+        for (int t = threadIdx.x; t < 2 * M; t += NT) {
             const int i = t % M, j = t < M ? 0 : N + 1;
             const cplx w = wall_node(a, src, i, j);
             cplx *o = z + (size_t)i + (size_t)M * j;
@@ -338,65 +427,64 @@ __device__ __forceinline__ static void fourier_inverse_body(const FourierArgs &a
 constexpr int kModePow = 7;
 constexpr int kModeTab = 4 * (3 + kModePow);
 
-struct v4 { double ux, uy, wx, wy; };  // (u, v') of a row, complex
+// (u, v') of a row: its real or its imaginary part.  The two are solved by
+// waves of their own (the blocks are real), which halves the registers and
+// lane exchanges of each and doubles the waves in flight.
+struct v2 { double u, w; };
 
-// r = A x + r with A row-major 2x2 acting on (u, v')
-__device__ __forceinline__ static void mad2(const double *A, const v4 &x, v4 &r) {
-    r.ux = fmav(A[1], x.wx, fmav(A[0], x.ux, r.ux));
-    r.uy = fmav(A[1], x.wy, fmav(A[0], x.uy, r.uy));
-    r.wx = fmav(A[3], x.wx, fmav(A[2], x.ux, r.wx));
-    r.wy = fmav(A[3], x.wy, fmav(A[2], x.uy, r.wy));
+// r += A x with A row-major 2x2 acting on (u, v')
+__device__ __forceinline__ static void mad2(const double *A, const v2 &x, v2 &r) {
+    r.u = fmav(A[1], x.w, fmav(A[0], x.u, r.u));
+    r.w = fmav(A[3], x.w, fmav(A[2], x.u, r.w));
 }
-__device__ __forceinline__ static void mad2t(const double *A, const v4 &x, v4 &r) {  // transpose
-    r.ux = fmav(A[2], x.wx, fmav(A[0], x.ux, r.ux));
-    r.uy = fmav(A[2], x.wy, fmav(A[0], x.uy, r.uy));
-    r.wx = fmav(A[3], x.wx, fmav(A[1], x.ux, r.wx));
-    r.wy = fmav(A[3], x.wy, fmav(A[1], x.uy, r.wy));
+__device__ __forceinline__ static void mad2t(const double *A, const v2 &x, v2 &r) {  // transpose
+    r.u = fmav(A[2], x.w, fmav(A[0], x.u, r.u));
+    r.w = fmav(A[3], x.w, fmav(A[1], x.u, r.w));
 }
-__device__ __forceinline__ static v4 mul2(const double *A, const v4 &x) {
-    v4 r = {0, 0, 0, 0};
+__device__ __forceinline__ static v2 mul2(const double *A, const v2 &x) {
+    v2 r = {0, 0};
     mad2(A, x, r);
     return r;
 }
-template <bool UP> __device__ __forceinline__ static v4 lane_shift(const v4 &x, int d) {
+template <bool UP> __device__ __forceinline__ static v2 lane_shift(const v2 &x, int d) {
     // the value d lanes below (UP) or above; zero past the wave's end
     const int lane = threadIdx.x & 63;
-    v4 r;
+    v2 r;
     if (UP) {
-        r = {__shfl_up(x.ux, d, 64), __shfl_up(x.uy, d, 64), __shfl_up(x.wx, d, 64), __shfl_up(x.wy, d, 64)};
-        if (lane < d) r = {0, 0, 0, 0};
+        r = {__shfl_up(x.u, d, 64), __shfl_up(x.w, d, 64)};
+        if (lane < d) r = {0, 0};
     } else {
-        r = {__shfl_down(x.ux, d, 64), __shfl_down(x.uy, d, 64), __shfl_down(x.wx, d, 64),
-             __shfl_down(x.wy, d, 64)};
-        if (lane + d >= 64) r = {0, 0, 0, 0};
+        r = {__shfl_down(x.u, d, 64), __shfl_down(x.w, d, 64)};
+        if (lane + d >= 64) r = {0, 0};
     }
     return r;
 }
 
 // carry into each lane of a recurrence whose lanes' own results are `t`:
 // the inclusive scan of t with the factor F^P per lane (or its transpose,
-// backwards), shifted by one lane; W waves combined through `xw` in LDS
+// backwards), shifted by one lane; the W waves of a part combined through
+// `xw` in LDS (`wave`: this one of them)
 template <int W, bool UP>
-__device__ __forceinline__ static v4 scan_carry(const double *pw, v4 t, v4 *xw) {
+__device__ __forceinline__ static v2 scan_carry(const double *pw, v2 t, v2 *xw, int wave) {
 #pragma unroll
     for (int s = 0; s < 6; s++) {
-        const v4 n = lane_shift<UP>(t, 1 << s);
+        const v2 n = lane_shift<UP>(t, 1 << s);
         if (UP) mad2(pw + 4 * s, n, t);
         else mad2t(pw + 4 * s, n, t);
     }
-    v4 c = lane_shift<UP>(t, 1);
+    v2 c = lane_shift<UP>(t, 1);
     if constexpr (W > 1) {
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+        const int lane = threadIdx.x & 63;
         __syncthreads();
         if (lane == (UP ? 63 : 0)) xw[wave] = t;
         __syncthreads();
         // the waves before (after) this one, combined in their order
-        v4 in = {0, 0, 0, 0};
+        v2 in = {0, 0};
 #pragma unroll
         for (int q = 0; q < W - 1; q++) {
             const int w = UP ? q : W - 1 - q;
             if (UP ? w < wave : w > wave) {
-                v4 r = xw[w];
+                v2 r = xw[w];
                 if (UP) mad2(pw + 4 * 6, in, r);
                 else mad2t(pw + 4 * 6, in, r);
                 in = r;
@@ -407,114 +495,110 @@ __device__ __forceinline__ static v4 scan_carry(const double *pw, v4 t, v4 *xw) 
 #pragma unroll
         for (int s = 0; s < 6; s++)
             if ((d >> s) & 1) {
-                v4 r = {0, 0, 0, 0};
+                v2 r = {0, 0};
                 if (UP) mad2(pw + 4 * s, in, r);
                 else mad2t(pw + 4 * s, in, r);
                 in = r;
             }
-        c = {c.ux + in.ux, c.uy + in.uy, c.wx + in.wx, c.wy + in.wy};
+        c = {c.u + in.u, c.w + in.w};
     }
     return c;
 }
 
 // LDS column of a mode: row j of P rows per thread at slot 2 j + (j / P), in
-// 16-byte units: a thread's rows are contiguous and threads start one slot
-// apart in the banks
+// 16-byte units (u complex, v' complex): a thread's rows are contiguous and
+// threads start one slot apart in the banks
 template <int P> __host__ __device__ constexpr int mode_slot(int j) { return 2 * j + j / P; }
 
 template <int W, int P>
 __device__ __forceinline__ static void fourier_mode_body(const FourierArgs &a, int k) {
     extern __shared__ __align__(16) unsigned char fourier_smem[];
-    constexpr int NT = 64 * W, ROWS = NT * P;
+    constexpr int NT = 128 * W;
     double2 *col = reinterpret_cast<double2 *>(fourier_smem);
-    __shared__ v4 xw[W];
-    __shared__ v4 first;
+    __shared__ v2 xw[2][W];
+    __shared__ v2 first[2];
     const int N = a.N, tid = threadIdx.x;
+    const int part = tid / (64 * W), ln = tid % (64 * W);  // real or imaginary part; lane of it
+    const int wave = ln >> 6;
     const double *tab = a.tab + (size_t)kModeTab * k;
     const double *F = tab, *Di = tab + 4, *C = tab + 8, *pw = tab + 12;
-    double2 *S = reinterpret_cast<double2 *>(a.S) + (size_t)2 * k * N;
+    double2 *S = reinterpret_cast<double2 *>(a.S) + (size_t)2 * k * a.NP;
     // the column, coalesced, all of a thread's loads in flight
-    double2 in[2 * P];
+    double2 in[P];
 #pragma unroll
-    for (int q = 0; q < 2 * P; q++) {
+    for (int q = 0; q < P; q++) {
         const int t = tid + NT * q;
         in[q] = S[t < 2 * N ? t : 0];
     }
 #pragma unroll
-    for (int q = 0; q < 2 * P; q++) {
+    for (int q = 0; q < P; q++) {
         const int t = tid + NT * q;
         col[mode_slot<P>(t >> 1) + (t & 1)] = t < 2 * N ? in[q] : make_double2(0, 0);
     }
     __syncthreads();
-    v4 g[P];
-    const int r0 = tid * P;
+    v2 g[P];
+    const int r0 = ln * P;
+    // this part of the thread's rows (u at even, v' at odd places)
+    double *mine = reinterpret_cast<double *>(col + mode_slot<P>(r0)) + part;
 #pragma unroll
-    for (int p = 0; p < P; p++) {
-        const double2 u = col[mode_slot<P>(r0) + 2 * p], w = col[mode_slot<P>(r0) + 2 * p + 1];
-        g[p] = {u.x, u.y, w.x, w.y};
-    }
-    static_assert(ROWS > 0, "rows");
+    for (int p = 0; p < P; p++) g[p] = {mine[4 * p], mine[4 * p + 2]};
     // forward: g_j = f_j + F g_{j-1}
 #pragma unroll
     for (int p = 1; p < P; p++) mad2(F, g[p - 1], g[p]);
-    v4 c = scan_carry<W, true>(pw, g[P - 1], xw);
+    v2 c = scan_carry<W, true>(pw, g[P - 1], xw[part], wave);
 #pragma unroll
     for (int p = 0; p < P; p++) {
         c = mul2(F, c);
-        g[p] = {g[p].ux + c.ux, g[p].uy + c.uy, g[p].wx + c.wx, g[p].wy + c.wy};
-        if (r0 + p >= N) g[p] = {0, 0, 0, 0};
+        g[p] = {g[p].u + c.u, g[p].w + c.w};
+        if (r0 + p >= N) g[p] = {0, 0};
     }
     // backward for the first row only: y_1
-    v4 y = mul2(Di, g[P - 1]);
+    v2 y = mul2(Di, g[P - 1]);
 #pragma unroll
     for (int p = P - 2; p >= 0; p--) {
-        v4 t = mul2(Di, g[p]);
+        v2 t = mul2(Di, g[p]);
         mad2t(F, y, t);
         y = t;
     }
-    v4 t0 = scan_carry<W, false>(pw, y, xw);
-    if (tid == 0) {
+    v2 t0 = scan_carry<W, false>(pw, y, xw[part], wave);
+    if (ln == 0) {
         // y_1 = this thread's own part + E^P times the carry from the next
         mad2t(pw, t0, y);
-        first = mul2(C, y);  // -P w_1
+        first[part] = mul2(C, y);  // -P w_1
     }
     __syncthreads();
     // g_j += F^{j-1} (-P w_1)
-    v4 h = first;
+    v2 h = first[part];
 #pragma unroll
     for (int s = 0; s < 6; s++)
-        if ((tid >> s) & 1) h = mul2(pw + 4 * s, h);
+        if ((ln >> s) & 1) h = mul2(pw + 4 * s, h);
     if constexpr (W > 1)
-        for (int w = 0; w < (tid >> 6); w++) h = mul2(pw + 4 * 6, h);
+        for (int w = 0; w < wave; w++) h = mul2(pw + 4 * 6, h);
 #pragma unroll
     for (int p = 0; p < P; p++) {
-        if (r0 + p < N) g[p] = {g[p].ux + h.ux, g[p].uy + h.uy, g[p].wx + h.wx, g[p].wy + h.wy};
+        if (r0 + p < N) g[p] = {g[p].u + h.u, g[p].w + h.w};
         h = mul2(F, h);
     }
     // backward: w_j = D^{-1} g_j + E w_{j+1}
     g[P - 1] = mul2(Di, g[P - 1]);
 #pragma unroll
     for (int p = P - 2; p >= 0; p--) {
-        v4 t = mul2(Di, g[p]);
+        v2 t = mul2(Di, g[p]);
         mad2t(F, g[p + 1], t);
         g[p] = t;
     }
-    c = scan_carry<W, false>(pw, g[0], xw);
+    c = scan_carry<W, false>(pw, g[0], xw[part], wave);
 #pragma unroll
     for (int p = P - 1; p >= 0; p--) {
-        v4 t = {0, 0, 0, 0};
+        v2 t = {0, 0};
         mad2t(F, c, t);
         c = t;
-        g[p] = {g[p].ux + c.ux, g[p].uy + c.uy, g[p].wx + c.wx, g[p].wy + c.wy};
-    }
-#pragma unroll
-    for (int p = 0; p < P; p++) {
-        col[mode_slot<P>(r0) + 2 * p] = make_double2(g[p].ux, g[p].uy);
-        col[mode_slot<P>(r0) + 2 * p + 1] = make_double2(g[p].wx, g[p].wy);
+        mine[4 * p] = g[p].u + c.u;
+        mine[4 * p + 2] = g[p].w + c.w;
     }
     __syncthreads();
 #pragma unroll
-    for (int q = 0; q < 2 * P; q++) {
+    for (int q = 0; q < P; q++) {
         const int t = tid + NT * q;
         if (t < 2 * N) S[t] = col[mode_slot<P>(t >> 1) + (t & 1)];
     }
@@ -523,16 +607,20 @@ __device__ __forceinline__ static void fourier_mode_body(const FourierArgs &a, i
 // ---------------------------------------------------------------------------
 // kernels
 // ---------------------------------------------------------------------------
-template <int MT>
-__global__ void __launch_bounds__(kRowThreads) fourier_forward_kernel(FourierArgs a, const double *src) {
-    fourier_forward_body<MT>(a, src, blockIdx.x);
+template <int MT, int R>
+__global__ void __launch_bounds__(kRowThreads *R) fourier_forward_kernel(FourierArgs a, const double *src) {
+    fourier_forward_body<MT, R>(a, src, blockIdx.x);
 }
-template <int MT>
-__global__ void __launch_bounds__(kRowThreads) fourier_inverse_kernel(FourierArgs a, const double *src, double *z,
-                                                                      bool add) {
-    fourier_inverse_body<MT>(a, src, z, add, blockIdx.x);
+template <int MT, int R>
+__global__ void __launch_bounds__(kRowThreads *R) fourier_source_kernel(FourierArgs a, SourceArgs f, double *src) {
+    fourier_source_body<MT, R>(a, f, src, blockIdx.x);
 }
-template <int W, int P> __global__ void __launch_bounds__(64 * W) fourier_mode_kernel(FourierArgs a) {
+template <int MT, int R>
+__global__ void __launch_bounds__(kRowThreads *R) fourier_inverse_kernel(FourierArgs a, const double *src, double *z,
+                                                                         bool add) {
+    fourier_inverse_body<MT, R>(a, src, z, add, blockIdx.x);
+}
+template <int W, int P> __global__ void __launch_bounds__(128 * W) fourier_mode_kernel(FourierArgs a) {
     fourier_mode_body<W, P>(a, blockIdx.x);
 }
 
@@ -540,27 +628,27 @@ template <int W, int P> __global__ void __launch_bounds__(64 * W) fourier_mode_k
 // members whose slot flag is clear return at once, and those past their first
 // test solve for the residual and add
 template <int MT>
-__global__ void __launch_bounds__(kRowThreads) fourier_forward_batch_kernel(const FourierEntry *E, const int *map,
-                                                                            const EnsState *St) {
+__global__ void __launch_bounds__(2 * kRowThreads) fourier_forward_batch_kernel(const FourierEntry *E, const int *map,
+                                                                                const EnsState *St) {
     const int2 el = batch_slot(map, blockIdx.x);
     const FourierEntry &x = E[el.x];
     if (!St[x.member].active) return;
     const FourierArgs a = x.a;
-    fourier_forward_body<MT>(a, St[x.member].phase == ENS_LOOP ? x.r : x.src, el.y);
+    fourier_forward_body<MT, 2>(a, St[x.member].phase == ENS_LOOP ? x.r : x.src, el.y);
 }
 template <int MT>
-__global__ void __launch_bounds__(kRowThreads) fourier_inverse_batch_kernel(const FourierEntry *E, const int *map,
-                                                                            const EnsState *St) {
+__global__ void __launch_bounds__(2 * kRowThreads) fourier_inverse_batch_kernel(const FourierEntry *E, const int *map,
+                                                                                const EnsState *St) {
     const int2 el = batch_slot(map, blockIdx.x);
     const FourierEntry &x = E[el.x];
     if (!St[x.member].active) return;
     const FourierArgs a = x.a;
     const bool add = St[x.member].phase == ENS_LOOP;
-    fourier_inverse_body<MT>(a, add ? x.r : x.src, x.z, add, el.y);
+    fourier_inverse_body<MT, 2>(a, add ? x.r : x.src, x.z, add, el.y);
 }
 template <int W, int P>
-__global__ void __launch_bounds__(64 * W) fourier_mode_batch_kernel(const FourierEntry *E, const int *map,
-                                                                    const EnsState *St) {
+__global__ void __launch_bounds__(128 * W) fourier_mode_batch_kernel(const FourierEntry *E, const int *map,
+                                                                     const EnsState *St) {
     const int2 el = batch_slot(map, blockIdx.x);
     const FourierEntry &x = E[el.x];
     if (!St[x.member].active) return;
@@ -574,10 +662,13 @@ __global__ void __launch_bounds__(64 * W) fourier_mode_batch_kernel(const Fourie
 // lengths with the in-place transform of compile-time length
 static bool fixed_length(int M) { return M == 128 || M == 256 || M == 512 || M == 1024 || M == 2048 || M == 4096; }
 
-size_t fourier_row_lds(int M) { return (size_t)(fixed_length(M) ? 1 : 2) * kRows * fpad(M) * sizeof(cplx); }
+// rows per workgroup of a grid's own launches
+static int row_group(int M, int N) { return fixed_length(M) && M >= 512 && M <= 2048 && N >= 4 * 255 ? 4 : 2; }
+static size_t row_lds(int M, int R) { return (size_t)(fixed_length(M) ? 1 : 2) * R * fpad(M) * sizeof(cplx); }
+size_t fourier_row_lds(int M) { return row_lds(M, 2); }
 
-// rows per thread and waves per mode: eight rows a thread, fewer where one
-// wave then covers the column
+// rows per thread and waves per part of a mode: eight rows a thread, fewer
+// where one wave then covers the column
 static int mode_rows(int N) { return N <= 128 ? 2 : (N <= 256 ? 4 : 8); }
 static int mode_waves(int N) { return N <= 512 ? 1 : (N <= 1024 ? 2 : (N <= 2048 ? 4 : 8)); }
 size_t fourier_mode_lds(int N) {
@@ -621,16 +712,31 @@ template <typename K> static int allow_lds(K kernel, size_t bytes) {
     return STZ_OK;
 }
 
+// f(integral_constant) of the rows per workgroup of a grid's own launches:
+// four only with the lengths row_group gives them to
+template <int MT, typename F> static int with_rows(int M, int N, F f) {
+    if constexpr (MT >= 512 && MT <= 2048)
+        if (row_group(M, N) == 4) return f(std::integral_constant<int, 4>());
+    return f(std::integral_constant<int, 2>());
+}
+
 // raise the LDS limit of the kernels a grid uses (once per operator set-up)
 int fourier_set_lds_limit(const FourierArgs &a) {
-    const size_t rl = fourier_row_lds(a.M), ml = fourier_mode_lds(a.N);
+    const size_t ml = fourier_mode_lds(a.N);
     const int e = with_length(a.M, [&](auto mt) {
         constexpr int MT = decltype(mt)::value;
         int r;
-        if ((r = allow_lds(fourier_forward_kernel<MT>, rl)) || (r = allow_lds(fourier_inverse_kernel<MT>, rl)) ||
-            (r = allow_lds(fourier_forward_batch_kernel<MT>, rl)))
+        if ((r = allow_lds(fourier_forward_batch_kernel<MT>, fourier_row_lds(a.M))) ||
+            (r = allow_lds(fourier_inverse_batch_kernel<MT>, fourier_row_lds(a.M))))
             return r;
-        return allow_lds(fourier_inverse_batch_kernel<MT>, rl);
+        return with_rows<MT>(a.M, a.N, [&](auto rr) {
+            constexpr int R = decltype(rr)::value;
+            const size_t rl = row_lds(a.M, R);
+            int q;
+            if ((q = allow_lds(fourier_forward_kernel<MT, R>, rl)) || (q = allow_lds(fourier_source_kernel<MT, R>, rl)))
+                return q;
+            return allow_lds(fourier_inverse_kernel<MT, R>, rl);
+        });
     });
     if (e) return e;
     return with_column(a.N, [&](auto w, auto p) {
@@ -640,26 +746,36 @@ int fourier_set_lds_limit(const FourierArgs &a) {
     });
 }
 
-int fourier_row_workgroups(int N) { return (N + kRows - 1) / kRows; }
+int fourier_row_workgroups(int N) { return (N + 1) / 2; }
 int fourier_row_variant(int M) { return fixed_length(M) ? M : 0; }
 int fourier_mode_variant(int N) { return 16 * mode_waves(N) + mode_rows(N); }
 
-// z = A^{-1} src, or (add) z += A^{-1} src
-int mg_fourier_solve(const FourierArgs &a, const double *src, double *z, bool add, hipStream_t st) {
-    const dim3 g(fourier_row_workgroups(a.N)), b(kRowThreads);
-    const size_t rl = fourier_row_lds(a.M), ml = fourier_mode_lds(a.N);
-    with_length(a.M, [&](auto mt) {
-        hipLaunchKernelGGL((fourier_forward_kernel<decltype(mt)::value>), g, b, rl, st, a, src);
-        return 0;
+// z = A^{-1} src, or (add) z += A^{-1} src; with f the source is formed first
+int mg_fourier_solve(const FourierArgs &a, const SourceArgs *f, double *src, double *z, bool add, hipStream_t st) {
+    const size_t ml = fourier_mode_lds(a.N);
+    auto rows = [&](auto launch) {
+        with_length(a.M, [&](auto mt) {
+            constexpr int MT = decltype(mt)::value;
+            return with_rows<MT>(a.M, a.N, [&](auto rr) {
+                constexpr int R = decltype(rr)::value;
+                launch(mt, rr, dim3((a.N + R - 1) / R), dim3(kRowThreads * R), row_lds(a.M, R));
+                return 0;
+            });
+        });
+    };
+    rows([&](auto mt, auto rr, dim3 g, dim3 b, size_t lds) {
+        constexpr int MT = decltype(mt)::value, R = decltype(rr)::value;
+        if (f) hipLaunchKernelGGL((fourier_source_kernel<MT, R>), g, b, lds, st, a, *f, src);
+        else hipLaunchKernelGGL((fourier_forward_kernel<MT, R>), g, b, lds, st, a, (const double *)src);
     });
     with_column(a.N, [&](auto w, auto p) {
         constexpr int W = decltype(w)::value, P = decltype(p)::value;
-        hipLaunchKernelGGL((fourier_mode_kernel<W, P>), dim3(a.M / 2 + 1), dim3(64 * W), ml, st, a);
+        hipLaunchKernelGGL((fourier_mode_kernel<W, P>), dim3(a.M / 2 + 1), dim3(128 * W), ml, st, a);
         return 0;
     });
-    with_length(a.M, [&](auto mt) {
-        hipLaunchKernelGGL((fourier_inverse_kernel<decltype(mt)::value>), g, b, rl, st, a, src, z, add);
-        return 0;
+    rows([&](auto mt, auto rr, dim3 g, dim3 b, size_t lds) {
+        constexpr int MT = decltype(mt)::value, R = decltype(rr)::value;
+        hipLaunchKernelGGL((fourier_inverse_kernel<MT, R>), g, b, lds, st, a, (const double *)src, z, add);
     });
     STZ_HIP(hipGetLastError());
     return STZ_OK;
@@ -671,9 +787,9 @@ int batch_fourier_rows(bool inverse, int M, size_t lds, const FourierEntry *E, c
     with_length(M, [&](auto mt) {
         constexpr int MT = decltype(mt)::value;
         if (inverse)
-            hipLaunchKernelGGL((fourier_inverse_batch_kernel<MT>), dim3(total), dim3(kRowThreads), lds, st, E, map, St);
+            hipLaunchKernelGGL((fourier_inverse_batch_kernel<MT>), dim3(total), dim3(2 * kRowThreads), lds, st, E, map, St);
         else
-            hipLaunchKernelGGL((fourier_forward_batch_kernel<MT>), dim3(total), dim3(kRowThreads), lds, st, E, map, St);
+            hipLaunchKernelGGL((fourier_forward_batch_kernel<MT>), dim3(total), dim3(2 * kRowThreads), lds, st, E, map, St);
         return 0;
     });
     STZ_HIP(hipGetLastError());
@@ -686,7 +802,7 @@ int batch_fourier_modes(int N, const FourierEntry *E, const int *map, int total,
     const size_t ml = fourier_mode_lds(N);
     with_column(N, [&](auto w, auto p) {
         constexpr int W = decltype(w)::value, P = decltype(p)::value;
-        hipLaunchKernelGGL((fourier_mode_batch_kernel<W, P>), dim3(total), dim3(64 * W), ml, st, E, map, St);
+        hipLaunchKernelGGL((fourier_mode_batch_kernel<W, P>), dim3(total), dim3(128 * W), ml, st, E, map, St);
         return 0;
     });
     STZ_HIP(hipGetLastError());
@@ -713,18 +829,25 @@ m2 inv(const m2 &x) {
 real big(const m2 &x) { return std::fmax(std::fmax(std::fabs(x.a), std::fabs(x.b)), std::fmax(std::fabs(x.c), std::fabs(x.d))); }
 }  // namespace
 
-size_t fourier_spectrum_elems(int M, int N) { return (size_t)4 * (M / 2 + 1) * N; }
-size_t fourier_table_elems(int M) { return (size_t)2 * M + (size_t)kModeTab * (M / 2 + 1); }
+size_t fourier_spectrum_elems(int M, int N) { return (size_t)4 * (M / 2 + 1) * ((N + 3) & ~3); }
+static size_t table_elems(int M) { return (size_t)4 * M + (size_t)kModeTab * (M / 2 + 1); }
 
 // The constants of the solve for M x (N + 2) nodes with the interior stencil
 // s40 and the wall rows' stencil w40 (sim.hip, top_row_stencil): T receives
-// the M roots of unity e^{-2 pi i m / M} and the mode tables.  Returns false
+// the stages' twiddles, the M roots of unity e^{-2 pi i m / M} and, from element
+// 4 M on, the mode tables.  Returns false
 // if the operator does not have the form above or a mode is singular.
 bool fourier_setup(const double *s40, const double *w40, int M, int N, FourierArgs &a, std::vector<double> &T) {
     a.M = M;
     a.N = N;
+    a.NP = (N + 3) & ~3;
     a.nst = 0;
     int left = M;
+    if (fixed_length(M))
+        while (left > 1) {
+            a.radix[a.nst++] = fixed_radix(left);
+            left /= fixed_radix(left);
+        }
     for (int r : {4, 2, 3, 5})
         while (left % r == 0) {
             a.radix[a.nst++] = r;
@@ -749,15 +872,22 @@ bool fourier_setup(const double *s40, const double *w40, int M, int N, FourierAr
     a.cxy = s40[1];
     a.wix = w40[36];
     a.wiy = w40[39];
-    T.assign(fourier_table_elems(M), 0.0);
+    T.assign(table_elems(M), 0.0);
     const real pi = 3.14159265358979323846264338327950288L;
+    double *root = T.data() + 2 * (size_t)M;
     for (int m = 0; m < M; m++) {
-        // octant symmetry is not needed: sine and cosine in extended
-        // precision are correctly rounded to double all but always
         const real th = 2 * pi * m / M;
-        T[2 * m] = (double)std::cos(th);
-        T[2 * m + 1] = (double)-std::sin(th);
+        root[2 * m] = (double)std::cos(th);
+        root[2 * m + 1] = (double)-std::sin(th);
     }
+    // the stage after a product of L: entries (q - 1) L + k from L - 1 on
+    for (int s = 0, L = 1; s < a.nst; L *= a.radix[s++])
+        for (int q = 1; q < a.radix[s]; q++)
+            for (int k = 0; k < L; k++) {
+                const size_t o = (size_t)(L - 1) + (size_t)(q - 1) * L + k, r = (size_t)k * q * (M / (L * a.radix[s]));
+                T[2 * o] = root[2 * r];
+                T[2 * o + 1] = root[2 * r + 1];
+            }
     const int P = mode_rows(N);
     const real e0 = (real)s40[16] + 2 * xx + 2 * yx, e1 = (real)s40[19] + 2 * xy + 2 * yy;  // row sums: rounding
     for (int k = 0; k <= M / 2; k++) {
@@ -799,7 +929,7 @@ bool fourier_setup(const double *s40, const double *w40, int M, int N, FourierAr
         const m2 Pm = k == 0 ? m2{-yx, 0, 0, -yy} : B - D;
         const m2 one = {1, 0, 0, 1};
         const m2 Cm = neg(Pm * inv(one + G * Pm));
-        double *t = T.data() + 2 * (size_t)M + (size_t)kModeTab * k;
+        double *t = T.data() + 4 * (size_t)M + (size_t)kModeTab * k;
         auto put = [](double *o, const m2 &x) {
             o[0] = (double)x.a;
             o[1] = (double)x.b;

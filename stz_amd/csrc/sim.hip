@@ -452,7 +452,7 @@ static int set_fourier(stz_sim *s) {
     if (!s->fspec) STZ_HIP(hipMalloc(&s->fspec, fourier_spectrum_elems(M, n - 2) * sizeof(double)));
     STZ_HIP(hipMemcpy(s->ftab, T.data(), T.size() * sizeof(double), hipMemcpyHostToDevice));
     s->fa.tw = s->ftab;
-    s->fa.tab = s->ftab + 2 * (size_t)M;
+    s->fa.tab = s->ftab + 4 * (size_t)M;
     s->fa.S = s->fspec;
     int e;
     if ((e = fourier_set_lds_limit(s->fa))) return e;
@@ -589,10 +589,12 @@ static int read_test(stz_sim *s, double *acc) {
 // whose first test comes before any counted cycle and that adds one cycle
 // per failed test; there is no extra cycle, since what it adds to an iterate
 // stopped at its threshold the direct solve's rounding floor already has.
+// `from`: what the source is formed from, or null (src holds it).
 // `ahead` is enqueued after the first test, before the host waits for it: the
 // caller's next launch, which tests the same norm on the device (s->gate) and
 // does nothing where the test fails; *ran says whether it took effect.
-template <typename F> static int fourier_solve(stz_sim *s, F ahead, bool *ran) {
+template <typename F>
+static int fourier_solve(stz_sim *s, const SourceArgs *from, F ahead, bool *ran) {
     int e;
     const stz_mg_config &g = s->cfg;
     const double tol = s->acc_base * g.tol_mult;
@@ -603,7 +605,7 @@ template <typename F> static int fourier_solve(stz_sim *s, F ahead, bool *ran) {
     double acc;
     int n = 0;
     double *scratch = s->mg64.args.lv[0].z2;
-    if ((e = mg_fourier_solve(s->fa, s->src, s->vel, false, s->stream))) return e;
+    if ((e = mg_fourier_solve(s->fa, from, s->src, s->vel, false, s->stream))) return e;
     if ((e = mg_resid_test(s->top64(), nullptr, s->partial, s->dnorm, s->gate, s->stream))) return e;
     STZ_HIP(hipEventRecord(s->norm_ev, s->stream));
     if ((e = ahead())) return e;
@@ -624,7 +626,7 @@ template <typename F> static int fourier_solve(stz_sim *s, F ahead, bool *ran) {
             }
             n++;
             if ((e = mg_resid_test(s->top64(), scratch, s->partial, s->dnorm, s->gate, s->stream))) return e;
-            if ((e = mg_fourier_solve(s->fa, scratch, s->vel, true, s->stream))) return e;
+            if ((e = mg_fourier_solve(s->fa, nullptr, scratch, s->vel, true, s->stream))) return e;
             if ((e = mg_resid_test(s->top64(), nullptr, s->partial, s->dnorm, s->gate, s->stream))) return e;
             STZ_HIP(hipEventRecord(s->norm_ev, s->stream));
             s->last.total_cycles++;
@@ -650,7 +652,7 @@ static int mg_solve_impl(stz_sim *s) {
     int e;
     if (fourier_active(s)) {
         bool ran;
-        return fourier_solve(s, [] { return (int)STZ_OK; }, &ran);
+        return fourier_solve(s, nullptr, [] { return (int)STZ_OK; }, &ran);
     }
     const stz_mg_config &g = s->cfg;
     const double tol = s->acc_base * g.tol_mult;
@@ -749,18 +751,21 @@ static int projection_impl(stz_sim *s, double dt) {
     if ((e = mg_build(s, s->p.viscosity / dt))) return e;
     const double cxx = s->hl[0].S[40 + 16];  // interior centre block, x row
     const double xbc = s->c.bcs * cxx;
-    if ((e = launch_source(s->c, s->cur, dt, xbc, bdry_vel(s), s->src, s->stream))) return e;
     if (fourier_active(s)) {
         bool ran;
+        // the source is formed by the solve's first launch
+        SourceArgs from{{s->cur.p, s->cur.q, s->cur.s, s->cur.tau},
+                        0.5 / dt * s->c.xsp, 0.5 / dt * s->c.ysp, xbc * bdry_vel(s)};
         const double denom = (double)s->c.m * (s->c.n + 1), tol = s->acc_base * s->cfg.tol_mult;
-        if ((e = fourier_solve(s, [&] {
+        if ((e = fourier_solve(s, &from, [&] {
                 return launch_correct(s->c, s->cur, s->vel, dt, bdry_vel(s), bdry_pos(s), s->stream, s->gate, denom,
                                       tol);
             }, &ran)))
             return e;
         if (ran) return STZ_OK;
-    } else if ((e = mg_solve_impl(s))) {
-        return e;
+    } else {
+        if ((e = launch_source(s->c, s->cur, dt, xbc, bdry_vel(s), s->src, s->stream))) return e;
+        if ((e = mg_solve_impl(s))) return e;
     }
     return launch_correct(s->c, s->cur, s->vel, dt, bdry_vel(s), bdry_pos(s), s->stream);
 }
