@@ -150,7 +150,7 @@ int batch_refine(const RefineEntry *E, const int *map, int ne, int total, int sp
                  hipStream_t st);
 template <typename T> int batch_coarse(const CoarseEntry<T> *E, int ne, size_t lds, const EnsState *S, hipStream_t st);
 // direct-level solves: a mode launch (direct_mode_workgroups(M, Nn)
-// workgroups per entry) and an inverse launch (direct_inverse_workgroups)
+// workgroups per entry, one per mode) and an inverse launch (direct_inverse_workgroups)
 template <typename T>
 int batch_direct(const DirectEntry<T> *E, const int *mode_map, int mode_total, const int *inv_map, int inv_total,
                  int ne, size_t lds, const EnsState *S, hipStream_t st);

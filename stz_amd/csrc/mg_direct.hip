@@ -7,7 +7,10 @@
 // A discrete Fourier transform along x turns such a level of M x Nn nodes
 // into M/2 + 1 independent complex systems of N2 = 2 Nn unknowns (mode k:
 // the row stencils' blocks summed as sum_dx S_j[dx,dy] e^{i theta_k dx},
-// theta_k = 2 pi k / M; the other modes are their conjugates).  The host
+// theta_k = 2 pi k / M; the other modes are their conjugates).  The operator is
+// symmetric under reflection in x with v -> -v (qs_multi's stencil is, and
+// bilinear coarsening keeps it), so its u-u and v-v blocks are even in dx and
+// its u-v blocks odd: with v = i v' every mode's system is real.  The host
 // inverts each once per operator (Gauss-Jordan with partial pivoting) and
 // folds the inverse transform's weights into the inverses; the device then
 // solves the level in two launches:
@@ -17,11 +20,11 @@
 //   inverse launch  one workgroup per row (j, component): the real inverse
 //                   DFT of the solved modes
 // Every sum runs in a fixed order, so the result is deterministic.  Per
-// solve: M N2 (M/2 + 1) complex multiply-adds for the transforms and
-// (M/2 + 1) N2^2 for the modes, instead of a V-cycle's chain of
+// solve: M N2 (M/2 + 1) complex multiply-adds for the transforms and twice
+// (M/2 + 1) N2^2 real ones for the modes, instead of a V-cycle's chain of
 // barrier-separated smoothing passes on ever smaller levels.
 //
-// Both launches are latency bound (a 64 x 65 level: 66 KB of source, 9 MB of
+// Both launches are latency bound (a 64 x 65 level: 66 KB of source, 4.5 MB of
 // mode inverses in FP64 over 132 workgroups), so each is laid out for as few
 // dependent memory round trips as possible: the mode launch issues its rows
 // of the inverse before it stages the source, stages the source with all of
@@ -30,13 +33,12 @@
 // table of the M roots of unity indexed by k i mod M.
 //
 // Device buffer of a direct level (direct_elems values of T):
-//   Gh  [k][r][q]  complex inverse of mode k, weighted for the inverse DFT
+//   Gh  [k][r][q]  inverse of mode k (real), weighted for the inverse DFT
 //   tw  [m]        (cos, sin) of 2 pi m / M, m < M
 //   Xh  [r][k]     the solved modes (written by the mode launch)
 #include <hip/hip_runtime.h>
 
 #include <cmath>
-#include <complex>
 #include <vector>
 
 #include "batch.h"
@@ -60,7 +62,7 @@ template <> struct Pair<float> { typedef float2 type; };
 constexpr int kMaxN2 = kRowBlocks * kModeWaves * kMaxRows < 64 * kMaxQ ? kRowBlocks * kModeWaves * kMaxRows
                                                                         : 64 * kMaxQ;
 
-__host__ __device__ static size_t gh_elems(int M, int Nn) { return (size_t)2 * (M / 2 + 1) * (2 * Nn) * (2 * Nn); }
+__host__ __device__ static size_t gh_elems(int M, int Nn) { return (size_t)(M / 2 + 1) * (2 * Nn) * (2 * Nn); }
 __host__ __device__ static size_t tw_elems(int M) { return (size_t)2 * M; }
 __host__ __device__ static size_t xh_elems(int M, int Nn) { return (size_t)2 * (M / 2 + 1) * (2 * Nn); }
 size_t direct_elems(int M, int Nn) { return gh_elems(M, Nn) + tw_elems(M) + xh_elems(M, Nn); }
@@ -74,16 +76,19 @@ bool direct_fits(int M, int Nn) {
            direct_lds_bytes(M, Nn) <= 150 * 1024;
 }
 
-// mode launch body: workgroup blk = k * kRowBlocks + row block; the
-// level's source is in T, everything else in FP64
+// mode launch body: row blocks rb0 .. rb1 - 1 of mode k; the level's source
+// is in T, everything else in FP64.  A row's result does not depend on which
+// blocks share a workgroup: one solve spreads a mode over kRowBlocks
+// workgroups, a batch, whose members fill the chip, gives each mode one and
+// stages and transforms the source once (20 members of sides 64 and 128: 39
+// -> 32 us a launch).
 template <typename T>
 __device__ __forceinline__ static void direct_mode_body(int M, int Nn, double *__restrict__ D,
-                                                        const T *__restrict__ b, int blk) {
+                                                        const T *__restrict__ b, int k, int rb0, int rb1) {
     extern __shared__ __align__(16) unsigned char smem_raw[];
     const int N2 = 2 * Nn, K = M / 2 + 1, P = N2 + 1, nodes = M * Nn;
-    const int k = blk / kRowBlocks, rb = blk % kRowBlocks;
     const int wave = threadIdx.x / 64, lane = threadIdx.x % 64;
-    const double *Gh = D + (size_t)2 * k * N2 * N2;
+    const double *Gh = D + (size_t)k * N2 * N2;
     const double *tw = D + gh_elems(M, Nn);
     double *Xh = D + gh_elems(M, Nn) + tw_elems(M);
     double *bt = reinterpret_cast<double *>(smem_raw);  // bt[i P + q] = b(i, q), q = 2 j' + c'
@@ -92,20 +97,23 @@ __device__ __forceinline__ static void direct_mode_body(int M, int Nn, double *_
 
     typedef typename Pair<T>::type V2;
     // this wave's rows of the mode's inverse: r = r0 + wave + 4 s
-    const int rows = (N2 + kRowBlocks - 1) / kRowBlocks, r0 = rb * rows, r1 = min(r0 + rows, N2);
-    double g[kMaxRows][kMaxQ][2];
+    const int rows = (N2 + kRowBlocks - 1) / kRowBlocks;
+    double g[kMaxRows][kMaxQ];
+    auto load_rows = [&](int rb) {
+        const int r0 = rb * rows, r1 = min(r0 + rows, N2);
 #pragma unroll
-    for (int s = 0; s < kMaxRows; s++) {
-        const int r = r0 + wave + kModeWaves * s;
+        for (int s = 0; s < kMaxRows; s++) {
+            const int r = r0 + wave + kModeWaves * s;
 #pragma unroll
-        for (int u = 0; u < kMaxQ; u++) {
-            const int q = lane + 64 * u;
-            const bool ok = r < r1 && q < N2;
-            const double2 gv = reinterpret_cast<const double2 *>(Gh)[(size_t)(ok ? r : 0) * N2 + (ok ? q : 0)];
-            g[s][u][0] = ok ? gv.x : 0.0;
-            g[s][u][1] = ok ? gv.y : 0.0;
+            for (int u = 0; u < kMaxQ; u++) {
+                const int q = lane + 64 * u;
+                const bool ok = r < r1 && q < N2;
+                const double gv = Gh[(size_t)(ok ? r : 0) * N2 + (ok ? q : 0)];
+                g[s][u] = ok ? gv : 0.0;
+            }
         }
-    }
+    };
+    load_rows(rb0);
     // stage the source (vec2 nodes) transposed, and the twiddle table
     const V2 *bv = reinterpret_cast<const V2 *>(b);
     for (int base = 0; base < nodes; base += kStage * kModeThreads) {
@@ -141,8 +149,9 @@ __device__ __forceinline__ static void direct_mode_body(int M, int Nn, double *_
             m += k;
             if (m >= M) m -= M;
         }
-        bh[2 * q] = re;
-        bh[2 * q + 1] = im;
+        // the transverse component as -i times its transform
+        bh[2 * q] = (q & 1) ? im : re;
+        bh[2 * q + 1] = (q & 1) ? -re : im;
     }
     __syncthreads();
     // rows of the mode's (weighted) inverse applied to bhat: each lane sums
@@ -154,24 +163,28 @@ __device__ __forceinline__ static void direct_mode_body(int M, int Nn, double *_
         br[u] = q < N2 ? bh[2 * q] : 0.0;
         bi[u] = q < N2 ? bh[2 * q + 1] : 0.0;
     }
+    for (int rb = rb0; rb < rb1; rb++) {
+        const int r0 = rb * rows, r1 = min(r0 + rows, N2);
 #pragma unroll
-    for (int s = 0; s < kMaxRows; s++) {
-        const int r = r0 + wave + kModeWaves * s;
-        if (r0 + wave + kModeWaves * s >= r1) break;  // uniform over the wave
-        double re = 0, im = 0;
+        for (int s = 0; s < kMaxRows; s++) {
+            const int r = r0 + wave + kModeWaves * s;
+            if (r >= r1) break;  // uniform over the wave
+            double re = 0, im = 0;
 #pragma unroll
-        for (int u = 0; u < kMaxQ; u++) {
-            re = fmav(g[s][u][0], br[u], re);
-            re = fmav(-g[s][u][1], bi[u], re);
-            im = fmav(g[s][u][0], bi[u], im);
-            im = fmav(g[s][u][1], br[u], im);
+            for (int u = 0; u < kMaxQ; u++) {
+                re = fmav(g[s][u], br[u], re);
+                im = fmav(g[s][u], bi[u], im);
+            }
+#pragma unroll
+            for (int off = 32; off > 0; off >>= 1) {
+                re += __shfl_xor(re, off);
+                im += __shfl_xor(im, off);
+            }
+            if (lane == 0)  // and the transverse result times i
+                reinterpret_cast<double2 *>(Xh)[(size_t)r * K + k] =
+                    (r & 1) ? make_double2(-im, re) : make_double2(re, im);
         }
-#pragma unroll
-        for (int off = 32; off > 0; off >>= 1) {
-            re += __shfl_xor(re, off);
-            im += __shfl_xor(im, off);
-        }
-        if (lane == 0) reinterpret_cast<double2 *>(Xh)[(size_t)r * K + k] = make_double2(re, im);
+        if (rb + 1 < rb1) load_rows(rb + 1);
     }
 }
 
@@ -205,7 +218,8 @@ __device__ __forceinline__ static void direct_inverse_body(int M, int Nn, const 
 }
 template <typename T>
 __global__ void __launch_bounds__(kModeThreads) direct_mode_kernel(int M, int Nn, double *D, const T *b) {
-    direct_mode_body(M, Nn, D, b, blockIdx.x);
+    const int k = blockIdx.x / kRowBlocks, rb = blockIdx.x % kRowBlocks;
+    direct_mode_body(M, Nn, D, b, k, rb, rb + 1);
 }
 template <typename T>
 __global__ void __launch_bounds__(kInvThreads) direct_inverse_kernel(int M, int Nn, const double *D, T *z) {
@@ -220,7 +234,7 @@ __global__ void __launch_bounds__(kModeThreads) direct_mode_batch_kernel(const D
     const int2 el = batch_slot(map, blockIdx.x);
     const DirectEntry<T> &x = E[el.x];
     if (St && !St[x.member].active) return;
-    direct_mode_body(x.M, x.Nn, x.D, x.b, el.y);
+    direct_mode_body(x.M, x.Nn, x.D, x.b, el.y, 0, kRowBlocks);
 }
 template <typename T>
 __global__ void __launch_bounds__(kInvThreads) direct_inverse_batch_kernel(const DirectEntry<T> *E, const int *map,
@@ -233,7 +247,7 @@ __global__ void __launch_bounds__(kInvThreads) direct_inverse_batch_kernel(const
 
 int direct_mode_workgroups(int M, int Nn) {
     (void)Nn;
-    return (M / 2 + 1) * kRowBlocks;
+    return M / 2 + 1;
 }
 int direct_inverse_workgroups(int M, int Nn) {
     (void)M;
@@ -242,7 +256,7 @@ int direct_inverse_workgroups(int M, int Nn) {
 
 template <typename T> int mg_direct_solve(const LevelArgs<T> &L, double *D, hipStream_t st) {
     const int M = L.m, Nn = L.n;
-    hipLaunchKernelGGL(direct_mode_kernel<T>, dim3(direct_mode_workgroups(M, Nn)), dim3(kModeThreads),
+    hipLaunchKernelGGL(direct_mode_kernel<T>, dim3((M / 2 + 1) * kRowBlocks), dim3(kModeThreads),
                        direct_lds_bytes(M, Nn), st, M, Nn, D, L.b);
     hipLaunchKernelGGL(direct_inverse_kernel<T>, dim3(direct_inverse_workgroups(M, Nn)), dim3(kInvThreads), 0, st,
                        M, Nn, D, L.z);
@@ -276,51 +290,61 @@ int batch_direct(const DirectEntry<T> *E, const int *mode_map, int mode_total, c
 // host: the device buffer of an x-invariant level with row stencils S (40
 // per row: blocks dl,dc,dr,cl,cc,cr,ul,uc,ur, then the centre inverse), M
 // nodes per row (even), Nn rows, in the layout above (Xh zero).  Returns
-// false if a mode's system is singular.
+// false if a mode's system is singular or the level lacks the symmetry above.
 bool direct_inverse(const double *S, int M, int Nn, std::vector<double> &D) {
-    typedef std::complex<double> cd;
     const int N2 = 2 * Nn, K = M / 2 + 1;
     D.assign(direct_elems(M, Nn), 0.0);
-    std::vector<cd> A((size_t)N2 * N2), I((size_t)N2 * N2);
+    std::vector<double> A((size_t)N2 * N2), I((size_t)N2 * N2);
     const double pi = 3.14159265358979323846;
+    // the reflection symmetry the real form rests on, to rounding
+    for (int j = 0; j < Nn; j++)
+        for (int jj = 0; jj < 3; jj++)
+            for (int r = 0; r < 4; r++) {
+                const double *s = S + (size_t)j * 40 + 12 * jj;
+                const double l = s[r], m = s[4 + r], u = s[8 + r], top = std::fabs(S[(size_t)j * 40 + 16]);
+                const bool even = r == 0 || r == 3;
+                if (std::fabs(even ? l - u : l + u) > 1e-9 * top || (!even && std::fabs(m) > 1e-9 * top)) return false;
+            }
     for (int k = 0; k < K; k++) {
-        const double th = 2 * pi * k / M;
-        const cd e[3] = {std::polar(1.0, -th), cd(1, 0), std::polar(1.0, th)};
-        std::fill(A.begin(), A.end(), cd(0, 0));
-        std::fill(I.begin(), I.end(), cd(0, 0));
+        const double th = 2 * pi * k / M, co = std::cos(th), si = std::sin(th);
+        std::fill(A.begin(), A.end(), 0.0);
+        std::fill(I.begin(), I.end(), 0.0);
         for (int r = 0; r < N2; r++) I[(size_t)r * N2 + r] = 1;
         for (int j = 0; j < Nn; j++) {
             const double *s = S + (size_t)j * 40;
-            for (int kb = 0; kb < 9; kb++) {
-                const int dx = kb % 3 - 1, jj = j + kb / 3 - 1;
+            for (int dj = -1; dj <= 1; dj++) {
+                const int jj = j + dj;
                 if (jj < 0 || jj >= Nn) continue;
-                const cd w = e[dx + 1];
-                A[(size_t)(2 * j) * N2 + 2 * jj] += s[4 * kb] * w;
-                A[(size_t)(2 * j) * N2 + 2 * jj + 1] += s[4 * kb + 1] * w;
-                A[(size_t)(2 * j + 1) * N2 + 2 * jj] += s[4 * kb + 2] * w;
-                A[(size_t)(2 * j + 1) * N2 + 2 * jj + 1] += s[4 * kb + 3] * w;
+                const double *l = s + 12 * (dj + 1), *m = l + 4, *u = l + 8;
+                // sum_dx s e^{i theta dx}: the even blocks' cosine part, the
+                // odd ones' sine part times i, which v = i v' turns real
+                double *a0 = &A[(size_t)(2 * j) * N2 + 2 * jj], *a1 = a0 + N2;
+                a0[0] += m[0] + co * (l[0] + u[0]);
+                a0[1] -= si * (u[1] - l[1]);
+                a1[0] += si * (u[2] - l[2]);
+                a1[1] += m[3] + co * (l[3] + u[3]);
             }
         }
         // Gauss-Jordan with partial pivoting
         for (int col = 0; col < N2; col++) {
             int piv = col;
             for (int r = col + 1; r < N2; r++)
-                if (std::abs(A[(size_t)r * N2 + col]) > std::abs(A[(size_t)piv * N2 + col])) piv = r;
-            if (std::abs(A[(size_t)piv * N2 + col]) == 0) return false;
+                if (std::fabs(A[(size_t)r * N2 + col]) > std::fabs(A[(size_t)piv * N2 + col])) piv = r;
+            if (A[(size_t)piv * N2 + col] == 0) return false;
             if (piv != col)
                 for (int c = 0; c < N2; c++) {
                     std::swap(A[(size_t)piv * N2 + c], A[(size_t)col * N2 + c]);
                     std::swap(I[(size_t)piv * N2 + c], I[(size_t)col * N2 + c]);
                 }
-            const cd d = 1.0 / A[(size_t)col * N2 + col];
+            const double d = 1.0 / A[(size_t)col * N2 + col];
             for (int c = 0; c < N2; c++) {
                 A[(size_t)col * N2 + c] *= d;
                 I[(size_t)col * N2 + c] *= d;
             }
             for (int r = 0; r < N2; r++) {
                 if (r == col) continue;
-                const cd f = A[(size_t)r * N2 + col];
-                if (f == cd(0, 0)) continue;
+                const double f = A[(size_t)r * N2 + col];
+                if (f == 0) continue;
                 for (int c = 0; c < N2; c++) {
                     A[(size_t)r * N2 + c] -= f * A[(size_t)col * N2 + c];
                     I[(size_t)r * N2 + c] -= f * I[(size_t)col * N2 + c];
@@ -329,11 +353,8 @@ bool direct_inverse(const double *S, int M, int Nn, std::vector<double> &D) {
         }
         // z = (1/M) [X_0 + X_{M/2} (-1)^i] + (2/M) sum_{0<k<M/2} Re(X_k e^{i theta_k i})
         const double w = (k == 0 || 2 * k == M) ? 1.0 / M : 2.0 / M;
-        double *g = D.data() + (size_t)2 * k * N2 * N2;
-        for (size_t t = 0; t < (size_t)N2 * N2; t++) {
-            g[2 * t] = w * I[t].real();
-            g[2 * t + 1] = w * I[t].imag();
-        }
+        double *g = D.data() + (size_t)k * N2 * N2;
+        for (size_t t = 0; t < (size_t)N2 * N2; t++) g[t] = w * I[t];
     }
     double *tw = D.data() + gh_elems(M, Nn);
     for (int i = 0; i < M; i++) {
