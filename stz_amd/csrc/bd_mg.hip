@@ -691,6 +691,237 @@ __device__ __forceinline__ static void gs_tile_body(Rows rows, const T *__restri
     }
 }
 
+// ---------------------------------------------------------------------------
+// Coarse levels that are a chain of latencies.  Each colour pass of
+// gs_tile_kernel loads its rows' stencils from memory, five to six round
+// trips a launch, and gs_bottom_kernel's passes leave three lanes in four
+// idle.  The kernels below give a thread CPT colours of one 2x2 block of
+// nodes and load everything it needs at once: stencils, right-hand sides and
+// start values stay in its registers for the whole launch.  FP32: all four
+// colours (160 registers of stencils), FP64: two (groups of whole waves take
+// colours 0, 1 and 2, 3).
+// ---------------------------------------------------------------------------
+template <typename T> struct alignas(2 * sizeof(T)) P2 { T x, y; };
+
+template <typename T> struct BlockShape { static constexpr int CPT = sizeof(T) == 4 ? 4 : 2, groups = 4 / CPT; };
+
+// off-diagonal part at the node of colour C (x parity C & 1, y parity C >> 1)
+// of block blk, from z in colour-split LDS: colour c of a block at c NB + blk,
+// blocks in rows of BX; nodes off the level hold zero.  The order of the sum
+// is lvl_offdiag_at's.
+template <typename T, int C>
+__device__ __forceinline__ V2T<T> block_offdiag(const T (&s)[40], const P2<T> *zs, int NB, int BX, int blk) {
+    T rx = 0, ry = 0;
+    P2<T> z[9];
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        const int x = (C & 1) + k % 3 - 1, y = (C >> 1) + k / 3 - 1;  // -1 .. 2
+        const int c = (x & 1) + 2 * (y & 1);
+        z[k] = zs[c * NB + blk + ((x + 2) / 2 - 1) + BX * ((y + 2) / 2 - 1)];
+    }
+#pragma unroll
+    for (int k = 0; k < 9; k++) {
+        if (k == 4) continue;
+        rx += s[4 * k] * z[k].x + s[4 * k + 1] * z[k].y;
+        ry += s[4 * k + 2] * z[k].x + s[4 * k + 3] * z[k].y;
+    }
+    return V2T<T>{rx, ry};
+}
+// the node of colour c: its value by one Gauss-Seidel update
+template <typename T>
+__device__ __forceinline__ P2<T> block_update(const T (&s)[40], const P2<T> &b, const V2T<T> &o) {
+    const T rx = b.x - o.x, ry = b.y - o.y;
+    return P2<T>{s[36] * rx + s[37] * ry, s[38] * rx + s[39] * ry};
+}
+template <typename T>
+__device__ __forceinline__ V2T<T> block_offdiag_of(int c, const T (&s)[40], const P2<T> *zs, int NB, int BX, int blk) {
+    // c is known at compile time wherever this is unrolled, or uniform
+    return c == 0 ? block_offdiag<T, 0>(s, zs, NB, BX, blk)
+                  : (c == 1 ? block_offdiag<T, 1>(s, zs, NB, BX, blk)
+                            : (c == 2 ? block_offdiag<T, 2>(s, zs, NB, BX, blk)
+                                      : block_offdiag<T, 3>(s, zs, NB, BX, blk)));
+}
+
+// the tile of a small level: 16 x 16 nodes with gs_tile_body's halo
+template <typename T, int MODE> struct BlockTile {
+    static constexpr int X = 16, H = MODE == 3 ? 6 : 4, RX = X + 2 * H, BX = RX / 2, NB = BX * BX;
+    static constexpr int GT = (NB + 63) / 64 * 64;  // threads of a colour group
+    static constexpr int NT = GT * BlockShape<T>::groups;
+};
+
+// One smoothing sweep of a coarse level, as gs_tile_kernel's modes 1 to 3
+template <typename T, int MODE>
+__global__ void __launch_bounds__((BlockTile<T, MODE>::NT)) block_tile_kernel(BdLevelT<T> L, const T *__restrict__ zin,
+                                                                            T *__restrict__ zout,
+                                                                            const T *__restrict__ zc,
+                                                                            T *__restrict__ cb, int cm, int cn) {
+    using D = BlockTile<T, MODE>;
+    constexpr int CPT = BlockShape<T>::CPT, NB = D::NB, BX = D::BX, H = D::H;
+    // one ring of blocks more than the region, so that no read is out of range
+    constexpr int LB = BX + 2, LN = LB * LB;
+    __shared__ P2<T> zs[4 * LN];
+    const int tid = threadIdx.x, group = tid / D::GT, blk = tid % D::GT;
+    const bool own = blk < NB;
+    const int bx = own ? blk % BX : 0, by = own ? blk / BX : 0, at = (bx + 1) + LB * (by + 1);
+    const int x0 = blockIdx.x * D::X, y0 = blockIdx.y * D::X, m = L.m, n = L.n;
+    T st[CPT][40];
+    P2<T> b[CPT], zo[CPT];
+    bool in[CPT];
+    for (int q = tid; q < 4 * LN; q += D::NT) zs[q] = P2<T>{0, 0};
+#pragma unroll
+    for (int q = 0; q < CPT; q++) {
+        const int c = group * CPT + q;
+        const int i = x0 - H + 2 * bx + (c & 1), j = y0 - H + 2 * by + (c >> 1);
+        in[q] = own && i >= 0 && i < m && j >= 0 && j < n;
+        const int ij = in[q] ? i + m * j : 0;
+        lvl_row(L, ij, st[q]);
+        b[q] = reinterpret_cast<const P2<T> *>(L.b)[ij];
+        zo[q] = P2<T>{0, 0};
+        if (MODE == 2 && in[q]) {
+            zo[q] = reinterpret_cast<const P2<T> *>(zin)[ij];
+            int px[2], py[2];  // as prolong_kernel
+            double wx[2], wy[2];
+            const int nx = parents(i, m, cm, px, wx), ny = parents(j, n, cn, py, wy);
+            T sx = 0, sy = 0;
+#pragma unroll
+            for (int bb = 0; bb < 2; bb++)
+#pragma unroll
+                for (int aa = 0; aa < 2; aa++) {
+                    if (bb >= ny || aa >= nx) continue;
+                    const T w = (T)(wx[aa] * wy[bb]);
+                    const P2<T> v = reinterpret_cast<const P2<T> *>(zc)[px[aa] + (size_t)cm * py[bb]];
+                    sx += w * v.x;
+                    sy += w * v.y;
+                }
+            zo[q].x += sx;
+            zo[q].y += sy;
+        }
+    }
+    __syncthreads();
+    if (MODE == 2) {
+#pragma unroll
+        for (int q = 0; q < CPT; q++)
+            if (in[q]) zs[(group * CPT + q) * LN + at] = zo[q];
+        __syncthreads();
+    }
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        constexpr int G = BlockShape<T>::groups;
+        const int q = G == 1 ? c : c % CPT;
+        if (G == 1 || group == c / CPT)
+            if (in[q]) {
+                zo[q] = block_update(st[q], b[q], block_offdiag_of(c, st[q], zs, LN, LB, at));
+                zs[c * LN + at] = zo[q];
+            }
+        __syncthreads();
+    }
+#pragma unroll
+    for (int q = 0; q < CPT; q++) {
+        const int c = group * CPT + q, li = 2 * bx + (c & 1), lj = 2 * by + (c >> 1);
+        if (!in[q] || li < H || li >= H + D::X || lj < H || lj >= H + D::X) continue;
+        reinterpret_cast<P2<T> *>(zout)[(x0 - H + li) + (size_t)m * (y0 - H + lj)] = zo[q];
+    }
+    if (MODE != 3) return;
+    // residuals of the tile and one node around it, in z's place
+    P2<T> r[CPT];
+#pragma unroll
+    for (int c = 0; c < 4; c++) {
+        constexpr int G = BlockShape<T>::groups;
+        const int q = G == 1 ? c : c % CPT;
+        if (G == 1 || group == c / CPT) {
+            r[q] = P2<T>{0, 0};
+            if (in[q]) {
+                const V2T<T> o = block_offdiag_of(c, st[q], zs, LN, LB, at);
+                r[q].x = b[q].x - o.x - (st[q][16] * zo[q].x + st[q][17] * zo[q].y);
+                r[q].y = b[q].y - o.y - (st[q][18] * zo[q].x + st[q][19] * zo[q].y);
+            }
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < CPT; q++)
+        if (own) zs[(group * CPT + q) * LN + at] = r[q];
+    __syncthreads();
+    // the coarse nodes under the tile, as gs_tile_body: b_c = P^T r
+    const int I0 = x0 / 2, I1 = blockIdx.x == gridDim.x - 1 ? cm : min(cm, I0 + D::X / 2);
+    const int J0 = y0 / 2, J1 = blockIdx.y == gridDim.y - 1 ? cn : min(cn, J0 + D::X / 2);
+    const int nI = I1 - I0;
+    for (int t = tid; t < nI * (J1 - J0); t += D::NT) {
+        const int I = I0 + t % nI, J = J0 + t / nI;
+        T sx = 0, sy = 0;
+        int c[2];
+        double w[2];
+        for (int fy = 2 * J - 1; fy <= 2 * J + 1; fy++) {
+            const double wy = weight_of(parents(fy, n, cn, c, w), c, w, J);
+            if (wy == 0) continue;
+            for (int fx = 2 * I - 1; fx <= 2 * I + 1; fx++) {
+                const double wx = weight_of(parents(fx, m, cm, c, w), c, w, I);
+                if (wx == 0) continue;
+                const int li = fx - x0 + H, lj = fy - y0 + H;
+                const P2<T> v = zs[((li & 1) + 2 * (lj & 1)) * LN + ((li >> 1) + 1) + LB * ((lj >> 1) + 1)];
+                sx += (T)(wx * wy) * v.x;
+                sy += (T)(wx * wy) * v.y;
+            }
+        }
+        cb[2 * (I + (size_t)cm * J)] = sx;
+        cb[2 * (I + (size_t)cm * J) + 1] = sy;
+    }
+}
+
+// The bottom level in one workgroup, a thread per block (and colour group):
+// 17^2 nodes are two waves (four in FP64) that all work in every pass, 21 us
+// for the 80 passes (gs_bottom_kernel: 42)
+constexpr int kBottomBlocks = 256;
+template <typename T>
+__global__ void __launch_bounds__((kBottomBlocks * BlockShape<T>::groups)) bottom_block_kernel(BdLevelT<T> L, int sweeps,
+                                                                                           int zero, int gt) {
+    extern __shared__ __align__(16) unsigned char bd_smem[];
+    P2<T> *zs = reinterpret_cast<P2<T> *>(bd_smem);
+    constexpr int CPT = BlockShape<T>::CPT, G = BlockShape<T>::groups;
+    const int m = L.m, n = L.n, bm = (m + 1) >> 1, bn = (n + 1) >> 1, LB = bm + 2, LN = LB * (bn + 2);
+    const int tid = threadIdx.x, group = tid / gt, blk = tid % gt;
+    const bool own = blk < bm * bn;
+    const int bx = own ? blk % bm : 0, by = own ? blk / bm : 0, at = (bx + 1) + LB * (by + 1);
+    T st[CPT][40];
+    P2<T> b[CPT], zo[CPT];
+    bool in[CPT];
+    for (int q = tid; q < 4 * LN; q += blockDim.x) zs[q] = P2<T>{0, 0};
+#pragma unroll
+    for (int q = 0; q < CPT; q++) {
+        const int c = group * CPT + q, i = 2 * bx + (c & 1), j = 2 * by + (c >> 1);
+        in[q] = own && i < m && j < n;
+        const int ij = in[q] ? i + m * j : 0;
+        lvl_row(L, ij, st[q]);
+        b[q] = reinterpret_cast<const P2<T> *>(L.b)[ij];
+        zo[q] = P2<T>{0, 0};
+        if (!zero && in[q]) zo[q] = reinterpret_cast<const P2<T> *>(L.z)[ij];
+    }
+    __syncthreads();
+    if (!zero) {
+#pragma unroll
+        for (int q = 0; q < CPT; q++)
+            if (in[q]) zs[(group * CPT + q) * LN + at] = zo[q];
+        __syncthreads();
+    }
+    for (int sw = 0; sw < sweeps; sw++) {
+#pragma unroll
+        for (int c = 0; c < 4; c++) {
+            const int q = G == 1 ? c : c % CPT;
+            if (G == 1 || group == c / CPT)
+                if (in[q]) {
+                    zo[q] = block_update(st[q], b[q], block_offdiag_of(c, st[q], zs, LN, LB, at));
+                    zs[c * LN + at] = zo[q];
+                }
+            __syncthreads();
+        }
+    }
+#pragma unroll
+    for (int q = 0; q < CPT; q++) {
+        const int c = group * CPT + q;
+        if (in[q]) reinterpret_cast<P2<T> *>(L.z)[(2 * bx + (c & 1)) + m * (2 * by + (c >> 1))] = zo[q];
+    }
+}
+
 template <typename T, int MODE, class Rows>
 __global__ void __launch_bounds__(kTileThreads) gs_tile_kernel(Rows rows, const T *__restrict__ z,
                                                                T *__restrict__ zout, const T *__restrict__ zc,
@@ -1269,6 +1500,29 @@ static int start_in_place(T *zout, const T *zin, int m, int n, int mode, const T
     return STZ_OK;
 }
 
+// One sweep of a coarse level (mode as tile_sweep): small levels by the block
+// kernel.  Its 16 x 16 tiles load every stencil of the halo too (2.3 to 3
+// times the level), which costs less than gs_tile_kernel's round trips while
+// the tiles are about a workgroup per CU: levels of 33^2 to 257^2 8.2 us with
+// the restriction and 6.0 without it in FP32 (8.3 and 6.1 in FP64), against
+// 17 and 13; 513^2 20 and 17 against 20 and 15.
+constexpr int kBlockTiles = 320;
+template <typename T>
+static int level_sweep(const BdLevelT<T> &L, const T *zin, T *zout, int mode, const T *zc, int cm, int cn,
+                       hipStream_t s, T *cb = nullptr) {
+    const dim3 g((L.m + 15) / 16, (L.n + 15) / 16);
+    if (mode == 0 || g.x * g.y > kBlockTiles)
+        return tile_sweep(LevelRows<T>{L}, L.m, L.n, zin, zout, mode, zc, cm, cn, s, cb);
+    if (mode == 3)
+        hipLaunchKernelGGL((block_tile_kernel<T, 3>), g, dim3(BlockTile<T, 3>::NT), 0, s, L, zin, zout, zc, cb, cm, cn);
+    else if (mode == 2)
+        hipLaunchKernelGGL((block_tile_kernel<T, 2>), g, dim3(BlockTile<T, 2>::NT), 0, s, L, zin, zout, zc, cb, cm, cn);
+    else
+        hipLaunchKernelGGL((block_tile_kernel<T, 1>), g, dim3(BlockTile<T, 1>::NT), 0, s, L, zin, zout, zc, cb, cm, cn);
+    STZ_HIP(hipGetLastError());
+    return STZ_OK;
+}
+
 // Smoothing of the top level from zin (mode as tile_sweep) into zout
 // (zout != zin): one sweep by the tiled kernel, more by one launch per
 // colour in place
@@ -1299,13 +1553,21 @@ int BdSolver::smooth_level(const BdLevelT<T> &L, bool bottom, int sweeps, int mo
         if (e) return e;
         BdLevelT<T> B = L;
         B.z = zout;
+        const int bm = (L.m + 1) / 2, bn = (L.n + 1) / 2;
+        if (bm * bn <= kBottomBlocks) {
+            const int gt = (bm * bn + 63) / 64 * 64;
+            hipLaunchKernelGGL(bottom_block_kernel<T>, dim3(1), dim3(gt * BlockShape<T>::groups),
+                               4 * (bm + 2) * (bn + 2) * sizeof(P2<T>), s, B, sweeps, mode == 1 ? 1 : 0, gt);
+            STZ_HIP(hipGetLastError());
+            return STZ_OK;
+        }
         const long nodes = (long)L.m * L.n;
         const int nt = nodes <= 1024 ? (int)((nodes + 63) / 64 * 64) : 1024;
         hipLaunchKernelGGL(gs_bottom_kernel<T>, dim3(1), dim3(nt), lds, s, B, sweeps, mode == 1 ? 1 : 0);
         STZ_HIP(hipGetLastError());
         return STZ_OK;
     }
-    if (sweeps == 1) return tile_sweep(LevelRows<T>{L}, L.m, L.n, zin, zout, mode, zc, cm, cn, s);
+    if (sweeps == 1) return level_sweep(L, zin, zout, mode, zc, cm, cn, s);
     const int e = start_in_place(zout, zin, L.m, L.n, mode, zc, cm, cn, s);
     if (e) return e;
     BdLevelT<T> B = L;
@@ -1350,7 +1612,7 @@ int BdSolver::vcycle_t(const TB *rhs, T *z, BdLevelT<T> *Lv, T *r0, T *zpre, hip
     for (int l = 0; l + 1 < nl; l++) {
         BdLevelT<T> &L = Lv[l], &C = Lv[l + 1];
         if (fused) {
-            if ((e = tile_sweep(LevelRows<T>{L}, L.m, L.n, none, L.z, 3, none, C.m, C.n, s, C.b))) return e;
+            if ((e = level_sweep(L, none, L.z, 3, none, C.m, C.n, s, C.b))) return e;
             continue;
         }
         if ((e = smooth_level(L, false, nu1, 1, none, L.z, none, 0, 0, s))) return e;

@@ -1,0 +1,32 @@
+"""The free-boundary V-cycle's small-level kernels (one thread per 2x2 block,
+bd_mg.hip) at level sizes on both sides of their tiles of 16 and with odd and
+even sides: the preconditioner differs from the one of two sweeps a smoothing
+(a launch per colour) only in speed of convergence, so the two projections
+agree to the solve's threshold, 1e-20 mean square."""
+import numpy as np
+import pytest
+
+from stz_amd import bd_bench
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("form", ["fp64", "mixed"])
+@pytest.mark.parametrize("N", [63, 64, 95, 126, 130, 161])
+def test_projection_over_level_sizes(N, form):
+    print("case bd levels", N, form, flush=True)
+    vel, its = [], []
+    for nu in (1, 2):
+        g = bd_bench.setup(N)
+        g.set_precision(form)
+        g.set_solver(nu, nu)
+        g.projection_step(0.5)
+        info = g.last_solve()
+        assert info["status"] == 0 and info["residual"] <= info["tolerance"], info
+        vel.append(g.get_vel())
+        its.append(info["iterations"])
+        g.close()
+    err = float(np.linalg.norm(vel[0] - vel[1]) / np.linalg.norm(vel[1]))
+    print(N, form, "iterations", its, "difference %.1e" % err)
+    assert its[0] <= 4 * its[1] + 20
+    assert err < 1e-7  # as test_projection_mixed_preconditioner
