@@ -121,8 +121,7 @@ template <typename T> int mg_set_lds_limit(size_t bytes);
 int mg_resid64_to32(const LevelArgs<double> &L, float *b32, float *z32, double *partial, double *out,
                     hipStream_t st);
 int mg_correct64(double *z, const float *e, int count, hipStream_t st);
-// out2: a second place for the sum, or null
-int mg_sum_partials(const double *partial, int np, double *out, hipStream_t st, double *out2 = nullptr);
+int mg_sum_partials(const double *partial, int np, double *out, hipStream_t st);
 template <typename T> int mg_fill_zero(T *p, size_t count, hipStream_t st);
 
 // tiled path (mg_tiled.hip)
@@ -151,8 +150,10 @@ template <typename T> int mg_smooth_level(LevelArgs<T> &L, int sweeps, hipStream
 int mg_refine(const LevelArgs<double> &L, float *b32, double *partial, double *out, hipStream_t st);
 int mg_refine_blocks(const LevelArgs<double> &L);
 // |b - A z|^2 of the FP64 top level summed to *out and *out2; with r, the
-// residual itself is stored there too
-int mg_resid_test(const LevelArgs<double> &L, double *r, double *partial, double *out, double *out2,
+// residual itself is stored there too.  count: kArriveInts ints, zero before
+// and after; a line of its own for each
+constexpr int kArrive = 32, kArriveStride = 32, kArriveInts = (1 + kArrive) * kArriveStride;
+int mg_resid_test(const LevelArgs<double> &L, double *r, double *partial, int *count, double *out, double *out2,
                   hipStream_t st);
 
 }  // namespace stz

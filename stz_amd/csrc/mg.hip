@@ -110,13 +110,9 @@ __device__ __forceinline__ static double sum_partials_body(const double *partial
     return (ws[0] + ws[1]) + (ws[2] + ws[3]);  // valid in thread 0
 }
 
-__global__ void __launch_bounds__(256) sum_partials_kernel(const double *partial, int np, double *out,
-                                                           double *out2) {
+__global__ void __launch_bounds__(256) sum_partials_kernel(const double *partial, int np, double *out) {
     const double v = sum_partials_body(partial, np);
-    if (threadIdx.x == 0) {
-        *out = v;
-        if (out2) *out2 = v;
-    }
+    if (threadIdx.x == 0) *out = v;
 }
 
 // mixed precision: FP64 residual of the top level -> FP32 source of the
@@ -784,7 +780,7 @@ template <typename T> int mg_coarse(const CoarseArgs<T> &A, hipStream_t st) {
 template <typename T> int mg_resid_norm(const LevelArgs<T> &L, double *partial, double *out, hipStream_t st) {
     const int nb = (L.m * L.n + 255) / 256;
     hipLaunchKernelGGL(resid_norm_kernel<T>, dim3(nb), dim3(256), 0, st, L, partial);
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, nb, out, (double *)nullptr);
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, nb, out);
     STZ_HIP(hipGetLastError());
     return STZ_OK;
 }
@@ -793,7 +789,7 @@ int mg_resid64_to32(const LevelArgs<double> &L, float *b32, float *z32, double *
                     hipStream_t st) {
     const int nb = (L.m * L.n + 255) / 256;
     hipLaunchKernelGGL(resid64_to32_kernel, dim3(nb), dim3(256), 0, st, L, b32, z32, partial);
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, nb, out, (double *)nullptr);
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, nb, out);
     STZ_HIP(hipGetLastError());
     return STZ_OK;
 }
@@ -806,8 +802,8 @@ template <typename T> int mg_fill_zero(T *p, size_t count, hipStream_t st) {
 template int mg_fill_zero<double>(double *, size_t, hipStream_t);
 template int mg_fill_zero<float>(float *, size_t, hipStream_t);
 
-int mg_sum_partials(const double *partial, int np, double *out, hipStream_t st, double *out2) {
-    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, np, out, out2);
+int mg_sum_partials(const double *partial, int np, double *out, hipStream_t st) {
+    hipLaunchKernelGGL(sum_partials_kernel, dim3(1), dim3(256), 0, st, partial, np, out);
     STZ_HIP(hipGetLastError());
     return STZ_OK;
 }

@@ -606,7 +606,7 @@ static int fourier_solve(stz_sim *s, const SourceArgs *from, F ahead, bool *ran)
     int n = 0;
     double *scratch = s->mg64.args.lv[0].z2;
     if ((e = mg_fourier_solve(s->fa, from, s->src, s->vel, false, s->stream))) return e;
-    if ((e = mg_resid_test(s->top64(), nullptr, s->partial, s->dnorm, s->gate, s->stream))) return e;
+    if ((e = mg_resid_test(s->top64(), nullptr, s->partial, s->arrived(), s->dnorm, s->gate, s->stream))) return e;
     STZ_HIP(hipEventRecord(s->norm_ev, s->stream));
     if ((e = ahead())) return e;
     s->last.total_cycles = 1;
@@ -625,9 +625,9 @@ static int fourier_solve(stz_sim *s, const SourceArgs *from, F ahead, bool *ran)
                 return STZ_ERR_NOT_CONVERGED;
             }
             n++;
-            if ((e = mg_resid_test(s->top64(), scratch, s->partial, s->dnorm, s->gate, s->stream))) return e;
+            if ((e = mg_resid_test(s->top64(), scratch, s->partial, s->arrived(), s->dnorm, s->gate, s->stream))) return e;
             if ((e = mg_fourier_solve(s->fa, nullptr, scratch, s->vel, true, s->stream))) return e;
-            if ((e = mg_resid_test(s->top64(), nullptr, s->partial, s->dnorm, s->gate, s->stream))) return e;
+            if ((e = mg_resid_test(s->top64(), nullptr, s->partial, s->arrived(), s->dnorm, s->gate, s->stream))) return e;
             STZ_HIP(hipEventRecord(s->norm_ev, s->stream));
             s->last.total_cycles++;
             if ((e = read_test(s, &acc))) return e;
@@ -840,7 +840,8 @@ int stz_sim_create(const stz_sim_params *p, int precision, stz_sim **out) {
     s->src = s->vel + 2 * nodes;
     if (hipMalloc(&s->dec, (size_t)c.m * c.n * sizeof(uint32_t)) != hipSuccess) return fail(STZ_ERR_HIP);
     (void)hipMemset(s->dec, 0, (size_t)c.m * c.n * sizeof(uint32_t));
-    if (hipMalloc(&s->gate, sizeof(double)) != hipSuccess) return fail(STZ_ERR_HIP);
+    if (hipMalloc(&s->gate, 128 + kArriveInts * sizeof(int)) != hipSuccess) return fail(STZ_ERR_HIP);
+    (void)hipMemset(s->gate, 0, 128 + kArriveInts * sizeof(int));
     s->nblocks_norm = (int)std::max<size_t>((nodes + 255) / 256,
                                             (size_t)((c.m + 63) / 64) * ((c.n + 1 + 15) / 16));
     {

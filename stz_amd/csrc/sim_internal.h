@@ -82,7 +82,8 @@ struct stz_sim {
     stz::FourierArgs fa{};
     double *ftab = nullptr, *fspec = nullptr;
     bool direct_pending = false;       // the direct level's inverses are not formed yet
-    double *gate = nullptr;            // device copy of a convergence test's norm
+    double *gate = nullptr;            // device copy of a convergence test's norm; the test's counts 128 bytes on
+    int *arrived() { return reinterpret_cast<int *>(gate + 16); }
     double *partial = nullptr, *dnorm = nullptr, *hnorm = nullptr;
     hipEvent_t norm_ev = nullptr;  // marks the end of a convergence test's norm
     int nblocks_norm = 0;
