@@ -184,44 +184,77 @@ __device__ __forceinline__ static void stages_fixed(cplx *buf, const cplx *__res
     if constexpr (RN > 1) stages_fixed<M, R>(buf, tw, next);
 }
 
-// any length: one stage from `in` to `out`, radix RX (0: the run-time radix
-// r as a plain sum per output with the roots of unity `root`, for the primes
-// without a butterfly above)
+// t / d for 0 <= t < 2^16 with inv = 1.0f / d: (t + 1/2) / d is at least
+// 1 / (2 d) from a whole number, more than the product's rounding
+__device__ __forceinline__ static int small_div(int t, float inv) { return (int)(((float)t + 0.5f) * inv); }
+
+// any length: one stage from `in` to `out`, radix RX
 template <int RX, int R>
-__device__ __forceinline__ static void stage_any(const cplx *in, cplx *out, const cplx *__restrict__ tw,
-                                                 const cplx *__restrict__ root, int M, int L, int r) {
+__device__ __forceinline__ static void stage_any(const cplx *in, cplx *out, const cplx *__restrict__ tw, int M, int L) {
     constexpr int NT = kRowThreads * R;
-    const int P = fpad(M);
-    if constexpr (RX > 0) {
-        const int nb = M / RX;
-        for (int t = threadIdx.x; t < R * nb; t += NT) {
-            const int row = t / nb, idx = t - row * nb, k = idx % L;
-            cplx x[RX];
+    const int P = fpad(M), nb = M / RX;
+    const float inb = 1.0f / nb, il = 1.0f / L;
+    for (int t = threadIdx.x; t < R * nb; t += NT) {
+        const int row = small_div(t, inb), idx = t - row * nb, k = idx - L * small_div(idx, il);
+        cplx x[RX];
 #pragma unroll
-            for (int q = 0; q < RX; q++) x[q] = in[row * P + fpad(idx + q * nb)];
-            if (L > 1)
+        for (int q = 0; q < RX; q++) x[q] = in[row * P + fpad(idx + q * nb)];
+        if (L > 1)
 #pragma unroll
-                for (int q = 1; q < RX; q++) x[q] = cmul(x[q], tw[L - 1 + (q - 1) * L + k]);
-            dft<RX>(x);
-            const int o = (idx - k) * RX + k;
+            for (int q = 1; q < RX; q++) x[q] = cmul(x[q], tw[L - 1 + (q - 1) * L + k]);
+        dft<RX>(x);
+        const int o = (idx - k) * RX + k;
 #pragma unroll
-            for (int q = 0; q < RX; q++) out[row * P + fpad(o + q * L)] = x[q];
+        for (int q = 0; q < RX; q++) out[row * P + fpad(o + q * L)] = x[q];
+    }
+}
+
+// the same for a prime r without a butterfly above.  In place in `in`, the
+// twiddles, and of each pair of inputs p, r - p the sum and the difference;
+// then a thread per pair of outputs q, r - q, which share
+//     x_0 + sum_p (x_p + x_{r-p}) cos(2 pi p q / r)  and
+//     sum_p (x_p - x_{r-p}) sin(2 pi p q / r),
+// a quarter of the multiplications of a sum per output.  rt: the r roots of
+// unity e^{-2 pi i m / r}, in LDS.  608 columns (19 x 32), a source
+// launch of 317 rows: 22.5 us as a plain sum per output with its roots from
+// memory, 14.2 this way.
+template <int R>
+__device__ __forceinline__ static void stage_prime(cplx *in, cplx *out, const cplx *__restrict__ tw, const cplx *rt,
+                                                   int M, int L, int r) {
+    constexpr int NT = kRowThreads * R;
+    const int P = fpad(M), nb = M / r, h = r / 2;
+    const float inb = 1.0f / nb, il = 1.0f / L, ih = 1.0f / h, ih1 = 1.0f / (h + 1);
+    for (int t = threadIdx.x; t < R * nb * h; t += NT) {
+        const int u = small_div(t, inb), idx = t - u * nb, row = small_div(u, ih), p = 1 + u - row * h;
+        const int k = idx - L * small_div(idx, il);
+        cplx *lo = in + row * P + fpad(idx + p * nb), *hi = in + row * P + fpad(idx + (r - p) * nb);
+        cplx x = *lo, y = *hi;
+        if (L > 1) {
+            x = cmul(x, tw[L - 1 + (p - 1) * L + k]);
+            y = cmul(y, tw[L - 1 + (r - p - 1) * L + k]);
         }
-    } else {
-        const int nb = M / r, step = M / (L * r);
-        for (int t = threadIdx.x; t < R * M; t += NT) {
-            const int row = t / M, e = t - row * M, q = e / nb, idx = e - q * nb, k = idx % L;
-            // sum_p in[idx + p nb] w^{p (k step + q nb)}
-            const int inc = (k * step + q * nb) % M;
-            cplx s = in[row * P + fpad(idx)];
-            int w = 0;
-            for (int p = 1; p < r; p++) {
-                w += inc;
-                if (w >= M) w -= M;
-                s = s + cmul(in[row * P + fpad(idx + p * nb)], root[w]);
-            }
-            out[row * P + fpad((idx - k) * r + k + q * L)] = s;
+        *lo = x + y;
+        *hi = x - y;
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < R * nb * (h + 1); t += NT) {
+        const int u = small_div(t, inb), idx = t - u * nb, row = small_div(u, ih1), q = u - row * (h + 1);
+        const int k = idx - L * small_div(idx, il);
+        const cplx *x = in + row * P;
+        cplx c = x[fpad(idx)], f = {0, 0};
+        int m = 0;
+#pragma unroll 3
+        for (int p = 1; p <= h; p++) {
+            m += q;
+            if (m >= r) m -= r;
+            const cplx w = rt[m], a = x[fpad(idx + p * nb)], b = x[fpad(idx + (r - p) * nb)];
+            c = {fmav(w.x, a.x, c.x), fmav(w.x, a.y, c.y)};
+            f = {fmav(w.y, b.x, f.x), fmav(w.y, b.y, f.y)};  // minus the sine sum
         }
+        cplx *o = out + row * P;
+        const int e = (idx - k) * r + k;
+        o[fpad(e + q * L)] = {c.x - f.y, c.y + f.x};
+        if (q > 0) o[fpad(e + (r - q) * L)] = {c.x + f.y, c.y - f.x};
     }
 }
 
@@ -238,11 +271,17 @@ __device__ __forceinline__ static cplx *transform_rows(const FourierArgs &a, cpl
         int L = 1;
         for (int s = 0; s < a.nst; s++) {
             const int r = a.radix[s];
-            if (r == 4) stage_any<4, R>(in, out, tw, root, a.M, L, r);
-            else if (r == 2) stage_any<2, R>(in, out, tw, root, a.M, L, r);
-            else if (r == 3) stage_any<3, R>(in, out, tw, root, a.M, L, r);
-            else if (r == 5) stage_any<5, R>(in, out, tw, root, a.M, L, r);
-            else stage_any<0, R>(in, out, tw, root, a.M, L, r);
+            if (r == 8) stage_any<8, R>(in, out, tw, a.M, L);
+            else if (r == 4) stage_any<4, R>(in, out, tw, a.M, L);
+            else if (r == 2) stage_any<2, R>(in, out, tw, a.M, L);
+            else if (r == 3) stage_any<3, R>(in, out, tw, a.M, L);
+            else if (r == 5) stage_any<5, R>(in, out, tw, a.M, L);
+            else {
+                cplx *rt = buf + 2 * R * fpad(a.M);
+                for (int m = threadIdx.x; m < r; m += kRowThreads * R) rt[m] = root[m * (a.M / r)];
+                // stage_prime's own barrier lies between these stores and their use
+                stage_prime<R>(in, out, tw, rt, a.M, L, r);
+            }
             __syncthreads();
             cplx *t = in;
             in = out;
@@ -664,7 +703,20 @@ static bool fixed_length(int M) { return M == 128 || M == 256 || M == 512 || M =
 
 // rows per workgroup of a grid's own launches
 static int row_group(int M, int N) { return fixed_length(M) && M >= 512 && M <= 2048 && N >= 4 * 255 ? 4 : 2; }
-static size_t row_lds(int M, int R) { return (size_t)(fixed_length(M) ? 1 : 2) * R * fpad(M) * sizeof(cplx); }
+// the largest prime factor from 7 on (0: none)
+static int large_prime(int M) {
+    for (int r : {2, 3, 5})
+        while (M % r == 0) M /= r;
+    int big = M > 1 ? M : 0;
+    for (int r = 7; M > 1; r += 2)
+        for (; M % r == 0; M /= r) big = r;
+    return big;
+}
+// the rows (twice for a transform that is not in place) and a prime's roots
+static size_t row_lds(int M, int R) {
+    if (fixed_length(M)) return (size_t)R * fpad(M) * sizeof(cplx);
+    return (size_t)(2 * R * fpad(M) + large_prime(M)) * sizeof(cplx);
+}
 size_t fourier_row_lds(int M) { return row_lds(M, 2); }
 
 // rows per thread and waves per part of a mode: eight rows a thread, fewer
@@ -848,12 +900,12 @@ bool fourier_setup(const double *s40, const double *w40, int M, int N, FourierAr
             a.radix[a.nst++] = fixed_radix(left);
             left /= fixed_radix(left);
         }
-    for (int r : {4, 2, 3, 5})
-        while (left % r == 0) {
-            a.radix[a.nst++] = r;
-            left /= r;
-        }
-    for (int r = 7; left > 1; r += 2)
+    // the primes first: the first stage has no twiddles
+    for (int big = large_prime(left); big >= 7; big = large_prime(left)) {
+        a.radix[a.nst++] = big;
+        left /= big;
+    }
+    for (int r : {8, 4, 2, 3, 5})
         while (left % r == 0) {
             a.radix[a.nst++] = r;
             left /= r;

@@ -73,6 +73,13 @@ def test_direct_solve_equals_dense_solve(m, n):
     assert differ(z, zd) <= floor * np.linalg.norm(zd)
 
 
+# row lengths with prime stages (alone, two of a kind, two kinds, before
+# others) and with a stage of eight
+@pytest.mark.parametrize("m,n", [(7, 9), (49, 7), (77, 6), (38, 14), (57, 8), (40, 10), (56, 9)])
+def test_row_transform_of_any_length(m, n):
+    test_direct_solve_equals_dense_solve(m, n)
+
+
 # rows n - 1 at both sides of 128, 256, 512 (rows per thread, waves), widths
 # with each fixed length and with the general transform
 @pytest.mark.parametrize("m,n", [(128, 129), (256, 130), (128, 257), (144, 258), (512, 100), (240, 300), (96, 513),
