@@ -990,66 +990,80 @@ template <int KIND> struct LvlConstSrc {
 
 // Galerkin coarse block row at coarse node (I,J): sum over fine nodes f
 // with weight P(f,(I,J)) of P(f,.)^T A(f,g) P(g,.), then the inverse of cc.
-// Returns -1 when every fine row used was an interior row, -2 when every
-// one was an outside row, 0 otherwise.
+// One wavefront: its lanes fetch the 81 entries A(f,g) of the nine rows at
+// once, then lane 4 blk + r forms component r of block blk, its sum in the
+// order of the entries; the result is in T.o.  (A thread that did all of it
+// was a chain of 81 loads: 94 us a level, 39 us for one shared stencil.)
+// The weights are powers of two, so the order of their products is free.
+struct RapTeam {
+    double A[81][4];            // P(f,(I,J)) A(f,g)
+    double wx[5][3], wy[5][3];  // weight of parent I - 1 + c (J - 1 + c) of fine column 2 I - 2 + f (row)
+    double o[40];
+};
+// LDS written by some lanes of a wavefront and read by others
+__device__ __forceinline__ void rap_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
 template <class Src>
-__device__ int rap_node(const Src &src, int cm, int cn, int I, int J, double *o) {
-    const int fm = src.m(), fn = src.n();
-    double acc[36];
+__device__ void rap_node(const Src &src, int cm, int cn, int I, int J, RapTeam &T) {
+    const int fm = src.m(), fn = src.n(), lane = threadIdx.x & 63;
+    int c[2];
+    double w[2];
+    double A[2][4];
 #pragma unroll
-    for (int q = 0; q < 36; q++) acc[q] = 0;
-    bool all_interior = true, all_outside = true;
-    int c[2], cx[2], cy[2];
-    double w[2], wx[2], wy[2];
-    for (int fy = 2 * J - 1; fy <= 2 * J + 1; fy++) {
-        const double wfy = weight_of(parents(fy, fn, cn, c, w), c, w, J);
-        if (wfy == 0) continue;
-        for (int fx = 2 * I - 1; fx <= 2 * I + 1; fx++) {
-            const double wfx = weight_of(parents(fx, fm, cm, c, w), c, w, I);
-            if (wfx == 0) continue;
-            const int fij = fx + fm * fy;
-            all_interior = all_interior && src.interior(fij);
-            all_outside = all_outside && src.outside(fij);
-            for (int k = 0; k < 9; k++) {
-                const int gx = fx + k % 3 - 1, gy = fy + k / 3 - 1;
-                if (gx < 0 || gx >= fm || gy < 0 || gy >= fn) continue;
-                double A[4];
-                src.entry(fij, k, A);
-                if (A[0] == 0 && A[1] == 0 && A[2] == 0 && A[3] == 0) continue;
-                const int ny = parents(gy, fn, cn, cy, wy), nx = parents(gx, fm, cm, cx, wx);
-                // every index below is a compile-time one after unrolling,
-                // so acc stays in registers; each entry's sum runs in the
-                // order of the parents (q, then p)
+    for (int q = 0; q < 2; q++) {
+        const int e = lane + 64 * q, f = e / 9, k = e - 9 * f, fx = 2 * I - 1 + f % 3, fy = 2 * J - 1 + f / 3;
+        const int gx = fx + k % 3 - 1, gy = fy + k / 3 - 1;
+        const double wf = weight_of(parents(fx, fm, cm, c, w), c, w, I) * weight_of(parents(fy, fn, cn, c, w), c, w, J);
 #pragma unroll
-                for (int q = 0; q < 2; q++)
+        for (int r = 0; r < 4; r++) A[q][r] = 0;
+        if (e < 81 && wf != 0 && gx >= 0 && gx < fm && gy >= 0 && gy < fn) src.entry(fx + fm * fy, k, A[q]);
 #pragma unroll
-                    for (int p = 0; p < 2; p++) {
-                        if (q >= ny || p >= nx) continue;
-                        const int dI = cx[p] - I, dJ = cy[q] - J;
-                        if (dI < -1 || dI > 1 || dJ < -1 || dJ > 1) continue;
-                        const double ww = wfx * wfy * wx[p] * wy[q];
-                        const int blk = (dI + 1) + 3 * (dJ + 1);
-#pragma unroll
-                        for (int bb = 0; bb < 9; bb++)
-                            if (bb == blk)
-#pragma unroll
-                                for (int r = 0; r < 4; r++) acc[4 * bb + r] += ww * A[r];
-                    }
-            }
-        }
+        for (int r = 0; r < 4; r++) A[q][r] *= wf;
     }
 #pragma unroll
-    for (int q = 0; q < 36; q++) o[q] = acc[q];
-    const double a = acc[16], b = acc[17], cc = acc[18], d = acc[19];
-    const double idet = 1. / (a * d - b * cc);
-    o[36] = d * idet;
-    o[37] = -b * idet;
-    o[38] = -cc * idet;
-    o[39] = a * idet;
-    return all_interior ? -1 : (all_outside ? -2 : 0);
+    for (int r = 0; r < 4; r++) T.A[lane][r] = A[0][r];
+    if (lane < 17)
+#pragma unroll
+        for (int r = 0; r < 4; r++) T.A[64 + lane][r] = A[1][r];
+    if (lane < 15) T.wx[lane / 3][lane % 3] = weight_of(parents(2 * I - 2 + lane / 3, fm, cm, c, w), c, w, I - 1 + lane % 3);
+    else if (lane < 30) {
+        const int q = lane - 15;
+        T.wy[q / 3][q % 3] = weight_of(parents(2 * J - 2 + q / 3, fn, cn, c, w), c, w, J - 1 + q % 3);
+    }
+    rap_sync();
+    if (lane < 36) {
+        const int blk = lane >> 2, r = lane & 3, dI = blk % 3, dJ = blk / 3;
+        double acc = 0, ww[5][5];
+#pragma unroll
+        for (int y = 0; y < 5; y++)
+#pragma unroll
+            for (int x = 0; x < 5; x++) ww[y][x] = T.wx[x][dI] * T.wy[y][dJ];
+#pragma unroll
+        for (int f = 0; f < 9; f++)
+#pragma unroll
+            for (int k = 0; k < 9; k++) {
+                const double v = ww[f / 3 + k / 3][f % 3 + k % 3], a = T.A[9 * f + k][r];
+                acc += v * (v != 0 ? a : 0.0);
+            }
+        T.o[lane] = acc;
+    }
+    rap_sync();
+    if (lane == 0) {
+        const double a = T.o[16], b = T.o[17], cc = T.o[18], d = T.o[19];
+        const double idet = 1. / (a * d - b * cc);
+        T.o[36] = d * idet;
+        T.o[37] = -b * idet;
+        T.o[38] = -cc * idet;
+        T.o[39] = a * idet;
+    }
+    rap_sync();
 }
 
-// The kind rap_node returns, from the same fine rows, without the product
+// -1 when every fine row a coarse row uses is an interior row, -2 when every
+// one is an outside row, 0 otherwise
 template <class Src> __device__ int rap_kind(const Src &src, int cm, int cn, int I, int J) {
     const int fm = src.m(), fn = src.n();
     bool all_interior = true, all_outside = true;
@@ -1067,44 +1081,60 @@ template <class Src> __device__ int rap_kind(const Src &src, int cm, int cn, int
     return all_interior ? -1 : (all_outside ? -2 : 0);
 }
 
+// whether a coarse index's fine neighbours carry the prolongation weights of
+// an index away from the ends
+__device__ __forceinline__ bool regular(int I, int fm) { return I >= 1 && 2 * I + 2 + ((fm & 1) == 0) < fm; }
+
 // Every row's stencil: a row whose fine rows were all interior rows takes
 // the shared interior stencil (its product is not formed), one whose fine
-// rows were all outside rows takes the shared outside stencil if its
-// product equals it bit for bit (near the level's edges the prolongation
-// weights differ); the others store their own product.  The shared
-// stencils are formed first (rap_const_kernel).
-template <class Src>
+// rows were all outside rows takes the shared outside stencil, near the
+// level's edges, where the prolongation weights differ, if its product equals
+// it bit for bit; the others store their own product.  The shared stencils
+// are formed first (rap_const_kernel).  A workgroup takes TILE x TILE rows:
+// products are needed along the surface and the edges only, so its wavefronts
+// list the rows that do and share the list.  Large tiles on large levels,
+// where most hold no such row; small ones where most rows need a product and
+// few workgroups would have them all (kRapSmall).
+constexpr int kRapSmall = 65536;
+template <int TILE, class Src>
 __global__ void __launch_bounds__(kThreads) rap_kernel(Src src, BdLevel C, int shared) {
-    const int IJ = blockIdx.x * kThreads + threadIdx.x;
-    if (IJ >= C.m * C.n) return;
-    const int I = IJ % C.m, J = IJ / C.m, kind = shared ? rap_kind(src, C.m, C.n, I, J) : 0;
-    if (kind == -1) {  // the shared interior stencil, no product needed
-        C.type[IJ] = -1;
-        return;
+    __shared__ RapTeam teams[kThreads / 64];
+    __shared__ int list[TILE * TILE], count;
+    const int tid = threadIdx.x, lane = tid & 63;
+    RapTeam &T = teams[tid >> 6];
+    if (tid == 0) count = 0;
+    __syncthreads();
+    const int tx = (C.m + TILE - 1) / TILE, I0 = (blockIdx.x % tx) * TILE, J0 = (blockIdx.x / tx) * TILE;
+    if (tid < TILE * TILE) {
+        const int I = I0 + tid % TILE, J = J0 + tid / TILE;
+        if (I < C.m && J < C.n) {
+            const int IJ = I + C.m * J, kind = shared ? rap_kind(src, C.m, C.n, I, J) : 0;
+            if (kind == -1 || (kind == -2 && regular(I, src.m()) && regular(J, src.n()))) C.type[IJ] = kind;
+            else list[atomicAdd(&count, 1)] = kind == -2 ? ~IJ : IJ;
+        }
     }
-    double o[40];
-    (void)rap_node(src, C.m, C.n, I, J, o);
-    int type = 0;
-    if (kind == -2) {
-        bool same = true;
-        for (int q = 0; q < 40; q++) same = same && o[q] == C.Sc[40 + q];
-        type = same ? -2 : 0;
+    __syncthreads();
+    const int cnt = count;
+    for (int t = tid >> 6; t < cnt; t += kThreads / 64) {
+        const int v = list[t], IJ = v < 0 ? ~v : v;
+        rap_node(src, C.m, C.n, IJ % C.m, IJ / C.m, T);
+        const double o = lane < 40 ? T.o[lane] : 0;
+        const bool same = v < 0 && __all(lane >= 40 || o == C.Sc[40 + (lane < 40 ? lane : 0)]);
+        if (lane == 0) C.type[IJ] = same ? -2 : 0;
+        if (!same && lane < 40) C.S[40 * (size_t)IJ + lane] = o;
+        rap_sync();
     }
-    C.type[IJ] = type;
-    if (type < 0) return;
-    double *S = C.S + 40 * (size_t)IJ;
-    for (int q = 0; q < 40; q++) S[q] = o[q];
 }
 
-// a shared stencil of a level (KIND -1 interior, -2 outside): the product
-// at a node whose footprint lies away from the level's edges, every fine row
-// of the kind (same arithmetic as rap_kernel)
-template <int KIND, class Src>
-__global__ void rap_const_kernel(Src src, BdLevel C) {
-    if (threadIdx.x != 0) return;
-    double o[40];
-    (void)rap_node(src, C.m, C.n, 2, 2, o);
-    for (int q = 0; q < 40; q++) C.Sc[40 * (-1 - KIND) + q] = o[q];
+// the shared stencils of a level (interior, then outside): the products at a
+// node whose footprint lies away from the level's edges, every fine row of
+// the kind (same arithmetic as rap_kernel); a wavefront each
+template <class In, class Out>
+__global__ void __launch_bounds__(64) rap_const_kernel(In in, Out out, BdLevel C) {
+    __shared__ RapTeam T;
+    if (blockIdx.x == 0) rap_node(in, C.m, C.n, 2, 2, T);
+    else rap_node(out, C.m, C.n, 2, 2, T);
+    if (threadIdx.x < 40) C.Sc[40 * blockIdx.x + threadIdx.x] = T.o[threadIdx.x];
 }
 
 template <typename T> __global__ void __launch_bounds__(kThreads) fill_kernel(T *p, long n, T v) {
@@ -1406,27 +1436,22 @@ void BdSolver::free_all() {
 int BdSolver::setup(const BdTop &t, hipStream_t s) {
     top = t;
     for (int l = 0; l < nl; l++) {
-        const dim3 g = blocks((long)lv[l].m * lv[l].n);
         // the shared stencil needs a fine footprint of 7x7 nodes
         const bool cst = (l == 0 ? top_m : lv[l - 1].m) >= 7 && (l == 0 ? top_n : lv[l - 1].n) >= 7;
-        // the shared stencils first: rap_kernel compares outside rows with one
-        if (l == 0) {
-            if (cst) {
-                hipLaunchKernelGGL((rap_const_kernel<-1, TopConstSrc<-1>>), dim3(1), dim3(64), 0, s,
-                                   TopConstSrc<-1>{top}, lv[0]);
-                hipLaunchKernelGGL((rap_const_kernel<-2, TopConstSrc<-2>>), dim3(1), dim3(64), 0, s,
-                                   TopConstSrc<-2>{top}, lv[0]);
-            }
-            hipLaunchKernelGGL(rap_kernel<TopSrc>, g, dim3(kThreads), 0, s, TopSrc{top}, lv[0], cst ? 1 : 0);
-        } else {
-            if (cst) {
-                hipLaunchKernelGGL((rap_const_kernel<-1, LvlConstSrc<-1>>), dim3(1), dim3(64), 0, s,
-                                   LvlConstSrc<-1>{lv[l - 1]}, lv[l]);
-                hipLaunchKernelGGL((rap_const_kernel<-2, LvlConstSrc<-2>>), dim3(1), dim3(64), 0, s,
-                                   LvlConstSrc<-2>{lv[l - 1]}, lv[l]);
-            }
-            hipLaunchKernelGGL(rap_kernel<LvlSrc>, g, dim3(kThreads), 0, s, LvlSrc{lv[l - 1]}, lv[l], cst ? 1 : 0);
-        }
+        auto products = [&](auto src, auto in, auto out) {
+            typedef decltype(src) Src;
+            // the shared stencils first: rap_kernel compares outside rows with one
+            if (cst)
+                hipLaunchKernelGGL((rap_const_kernel<decltype(in), decltype(out)>), dim3(2), dim3(64), 0, s, in, out,
+                                   lv[l]);
+            const int tile = (long)lv[l].m * lv[l].n > kRapSmall ? 16 : 4;
+            const dim3 g(((lv[l].m + tile - 1) / tile) * ((lv[l].n + tile - 1) / tile));
+            if (tile == 16)
+                hipLaunchKernelGGL((rap_kernel<16, Src>), g, dim3(kThreads), 0, s, src, lv[l], cst ? 1 : 0);
+            else hipLaunchKernelGGL((rap_kernel<4, Src>), g, dim3(kThreads), 0, s, src, lv[l], cst ? 1 : 0);
+        };
+        if (l == 0) products(TopSrc{top}, TopConstSrc<-1>{top}, TopConstSrc<-2>{top});
+        else products(LvlSrc{lv[l - 1]}, LvlConstSrc<-1>{lv[l - 1]}, LvlConstSrc<-2>{lv[l - 1]});
         STZ_HIP(hipGetLastError());
     }
     if (mixed)
