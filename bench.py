@@ -9,34 +9,31 @@ to 1e-4 x the reference's residual threshold.  The timed steps are the
 shear_sim::step_forward_quasistatic: explicit ENO/STZ update, projection
 source, adaptive multigrid solve, stress correction and boundaries.
 
-The headline value is the mixed-precision form (FP32 V-cycles inside FP64
-iterative refinement); the plain FP64 form runs the same steps from the same
-state, and the two are compared field by field.
-
-Both forms use the reference's adaptive V-cycle count (tgmg::solve with a
-tgmg_predict, tgmg.in.cc:266-301: run the predicted number of cycles, test
-the residual, add cycles until it is below the threshold, then one extra
-cycle) with settings for this solver: first test after 1 cycle, decay 2,
-one more cycle per failed test (stz_mg_config.predict_unit), against the
-reference's compile-time 8 and 32 (tgmg_config.hh:26-37) and triangular
-steps (1, 2, 3, ... cycles between tests), which suit a CPU solver whose
-cycles each gain less and whose tests cost a residual sweep.  Here a test
-costs a norm launch and the next cycle is already enqueued while the host
-reads it.  Every solve still stops only below the same threshold: over the
-whole 5000-step run the cycle counts are the reference predictor's to
-0.1 %, and at the start of the run (the benchmark's window) the settings
-skip cycles the residual no longer needs.  The same steps with the
-reference's settings are timed as well and reported under
-`with_reference_predictor`.
+The headline value is the mixed-precision form; the plain FP64 form runs the
+same steps from the same state, and the two are compared field by field.  At
+this size both forms solve the projection's top level directly, in FP64
+(Fourier modes along x, block recurrences along y), so a solve counts no
+V-cycles: one direct solve, a residual test against the threshold, and a
+correction after a failed test.  On grids that keep V-cycles the mixed form
+runs them in FP32 inside FP64 iterative refinement, and both forms use the
+reference's adaptive cycle count (tgmg::solve with a tgmg_predict,
+tgmg.in.cc:266-301) with settings for this solver: first test after 1 cycle,
+decay 2, one more cycle per failed test (stz_mg_config.predict_unit), against
+the reference's compile-time 8 and 32 (tgmg_config.hh:26-37) and triangular
+steps.  The same steps with the reference's settings are timed as well and
+reported under `with_reference_predictor`.
 
 `roofline` is for the kernel that takes the largest share of a mixed step
-(top-level smoothing launches, advection), each timed live with HIP events
-on the simulation's own stream; its algorithmic bytes follow the scope
-table's per-node figures (24 B FP32 / 48 B FP64 per node and sweep, 4.5 words
-(18 B FP32, 36 B FP64) per fine node for a restriction or a prolongation, 32 B for the FP64 read-
-modify-write of vel += e, 136 B per cell for the advection).  `roofline_step`
-is the whole step: cells x bytes per cell-step (312 + 176 k + 80 r mixed,
-312 + 352 k FP64, for k V-cycles and r refinements per solve) / time.
+(advection; with V-cycles the top-level smoothing launches), each timed live
+with HIP events on the simulation's own stream; its algorithmic bytes follow
+the scope table's per-node figures (136 B per cell for the advection; 24 B
+FP32 / 48 B FP64 per node and sweep, 4.5 words (18 B FP32, 36 B FP64) per fine
+node for a restriction or a prolongation, 32 B for the FP64 read-modify-write
+of vel += e).  `roofline_step` is the whole step: cells x bytes per cell-step /
+time, with 392 bytes for a step that solves directly (advection 136, source
+and forward transform 64, modes 32, inverse transform 32, residual test 32,
+correction 96) and, with k V-cycles and r refinements per solve,
+312 + 176 k + 80 r (mixed) or 312 + 352 k (FP64).
 
 The CPU baseline is the reference's own code (oracle/_ref) timed on the
 host's cores on bounded samples of the same run (or the FP64 restatement
@@ -338,12 +335,13 @@ def main():
                                                 if k <= 3750), default=None),
             "final": final}
 
-    # step-level roofline from the scope table's bytes per cell-step
-    extra = 1
+    # step-level roofline from the bytes per cell-step; solves that count no
+    # cycles are direct, V-cycle solves count at least one and run one more
     step_roof = {}
     for form in ("fp64", "mixed"):
-        k = res[form]["cycles"] + extra
-        bps = 312 + 176 * k + 80 * k if form == "mixed" else 312 + 352 * k
+        k = res[form]["cycles"]
+        k = res[form]["cycles_run"] = k + 1 if k >= 1 else 0
+        bps = 392 if k == 0 else (312 + 176 * k + 80 * k if form == "mixed" else 312 + 352 * k)
         ach = cells * bps * args.steps / res[form]["elapsed"] / 1e9
         step_roof[form] = {"bytes_per_cell_step": bps, "cycles_per_solve_run": k, "achieved_GBps": ach,
                            "frac": ach / HBM_PEAK_GBS}
@@ -354,7 +352,7 @@ def main():
     for k, v in kern.items():
         log("bench: %-16s %8.2f us  %6.0f GB/s  %s" % (k, v["avg_launch_us"], v["achieved_GBps"], v["kernel"]))
     # the dominant kernel of the mixed step: largest time per step
-    per_step = {"mixed_top_pre": res["mixed"]["cycles"] + extra, "mixed_top_post": res["mixed"]["cycles"] + extra,
+    per_step = {"mixed_top_pre": res["mixed"]["cycles_run"], "mixed_top_post": res["mixed"]["cycles_run"],
                 "mixed_advect": 1}
     dom = max(per_step, key=lambda k: kern[k]["avg_launch_us"] * per_step[k])
     dk = kern[dom]
@@ -393,14 +391,15 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": "f32+f64",
+        "dtype": "f32+f64" if mixed["cycles_run"] else "f64",
         "data": "synthetic",
         "config": {
             "workload": "simple shear %dx%d, chi 600K+25K seeded (corr 3 cells), dt %.3g, steps %d..%d of 5000 "
                         "(t %.1f..%.1f), V(%d,%d), residual threshold %g x reference" %
                         (N, N, dt, args.warmup + 1, total, args.warmup * dt, total * dt, args.nu, args.nu,
                          args.tol),
-            "form": "FP32 V-cycles in FP64 iterative refinement",
+            "form": "FP32 V-cycles in FP64 iterative refinement" if mixed["cycles_run"] else
+                    "FP64 direct solve of the projection's top level",
             "fp64_value": fp64["value"],
             "fp64_ms_per_step": fp64["ms"],
             "mixed_over_fp64": mixed["value"] / fp64["value"],

@@ -30,3 +30,22 @@ def test_projection_over_level_sizes(N, form):
     print(N, form, "iterations", its, "difference %.1e" % err)
     assert its[0] <= 4 * its[1] + 20
     assert err < 1e-7  # as test_projection_mixed_preconditioner
+
+
+# levels on both sides of 65536 rows (253, 261 and 262 nodes a side below the
+# top), where the Galerkin products' tiles change, with odd and even sides: a
+# wrong coarse row costs iterations, and those of a V-cycle do not depend on
+# the grid but for the surface's place in its cells
+@pytest.mark.parametrize("N", [520, 522])
+def test_coarse_products_on_large_levels(N):
+    its = []
+    for k in (504, N):
+        print("case bd products", k, flush=True)
+        g = bd_bench.setup(k)
+        g.projection_step(0.5)
+        info = g.last_solve()
+        assert info["status"] == 0 and info["residual"] <= info["tolerance"], info
+        its.append(info["iterations"])
+        g.close()
+    print(N, "iterations", its)
+    assert its[1] <= 1.5 * its[0] + 3
