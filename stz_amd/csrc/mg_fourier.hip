@@ -28,6 +28,11 @@
 //             transform, the two real signals' modes separated on the way out
 //   modes     one workgroup per mode, the column in LDS
 //   inverse   R rows per workgroup, back to (u, v)
+// Each is bound by its memory passes and, in front of them, by one chain of
+// loads, barriers and stores: at 1024^2 19.4 (64 bytes a node, source
+// included), 13.3 and 10.7 us (32 bytes a node each; the copy rate gives 13,
+// 6.6 and 6.6), where the V-cycles of a step took 250 to 1200; at 2048^2 79, 38
+// and 38 us (53, 26 and 26).
 // The spectrum is kept mode-major, S[k][j] of 32 bytes (u, v' complex), a
 // column padded to four rows, so the mode launch reads and writes whole
 // columns and a row workgroup touches R * 32 contiguous bytes per mode.

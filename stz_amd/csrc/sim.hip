@@ -431,11 +431,11 @@ static bool all_tiled(const stz_sim *s) {
 // fourier_active):
 //   - any grid with a level the tiled launches do not cover, where a V-cycle
 //     is a launch per colour and level: 240 x 191 at the default settings
-//     2.4 ms a step with V-cycles, 0.067 ms with it;
+//     2.4 ms a step with V-cycles, 0.058 ms with it;
 //   - tiled grids of more than direct_nodes nodes (FP64 form) or four times
-//     that (mixed form).  It is faster there too (128^2 FP64 0.36 -> 0.043 ms
-//     a step, 1024^2 mixed in elastic loading 0.33 -> 0.12, 1024^2 FP64 in
-//     plastic flow 1.27 -> 0.14); the grids below the line keep the V-cycle
+//     that (mixed form).  It is faster there too (128^2 FP64 0.36 -> 0.037 ms
+//     a step, 1024^2 mixed in elastic loading 0.33 -> 0.11, 1024^2 FP64 in
+//     plastic flow 1.27 -> 0.12); the grids below the line keep the V-cycle
 //     and with it the adaptive cycle counts by which a batch of small members
 //     plans its launches;
 // unless direct_nodes = 0 asks for V-cycles down to the coarsest level

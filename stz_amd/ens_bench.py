@@ -63,10 +63,9 @@ def main():
     ap.add_argument("--serial-steps", type=int, default=3)
     ap.add_argument("--block", type=int, default=10, help="steps per block of one launch mode")
     ap.add_argument("--direct-nodes", type=int, default=None,
-                    help="largest coarse level solved exactly (stz_mg_config.direct_nodes); 0: none, the "
-                         "V-cycles go down to the workgroup coarse solve, which batches better than the "
-                         "exact level's mode inverses (default 0 in the mixed form; the FP64 form keeps "
-                         "the library's default, its 384-side members need their exact 48x49 level)")
+                    help="stz_mg_config.direct_nodes of the members (default: the library's, with which large "
+                         "members solve their top level directly: 3.33 ms/step for 256 mixed members; 0: V-cycles "
+                         "down to the workgroup coarse solve, 3.79 ms/step)")
     ap.add_argument("--tune-sweeps", action="store_true",
                     help="pick V(nu, nu), nu in 1..4, with the ensemble's sweep-count tuner after the warm-up")
     ap.add_argument("--one-mode", action="store_true",
@@ -76,8 +75,7 @@ def main():
     dt = problems.T_END / 5000
 
     t0 = time.perf_counter()
-    direct = args.direct_nodes if args.direct_nodes is not None else (0 if args.form == "mixed" else None)
-    ens, sides = build(args.members, args.seed, args.form, args.nu, args.tol, direct)
+    ens, sides = build(args.members, args.seed, args.form, args.nu, args.tol, args.direct_nodes)
     cells = sum(s * s for s in sides)
     print("ens_bench: %d members, %.2fM cells, set-up %.1f s" % (len(sides), cells / 1e6, time.perf_counter() - t0),
           file=sys.stderr, flush=True)
