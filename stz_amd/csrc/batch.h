@@ -173,8 +173,13 @@ int batch_fourier_modes(int N, const FourierEntry *E, const int *map, int total,
 int batch_resid_test(bool store, int sparse, const FourierEntry *E, const int *map, int total, const EnsState *S,
                      hipStream_t st);
 
-// the per-member V-cycle count (mg.hip): mode 0 starts a solve, mode 1
-// follows a cycle slot, mode 2 marks corrected members
+// the per-member cycle count (mg.hip): what the launch follows
+enum {
+    ENS_START,          // a step's first residuals: starts the solves
+    ENS_COUNT,          // a slot that cycled and solved directly
+    ENS_COUNT_CYCLES,   // a slot that cycled only
+    ENS_CORRECT         // the velocity corrections of members that are done
+};
 int batch_control(EnsState *S, const NormEntry *N, int nmem, EnsPredict P, int mode, hipStream_t st);
 
 }  // namespace stz

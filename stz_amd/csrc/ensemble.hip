@@ -533,7 +533,7 @@ int launch_head(stz_ensemble *e, int parity, double dt) {
     if (e->precision == STZ_PREC_MIXED) rc = batch_refine(R.E, R.map, R.ne, R.total, e->top_sparse, nullptr, st);
     else rc = batch_resid_norm(R.E, R.map, R.ne, R.total, nullptr, st);
     if (rc) return rc;
-    return batch_control(e->dst, e->norms, N, e->pred, 0, st);
+    return batch_control(e->dst, e->norms, N, e->pred, ENS_START, st);
 }
 
 template <typename T> int launch_vcycle(stz_ensemble *e, const VCyclePlan<T> &P) {
@@ -567,9 +567,10 @@ int launch_fourier(stz_ensemble *e, bool again) {
 }
 
 // What a slot does for the members that solve directly: the solve of the
-// first slot, nothing in the planned ones after it (they are done, and the
-// empty launches cost some 50 us a slot over 48 members), a correction in a
-// slot beyond the plan where one of them has failed its test.
+// first slot, nothing in the planned ones after it (as a rule they are done,
+// and the empty launches cost some 50 us a slot over 48 members; one that
+// failed its test waits, uncounted), a correction in a slot beyond the plan
+// where one of them has failed its test.
 enum { SLOT_FIRST, SLOT_CYCLE, SLOT_AGAIN };
 
 int launch_slot(stz_ensemble *e, int kind) {
@@ -585,14 +586,14 @@ int launch_slot(stz_ensemble *e, int kind) {
         if ((rc = launch_vcycle<double>(e, e->plan64))) return rc;
         if ((rc = batch_resid_norm(R.E, R.map, R.ne, R.total, e->dst, st))) return rc;
     }
-    return batch_control(e->dst, e->norms, e->nmem(), e->pred, 1, st);
+    return batch_control(e->dst, e->norms, e->nmem(), e->pred, kind == SLOT_CYCLE ? ENS_COUNT_CYCLES : ENS_COUNT, st);
 }
 
 int launch_tail(stz_ensemble *e, int parity, double dt) {
     int rc;
     const DevTable<CellEntry> &C = e->cells;
     if ((rc = batch_correct(C.E, C.map, C.ne, C.total, parity ^ 1, e->dst, dt, e->stream))) return rc;
-    return batch_control(e->dst, e->norms, e->nmem(), e->pred, 2, e->stream);
+    return batch_control(e->dst, e->norms, e->nmem(), e->pred, ENS_CORRECT, e->stream);
 }
 
 // capture fn() on the ensemble's stream into an executable graph

@@ -986,19 +986,23 @@ __device__ static void ens_resolve_direct(EnsState &st, double acc, const EnsPre
     st.status = isnan(acc) ? STZ_ERR_NAN : STZ_OK;
 }
 
-// one workgroup per member: mode 0 starts the solve from the residual of the
-// step's first evaluation, mode 1 counts the slot's cycle of every member
-// that ran it and tests its residual, mode 2 marks members corrected
+// one workgroup per member: ENS_START starts the solve from the residual of
+// the step's first evaluation, ENS_COUNT counts the slot's cycle of every
+// member that ran it and tests its residual, ENS_COUNT_CYCLES the same in a
+// slot without direct solves, whose active direct members wait with their
+// failed test as it is for a slot that corrects them, ENS_CORRECT marks
+// members corrected
 __global__ void __launch_bounds__(256) control_batch_kernel(EnsState *S, const NormEntry *N, EnsPredict P,
                                                             int mode) {
     const NormEntry &x = N[blockIdx.x];
     EnsState &st = S[x.member];
-    if (mode == 2) {
+    if (mode == ENS_CORRECT) {
         if (threadIdx.x == 0 && st.phase == ENS_DONE) st.phase = ENS_CORRECTED;
         return;
     }
-    if (mode == 1 && !st.active) return;
-    if (st.direct && mode == 0) {
+    if (mode != ENS_START && !st.active) return;
+    if (st.direct && mode == ENS_COUNT_CYCLES) return;
+    if (st.direct && mode == ENS_START) {
         if (threadIdx.x == 0) {
             st.n = st.k = st.remaining = st.cycles_run = 0;
             st.phase = ENS_FIRST;
@@ -1015,7 +1019,7 @@ __global__ void __launch_bounds__(256) control_batch_kernel(EnsState *S, const N
         ens_resolve_direct(st, sum / st.denom, P);
         return;
     }
-    if (mode == 0) {
+    if (mode == ENS_START) {
         st.n = st.lim / P.mult;
         st.k = 0;
         st.remaining = st.n;

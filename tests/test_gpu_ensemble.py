@@ -178,6 +178,51 @@ def test_failed_solve_leaves_member_as_single_does():
     ens.close()
 
 
+@pytest.mark.parametrize("graphs", [True, False])
+@pytest.mark.parametrize("form,sizes", [("mixed", [256, 64]), ("fp64", [128, 64])])
+def test_failed_first_test_of_a_direct_member(form, sizes, graphs):
+    """member 0 solves directly, member 1 by V-cycles, several slots planned.
+    The threshold lies between the residual of member 0's first solve and that
+    of a corrected one, so that its first test fails in the first of the
+    planned slots: one correction, counted once, as in its single simulation.
+    Then a threshold that neither meets, which ends at the predictor's limit
+    after as many corrections."""
+    print("case ensemble direct member fails its first test", form, graphs, flush=True)
+    ens, singles = setup(form, sizes=sizes)
+    ens.use_graphs(graphs)
+    probe = ShearSim(simple_shear(sizes[0], u_bdry=2e-3), form)
+    probe.set_fields(singles[0].get_fields())
+    probe.set_vel(singles[0].get_vel())
+    probe.time = singles[0].time
+    probe.set_mg_config(nu1=2, nu2=2, tol_mult=1e-40, predict_init=1, predict_max_iters=1)
+    with pytest.raises(StzError):
+        probe.step_forward_quasistatic(0.5, 1)
+    first = probe.last_solve()
+    assert first["total_cycles"] == 1, first
+    probe.close()
+    # a correction brings the residual down to a third or less
+    tol_mult = 1e-40 * 0.7 * first["residual"] / first["tolerance"]
+    for g in [ens] + singles:
+        g.set_mg_config(tol_mult=tol_mult)
+        g.step_forward_quasistatic(0.5, 1)
+    print(form, [g.last_solve() for g in singles], ens.stats())
+    assert singles[0].last_solve()["cycles"] == 1 and singles[0].last_solve()["total_cycles"] == 2
+    assert singles[1].last_solve()["cycles"] > 2
+    assert_same(ens, singles, "corrected")
+    for g in [ens] + singles:
+        g.set_mg_config(tol_mult=1e-2)
+        g.step_forward_quasistatic(0.5, 2)
+    assert_same(ens, singles, "the next steps")
+    for g in [ens] + singles:
+        g.set_mg_config(tol_mult=1e-40, predict_max_iters=20)
+        with pytest.raises(StzError) as e:
+            g.step_forward_quasistatic(0.5, 1)
+        assert e.value.code == 3
+    assert singles[0].last_solve()["cycles"] > 8
+    assert_same(ens, singles, "not converged")
+    ens.close()
+
+
 def test_member_matches_reference_fixture():
     """member 0 from the reference's rand64 fixture, beside random members"""
     fx = load_fixture("rand64")
