@@ -723,6 +723,8 @@ static size_t row_lds(int M, int R) {
     return (size_t)(2 * R * fpad(M) + large_prime(M)) * sizeof(cplx);
 }
 size_t fourier_row_lds(int M) { return row_lds(M, 2); }
+// the most a row launch of any length takes (fourier_fits)
+constexpr size_t kMaxRowLds = 152 * 1024;
 
 // rows per thread and waves per part of a mode: eight rows a thread, fewer
 // where one wave then covers the column
@@ -735,7 +737,7 @@ size_t fourier_mode_lds(int N) {
 
 bool fourier_fits(int M, int n) {
     const int N = n - 2;  // n node rows, walls included
-    return M >= 4 && M <= 4096 && N >= 1 && N <= 4096 && fourier_row_lds(M) <= 152 * 1024;
+    return M >= 4 && M <= 4096 && N >= 1 && N <= 4096 && fourier_row_lds(M) <= kMaxRowLds;
 }
 
 // f(integral_constant) of the row kernels' compile-time length (0: any)
@@ -777,18 +779,22 @@ template <int MT, typename F> static int with_rows(int M, int N, F f) {
     return f(std::integral_constant<int, 2>());
 }
 
-// raise the LDS limit of the kernels a grid uses (once per operator set-up)
+// Raise the LDS limit of the kernels a grid uses (once per operator set-up).
+// The limit belongs to the kernel, not to a grid: a kernel of one length or
+// one column variant always takes the same, the general-length ones get the
+// most that any length takes, so that no grid lowers it for another.
 int fourier_set_lds_limit(const FourierArgs &a) {
     const size_t ml = fourier_mode_lds(a.N);
     const int e = with_length(a.M, [&](auto mt) {
         constexpr int MT = decltype(mt)::value;
+        const size_t bl = MT > 0 ? fourier_row_lds(a.M) : kMaxRowLds;
         int r;
-        if ((r = allow_lds(fourier_forward_batch_kernel<MT>, fourier_row_lds(a.M))) ||
-            (r = allow_lds(fourier_inverse_batch_kernel<MT>, fourier_row_lds(a.M))))
+        if ((r = allow_lds(fourier_forward_batch_kernel<MT>, bl)) ||
+            (r = allow_lds(fourier_inverse_batch_kernel<MT>, bl)))
             return r;
         return with_rows<MT>(a.M, a.N, [&](auto rr) {
             constexpr int R = decltype(rr)::value;
-            const size_t rl = row_lds(a.M, R);
+            const size_t rl = MT > 0 ? row_lds(a.M, R) : kMaxRowLds;
             int q;
             if ((q = allow_lds(fourier_forward_kernel<MT, R>, rl)) || (q = allow_lds(fourier_source_kernel<MT, R>, rl)))
                 return q;

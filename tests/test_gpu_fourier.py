@@ -133,6 +133,32 @@ def test_corrections_and_failure():
     g.close()
 
 
+def test_general_lengths_of_different_sizes_in_one_process():
+    """the general-length kernels take 72 bytes of LDS a column: 2160 is the
+    widest that fits, and a narrower grid that also needs a raised limit,
+    set up in between, must leave it in place"""
+    def new(m):
+        print("case fourier widths", m, flush=True)
+        g = ShearSim(simple_shear(m, 8), "fp64")
+        g.mg_setup(VISCDT)
+        g.mg_set_src(np.random.default_rng(m).normal(size=(9, m, 2)))
+        return g
+
+    def solve_again(g):
+        g.set_vel(np.zeros((9, g.m, 2)))
+        info = g.mg_solve()
+        assert info["status"] == 0 and info["total_cycles"] == 1, info
+        return g.get_vel()
+
+    wide = new(2160)
+    first = solve_again(wide)
+    narrow = new(960)
+    solve_again(narrow)
+    assert np.array_equal(solve_again(wide), first)
+    wide.close()
+    narrow.close()
+
+
 def test_nan_source():
     print("case fourier nan", flush=True)
     p = simple_shear(240, 96)
