@@ -60,6 +60,7 @@ template <typename T> struct VCyclePlan {
     int ncoarse = 0;
     size_t lds = 0;
     DevTable<DirectEntry<T>> direct;   // members whose V-cycle stops at a direct level
+    int dsplit = 1;                    // workgroups per mode of their mode launch
     int *dinv_map = nullptr;           // and the workgroups of their inverse launch
     int dinv_total = 0;
     size_t dlds = 0;
@@ -243,7 +244,7 @@ int build_plan(stz_ensemble *e, VCyclePlan<T> &P, DevMG<T> stz_sim::*mgp, bool t
             de.b = A.lv[A.ld].b;
             de.z = A.lv[A.ld].z;
             direct.push_back(de);
-            dwgs.push_back(direct_mode_workgroups(de.M, de.Nn));
+            dwgs.push_back(de.M / 2 + 1);
             iwgs.push_back(direct_inverse_workgroups(de.M, de.Nn));
             dlds = std::max(dlds, direct_lds_bytes(de.M, de.Nn));
             continue;
@@ -327,6 +328,10 @@ int build_plan(stz_ensemble *e, VCyclePlan<T> &P, DevMG<T> stz_sim::*mgp, bool t
         return STZ_ERR_STATE;
     }
     if (!direct.empty()) {
+        int modes = 0;
+        for (int w : dwgs) modes += w;
+        P.dsplit = direct_mode_split(modes);
+        for (int &w : dwgs) w *= P.dsplit;
         if ((rc = make_table(e, direct, dwgs, P.direct))) return rc;
         if ((rc = make_map(e, iwgs, &P.dinv_map, &P.dinv_total))) return rc;
         P.dlds = dlds;
@@ -542,7 +547,8 @@ template <typename T> int launch_vcycle(stz_ensemble *e, const VCyclePlan<T> &P)
         if ((rc = batch_tile<T>(l.key, l.t.E, l.t.map, l.t.ne, l.t.total, e->dst, e->stream))) return rc;
     if ((rc = batch_coarse<T>(P.coarse, P.ncoarse, P.lds, e->dst, e->stream))) return rc;
     const DevTable<DirectEntry<T>> &D = P.direct;
-    if ((rc = batch_direct<T>(D.E, D.map, D.total, P.dinv_map, P.dinv_total, D.ne, P.dlds, e->dst, e->stream)))
+    if ((rc = batch_direct<T>(D.E, D.map, D.total, P.dsplit, P.dinv_map, P.dinv_total, D.ne, P.dlds, e->dst,
+                              e->stream)))
         return rc;
     for (const TileLaunch<T> &l : P.up)
         if ((rc = batch_tile<T>(l.key, l.t.E, l.t.map, l.t.ne, l.t.total, e->dst, e->stream))) return rc;

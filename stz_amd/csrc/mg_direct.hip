@@ -79,9 +79,8 @@ bool direct_fits(int M, int Nn) {
 // mode launch body: row blocks rb0 .. rb1 - 1 of mode k; the level's source
 // is in T, everything else in FP64.  A row's result does not depend on which
 // blocks share a workgroup: one solve spreads a mode over kRowBlocks
-// workgroups, a batch, whose members fill the chip, gives each mode one and
-// stages and transforms the source once (20 members of sides 64 and 128: 39
-// -> 32 us a launch).
+// workgroups, a batch over as many as its launch has room for
+// (direct_mode_split).
 template <typename T>
 __device__ __forceinline__ static void direct_mode_body(int M, int Nn, double *__restrict__ D,
                                                         const T *__restrict__ b, int k, int rb0, int rb1) {
@@ -230,11 +229,12 @@ __global__ void __launch_bounds__(kInvThreads) direct_inverse_kernel(int M, int 
 // flag is clear return at once
 template <typename T>
 __global__ void __launch_bounds__(kModeThreads) direct_mode_batch_kernel(const DirectEntry<T> *E, const int *map,
-                                                                         int ne, const EnsState *St) {
+                                                                         int split, const EnsState *St) {
     const int2 el = batch_slot(map, blockIdx.x);
     const DirectEntry<T> &x = E[el.x];
     if (St && !St[x.member].active) return;
-    direct_mode_body(x.M, x.Nn, x.D, x.b, el.y, 0, kRowBlocks);
+    const int k = el.y / split, rb = el.y % split, each = kRowBlocks / split;
+    direct_mode_body(x.M, x.Nn, x.D, x.b, k, rb * each, (rb + 1) * each);
 }
 template <typename T>
 __global__ void __launch_bounds__(kInvThreads) direct_inverse_batch_kernel(const DirectEntry<T> *E, const int *map,
@@ -245,9 +245,19 @@ __global__ void __launch_bounds__(kInvThreads) direct_inverse_batch_kernel(const
     direct_inverse_body(x.M, x.Nn, x.D, x.z, el.y);
 }
 
-int direct_mode_workgroups(int M, int Nn) {
-    (void)Nn;
-    return M / 2 + 1;
+// Workgroups per mode (a divisor of kRowBlocks) of a batch's mode launch of
+// `modes` modes in all.  Each stages and transforms the whole source, which a
+// workgroup of its own for each row block repeats; on the other hand a few
+// modes leave most CUs idle and run their row blocks one after the other.
+// So the split stays within the workgroups that are resident at once (two a
+// CU, by LDS): a pass of four steps of 4, 8, 20 and 64 members of sides 64 and
+// 128 takes 3.20, 3.76, 5.19 and 11.5 ms; with one workgroup a mode 3.83, 4.03,
+// 5.16 and 11.4, with four 3.20, 4.09, 6.23 and 14.7.
+constexpr int kModeFill = 512;
+int direct_mode_split(int modes) {
+    int split = kRowBlocks;
+    while (split > 1 && modes * split > kModeFill) split /= 2;
+    return split;
 }
 int direct_inverse_workgroups(int M, int Nn) {
     (void)M;
@@ -276,11 +286,11 @@ template <typename T> int mg_direct_set_lds_limit(size_t bytes) {
 }
 
 template <typename T>
-int batch_direct(const DirectEntry<T> *E, const int *mode_map, int mode_total, const int *inv_map, int inv_total,
-                 int ne, size_t lds, const EnsState *St, hipStream_t st) {
+int batch_direct(const DirectEntry<T> *E, const int *mode_map, int mode_total, int split, const int *inv_map,
+                 int inv_total, int ne, size_t lds, const EnsState *St, hipStream_t st) {
     if (ne == 0) return STZ_OK;
-    hipLaunchKernelGGL(direct_mode_batch_kernel<T>, dim3(mode_total), dim3(kModeThreads), lds, st, E, mode_map, ne,
-                       St);
+    hipLaunchKernelGGL(direct_mode_batch_kernel<T>, dim3(mode_total), dim3(kModeThreads), lds, st, E, mode_map,
+                       split, St);
     hipLaunchKernelGGL(direct_inverse_batch_kernel<T>, dim3(inv_total), dim3(kInvThreads), 0, st, E, inv_map, ne,
                        St);
     STZ_HIP(hipGetLastError());
@@ -369,9 +379,9 @@ template int mg_direct_solve<double>(const LevelArgs<double> &, double *, hipStr
 template int mg_direct_solve<float>(const LevelArgs<float> &, double *, hipStream_t);
 template int mg_direct_set_lds_limit<double>(size_t);
 template int mg_direct_set_lds_limit<float>(size_t);
-template int batch_direct<double>(const DirectEntry<double> *, const int *, int, const int *, int, int, size_t,
+template int batch_direct<double>(const DirectEntry<double> *, const int *, int, int, const int *, int, int, size_t,
                                   const EnsState *, hipStream_t);
-template int batch_direct<float>(const DirectEntry<float> *, const int *, int, const int *, int, int, size_t,
+template int batch_direct<float>(const DirectEntry<float> *, const int *, int, int, const int *, int, int, size_t,
                                  const EnsState *, hipStream_t);
 
 }  // namespace stz

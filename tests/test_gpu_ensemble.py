@@ -130,6 +130,18 @@ def test_large_members_equal_single_simulations(form):
     ens.close()
 
 
+# 33 modes a member: four, two and one workgroup a mode
+@pytest.mark.parametrize("members", [3, 7, 8])
+def test_exact_level_in_batches_of_any_size(members):
+    print("case ensemble exact level", members, flush=True)
+    ens, singles = setup("mixed", sizes=[128] * members)
+    for g in [ens] + singles:
+        g.step_forward_quasistatic(0.5, 2)
+    assert singles[0].last_solve()["refinements"] > 0  # V-cycles, down to the exact 64x65 level
+    assert_same(ens, singles, "2 steps")
+    ens.close()
+
+
 def test_extra_slots_and_table_rebuilds():
     """A member whose predictor underestimates (velocity reset to zero after
     its count has decayed) needs slots beyond the planned ones; a new dt, a
