@@ -75,6 +75,15 @@ def errs_of(fa, fb):
             "velocity": group_err(fa, fb, [0, 1]), "refmap": group_err(fa, fb, [7, 8])}
 
 
+def step_bytes(form, direct, cycles):
+    """(V-cycles run per solve, bytes per cell-step).  A V-cycle solve runs one
+    cycle more than it counts, also where the predictor has decayed to none."""
+    if direct:
+        return 0, 392
+    k = cycles + 1
+    return k, 312 + 176 * k + 80 * k if form == "mixed" else 312 + 352 * k
+
+
 def run_form(params, planes, form, dt, warmup, steps, nu, tol, stream, keep=(), predict=(1, 2, 1)):
     import torch
     from stz_amd import ShearSim
@@ -335,13 +344,11 @@ def main():
                                                 if k <= 3750), default=None),
             "final": final}
 
-    # step-level roofline from the bytes per cell-step; solves that count no
-    # cycles are direct, V-cycle solves count at least one and run one more
+    # step-level roofline from the bytes per cell-step
     step_roof = {}
     for form in ("fp64", "mixed"):
-        k = res[form]["cycles"]
-        k = res[form]["cycles_run"] = k + 1 if k >= 1 else 0
-        bps = 392 if k == 0 else (312 + 176 * k + 80 * k if form == "mixed" else 312 + 352 * k)
+        k, bps = step_bytes(form, res[form]["sim"].solves_directly, res[form]["cycles"])
+        res[form]["cycles_run"] = k
         ach = cells * bps * args.steps / res[form]["elapsed"] / 1e9
         step_roof[form] = {"bytes_per_cell_step": bps, "cycles_per_solve_run": k, "achieved_GBps": ach,
                            "frac": ach / HBM_PEAK_GBS}

@@ -222,6 +222,10 @@ int stz_sim_get_predictor(stz_sim *sim, int32_t *lim);
 int stz_sim_set_predictor(stz_sim *sim, int32_t lim);
 
 int stz_sim_last_solve(stz_sim *sim, stz_solve_info *info);
+/* 1 if the next solve goes through the direct solver of the top level, 0 if
+ * it runs V-cycles (see stz_mg_config.direct_nodes); STZ_ERR_STATE before the
+ * first step or stz_mg_setup.  (No counterpart in the reference.) */
+int stz_sim_solves_directly(stz_sim *sim, int32_t *direct);
 /* shear_sim::avg_iters -> tgmg_predict::avg_iters (tgmg_predict.hh:28-33):
  * mean V-cycles per solve since the last call; resets the counters. */
 int stz_sim_avg_iters(stz_sim *sim, double *avg);

@@ -123,6 +123,7 @@ _SIGS = {
     "stz_sim_get_mg_config": [C.c_void_p, C.POINTER(MGConfig)],
     "stz_sim_set_mg_config": [C.c_void_p, C.POINTER(MGConfig)],
     "stz_sim_last_solve": [C.c_void_p, C.POINTER(SolveInfo)],
+    "stz_sim_solves_directly": [C.c_void_p, C.POINTER(C.c_int32)],
     "stz_sim_avg_iters": [C.c_void_p, C.POINTER(C.c_double)],
     "stz_sim_mg_hierarchy": [C.c_void_p, C.c_int, C.POINTER(C.c_int), _ip],
     "stz_mg_setup": [C.c_void_p, C.c_double],

@@ -1100,6 +1100,13 @@ int stz_sim_last_solve(stz_sim *s, stz_solve_info *info) {
     return STZ_OK;
 }
 
+int stz_sim_solves_directly(stz_sim *s, int32_t *direct) {
+    if (!s || !direct) { set_error("null argument"); return STZ_ERR_ARG; }
+    if (s->viscdt_prev < 0) { set_error("the operator has not been set up"); return STZ_ERR_STATE; }
+    *direct = fourier_active(s) ? 1 : 0;
+    return STZ_OK;
+}
+
 int stz_sim_avg_iters(stz_sim *s, double *avg) {
     if (!s || !avg) { set_error("null argument"); return STZ_ERR_ARG; }
     // tgmg_predict.hh:28-33 (float division, counters reset)

@@ -189,6 +189,14 @@ class ShearSim:
         check(self._lib.stz_sim_last_solve(self._h, C.byref(info)))
         return {k: getattr(info, k) for k, _ in info._fields_}
 
+    @property
+    def solves_directly(self):
+        """whether the next solve goes through the direct solver of the top
+        level (False: V-cycles); the operator must have been set up"""
+        v = C.c_int32()
+        check(self._lib.stz_sim_solves_directly(self._h, C.byref(v)))
+        return bool(v.value)
+
     def avg_iters(self):
         a = C.c_double()
         check(self._lib.stz_sim_avg_iters(self._h, C.byref(a)))

@@ -159,6 +159,32 @@ def test_general_lengths_of_different_sizes_in_one_process():
     narrow.close()
 
 
+def test_which_solver_is_taken():
+    """the reported solver is the one that runs: V-cycle solves of a mixed form
+    evaluate FP64 residuals (refinements), also where they count no cycle"""
+    print("case fourier choice", flush=True)
+    for m, n, form, kw, direct in [(128, 128, "mixed", {}, False), (256, 128, "mixed", {}, True),
+                                   (256, 128, "mixed", {"direct_nodes": 0}, False),
+                                   (128, 128, "fp64", {}, True), (64, 64, "fp64", {}, False),
+                                   (128, 128, "fp64", {"predict_decay": 7}, False),
+                                   (128, 128, "fp64", {"predict_decay": 8}, True),
+                                   (44, 30, "fp64", {}, True), (44, 30, "fp64", {"predict_decay": 2}, False),
+                                   (256, 160, "fp64", {"predict_decay": 2}, True)]:
+        g = ShearSim(simple_shear(m, n), form)
+        with pytest.raises(StzError):
+            g.solves_directly
+        g.set_mg_config(predict_init=0, **kw)
+        g.mg_setup(VISCDT)
+        assert g.solves_directly == direct, (m, n, form, kw)
+        g.mg_set_src(np.zeros((n + 1, m, 2)))
+        g.set_vel(np.zeros((n + 1, m, 2)))
+        info = g.mg_solve()  # zero source and velocity: the first test passes
+        assert info["cycles"] == 0 and info["total_cycles"] == 1, info
+        if form == "mixed":
+            assert (info["refinements"] == 0) == direct, info
+        g.close()
+
+
 def test_nan_source():
     print("case fourier nan", flush=True)
     p = simple_shear(240, 96)
