@@ -131,7 +131,17 @@ typedef struct stz_mg_config {
                                     direct_nodes > 0 most grids need no
                                     V-cycle at all: the top level itself is
                                     solved directly (Fourier modes along x,
-                                    block recurrences along y, FP64) */
+                                    block recurrences along y, FP64).
+                                    V-cycles run on grids of at most
+                                    direct_nodes nodes (mixed form: four
+                                    times that) whose levels are all tiled
+                                    (1 leaves no such grid), on grids of up
+                                    to 32768 nodes with predict_decay < 8,
+                                    and where the direct launches do not fit
+                                    (over 4096 columns or 4098 node rows;
+                                    over 2160 columns, fewer with a large
+                                    prime factor, unless a power of two).
+                                    See stz_sim_solves_directly */
     int32_t predict_unit;        /* 0: after a failed test run k more cycles
                                     (k = 1, 2, 3, ...) before the next, as
                                     tgmg.in.cc:282-292 (default); 1: one more

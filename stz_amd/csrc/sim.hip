@@ -435,9 +435,12 @@ static bool all_tiled(const stz_sim *s) {
 //   - tiled grids of more than direct_nodes nodes (FP64 form) or four times
 //     that (mixed form).  It is faster there too (128^2 FP64 0.36 -> 0.037 ms
 //     a step, 1024^2 mixed in elastic loading 0.33 -> 0.11, 1024^2 FP64 in
-//     plastic flow 1.27 -> 0.12); the grids below the line keep the V-cycle
-//     and with it the adaptive cycle counts by which a batch of small members
-//     plans its launches;
+//     plastic flow 1.27 -> 0.12).  The line is not one of speed: below it a
+//     step takes 0.36 to 0.52 ms with V-cycles at the default predictor and
+//     0.040 directly (32^2, 64^2 FP64, 128^2 mixed).  These grids keep the
+//     solve they had, its iterates and its adaptive counts, which are what
+//     the fixtures of the V-cycle path and of the ensemble's state machine
+//     are stated in; direct_nodes = 1 takes them to the direct solve;
 // unless direct_nodes = 0 asks for V-cycles down to the coarsest level
 // (`kernels` chooses the kernels of V-cycles only).
 static int set_fourier(stz_sim *s) {
