@@ -65,7 +65,8 @@ template <typename T> int mg_direct_solve(const LevelArgs<T> &L, double *D, hipS
 size_t direct_lds_bytes(int M, int Nn);
 template <typename T> int mg_direct_set_lds_limit(size_t bytes);
 size_t direct_elems(int M, int Nn);
-bool direct_inverse(const double *S, int M, int Nn, std::vector<double> &D);
+// (returns null, or why the level has no such solve)
+const char *direct_inverse(const double *S, int M, int Nn, std::vector<double> &D);
 // whether the two-launch solve covers an M x Nn level (M even, 2 Nn and M
 // within the launches' fixed register and LDS tiles)
 bool direct_fits(int M, int Nn);

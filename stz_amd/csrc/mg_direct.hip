@@ -300,8 +300,9 @@ int batch_direct(const DirectEntry<T> *E, const int *mode_map, int mode_total, i
 // host: the device buffer of an x-invariant level with row stencils S (40
 // per row: blocks dl,dc,dr,cl,cc,cr,ul,uc,ur, then the centre inverse), M
 // nodes per row (even), Nn rows, in the layout above (Xh zero).  Returns
-// false if a mode's system is singular or the level lacks the symmetry above.
-bool direct_inverse(const double *S, int M, int Nn, std::vector<double> &D) {
+// null, or why there is none: a mode's system is singular, or the level lacks
+// the symmetry above.
+const char *direct_inverse(const double *S, int M, int Nn, std::vector<double> &D) {
     const int N2 = 2 * Nn, K = M / 2 + 1;
     D.assign(direct_elems(M, Nn), 0.0);
     std::vector<double> A((size_t)N2 * N2), I((size_t)N2 * N2);
@@ -313,7 +314,8 @@ bool direct_inverse(const double *S, int M, int Nn, std::vector<double> &D) {
                 const double *s = S + (size_t)j * 40 + 12 * jj;
                 const double l = s[r], m = s[4 + r], u = s[8 + r], top = std::fabs(S[(size_t)j * 40 + 16]);
                 const bool even = r == 0 || r == 3;
-                if (std::fabs(even ? l - u : l + u) > 1e-9 * top || (!even && std::fabs(m) > 1e-9 * top)) return false;
+                if (std::fabs(even ? l - u : l + u) > 1e-9 * top || (!even && std::fabs(m) > 1e-9 * top))
+                    return "is not symmetric under reflection in x";
             }
     for (int k = 0; k < K; k++) {
         const double th = 2 * pi * k / M, co = std::cos(th), si = std::sin(th);
@@ -340,7 +342,7 @@ bool direct_inverse(const double *S, int M, int Nn, std::vector<double> &D) {
             int piv = col;
             for (int r = col + 1; r < N2; r++)
                 if (std::fabs(A[(size_t)r * N2 + col]) > std::fabs(A[(size_t)piv * N2 + col])) piv = r;
-            if (A[(size_t)piv * N2 + col] == 0) return false;
+            if (A[(size_t)piv * N2 + col] == 0) return "is singular";
             if (piv != col)
                 for (int c = 0; c < N2; c++) {
                     std::swap(A[(size_t)piv * N2 + c], A[(size_t)col * N2 + c]);
@@ -372,7 +374,7 @@ bool direct_inverse(const double *S, int M, int Nn, std::vector<double> &D) {
         tw[2 * i] = std::cos(a);
         tw[2 * i + 1] = std::sin(a);
     }
-    return true;
+    return nullptr;
 }
 
 template int mg_direct_solve<double>(const LevelArgs<double> &, double *, hipStream_t);

@@ -408,8 +408,8 @@ int mg_ensure_direct(stz_sim *s) {
     if (!s->direct_pending) return STZ_OK;
     const int ld = s->mg64.args.ld;
     std::vector<double> G;
-    if (!direct_inverse(s->hl[ld].S.data(), s->hl[ld].m, s->hl[ld].n, G)) {
-        set_error("multigrid level %d (%d x %d) is singular", ld, s->hl[ld].m, s->hl[ld].n);
+    if (const char *why = direct_inverse(s->hl[ld].S.data(), s->hl[ld].m, s->hl[ld].n, G)) {
+        set_error("multigrid level %d (%d x %d) %s", ld, s->hl[ld].m, s->hl[ld].n, why);
         return STZ_ERR_STATE;
     }
     int e;
