@@ -58,6 +58,22 @@ def top_dense(p, viscdt):
     return A
 
 
+def top_product(p, viscdt, z):
+    """A z of the same operator without forming A, z[n + 1, m, 2]"""
+    xsp, ysp = p["m"] / (p["bx"] - p["ax"]), p["n"] / (p["by"] - p["ay"])
+    Kp = p["K"] + p["mu"] / 3.0
+    K, mu = Kp + p["mu"] + viscdt, p["mu"] + viscdt
+    x = xsp ** 2 * np.array([K, mu])
+    y = ysp ** 2 * np.array([mu, K])
+    l, r = np.roll(z, 1, 1), np.roll(z, -1, 1)
+    c, d, u = z[1:-1], z[:-2], z[2:]
+    a = np.empty_like(z)
+    a[1:-1] = x * (l[1:-1] + r[1:-1]) + y * (d + u) - 2 * (x + y) * c
+    a[1:-1] += 0.25 * Kp * xsp * ysp * (l[:-2] + r[2:] - r[:-2] - l[2:])[..., ::-1]
+    a[[0, -1]] = -8 * (x + y) * z[[0, -1]]
+    return a
+
+
 def stencil_from_dense(Ac, m, n):
     S = np.zeros((n, m, 9, 4))
     for j in range(n):

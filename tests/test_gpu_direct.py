@@ -48,17 +48,18 @@ def test_direct_level_solve_equals_dense_solve(form):
 
 
 @pytest.mark.parametrize("form", ["fp64", "mixed"])
-@pytest.mark.parametrize("size", [64, 256])
-def test_direct_and_workgroup_coarse_solves_agree(form, size):
+@pytest.mark.parametrize("size,nodes", [(64, 4200), (256, 70000)])  # more nodes than the top level: V-cycles
+def test_direct_and_workgroup_coarse_solves_agree(form, size, nodes):
     print("case direct vs workgroup", form, size, flush=True)
     p = simple_shear(size)
     viscdt = 0.1
     rng = np.random.default_rng(4)
     b = rng.normal(size=(size + 1, size, 2))
-    za, ia = solve(p, form, viscdt, b, 1e-14, 4200)
+    za, ia = solve(p, form, viscdt, b, 1e-14, nodes)
     zb, ib = solve(p, form, viscdt, b, 1e-14, 0)
     err = np.abs(za - zb).max() / np.abs(zb).max()
     print(form, size, "cycles direct %d workgroup %d, difference %.2e" % (ia["cycles"], ib["cycles"], err))
     assert ia["status"] == 0 and ib["status"] == 0
+    assert ia["cycles"] > 1 and ib["cycles"] > 1
     assert err < 1e-10
 

@@ -7,7 +7,7 @@ V-cycles.
   odd and even) and of the smallest heights.
 * Against the V-cycle solve (direct_nodes = 0) of the same system to a tight
   threshold at the edges of the mode kernel's row ranges and the row
-  transform's lengths.
+  transform's lengths; the largest of both by the residual alone.
 * A correction after a failed test, the failure of a solve whose threshold
   cannot be met, and NaN in the source.
 * Tiled and per-colour V-cycle kernels on a grid that solves directly unless
@@ -23,7 +23,7 @@ import math
 import numpy as np
 import pytest
 
-from dense import top_dense
+from dense import top_dense, top_product
 from stz_amd import ShearSim, StzError
 from stz_amd.problems import simple_shear
 
@@ -101,13 +101,46 @@ def test_direct_solve_equals_v_cycles(m, n):
     assert bound < 1e-7 * norm and err <= bound
 
 
-def test_corrections_and_failure():
+# the largest of everything: rows at both sides of 1024 and 2048 and the most
+# there are, each compile-time length on its own and in workgroups of four
+# rows (from 1020 interior rows on), the widest general length
+@pytest.mark.parametrize("m,n", [(8, 1025), (8, 1026), (8, 2049), (8, 2050), (8, 4097), (2048, 8), (4096, 8),
+                                 (2160, 8), (512, 1021), (1024, 1022), (2048, 1023), (4096, 1021)])
+def test_residual_of_the_largest_variants(m, n):
+    """the host's residual of the solution is at the rounding floor: 9 products
+    of the operator a row, and as much again for the solve"""
+    print("case fourier largest", m, n, flush=True)
+    p = simple_shear(m, n)
+    p["by"], p["ay"] = n / m, -n / m
+    b = np.random.default_rng(m + n).normal(size=(n + 1, m, 2))
+    z, info = solve(p, "fp64", b, 1.0)
+    assert info["status"] == 0 and info["total_cycles"] == 1, info
+    r = float(np.linalg.norm(b - top_product(p, VISCDT, z)))
+    floor = 2 * 9 * 2.2e-16 * diagonal(p, VISCDT) * float(np.linalg.norm(z))
+    print(m, n, "residual %.1e of the source, floor %.1e" % (r / np.linalg.norm(b), floor / np.linalg.norm(b)))
+    assert floor < 1e-3 * np.linalg.norm(b) and r <= floor
+
+
+# one more row, and a width whose rows and prime root table no longer fit
+@pytest.mark.parametrize("m,n,direct", [(24, 4097, True), (24, 4098, False), (2112, 64, True), (2240, 64, False)])
+def test_limits_of_the_direct_launches(m, n, direct):
+    print("case fourier limits", m, n, flush=True)
+    g = ShearSim(simple_shear(m, n), "fp64")
+    g.mg_setup(VISCDT)
+    assert g.solves_directly == direct
+    g.close()
+
+
+# a general length, a compile-time one, the same in the mixed form, and four
+# rows a workgroup
+@pytest.mark.parametrize("m,n,form", [(240, 96, "fp64"), (256, 96, "fp64"), (256, 96, "mixed"), (512, 1021, "fp64")])
+def test_corrections_and_failure(m, n, form):
     """a threshold under the rounding floor: corrections until the predictor's
     limit, then the failure V-cycles end in; the state is left uncorrected"""
-    print("case fourier failure", flush=True)
-    p = simple_shear(240, 96)
+    print("case fourier failure", m, n, form, flush=True)
+    p = simple_shear(m, n)
     rng = np.random.default_rng(2)
-    g = ShearSim(p, "fp64")
+    g = ShearSim(p, form)
     planes = np.zeros((10,) + g.plane_shape)
     planes[2:6] = 0.1 * rng.normal(size=(4,) + g.plane_shape)
     planes[6] = 0.03

@@ -71,12 +71,29 @@ def test_step_matches_reference_fixture(case):
         assert max(err) < 1e-10, (case, k, err)
 
 
-@pytest.mark.parametrize("case", ["rand64", "odd24x31"])
-def test_mixed_precision_matches_reference(case):
+@pytest.mark.parametrize("case", ["rand128", "odd24x31", "odd25x20"])
+def test_v_cycle_step_matches_reference_fixture(case):
+    """the fixtures whose grids solve directly, by V-cycles: tiled ones at
+    128^2, a launch per colour and level at the untiled widths"""
     fx = load_fixture(case)
-    print("case", case, flush=True)
+    print("case V-cycles", case, flush=True)
+    k = int(fx["steps"][-1])
+    g = gpu_from_fixture(fx)
+    g.set_mg_config(direct_nodes=0)
+    g.step_forward_quasistatic(float(fx["dt"]), k)
+    assert not g.solves_directly and g.last_solve()["cycles"] > 1, g.last_solve()
+    err = field_errors(g.get_fields(), fx["planes_%d" % k])
+    print(case, k, "step errors", ["%.1e" % e for e in err], "cycles", g.last_solve()["cycles"])
+    assert max(err) < 1e-10, (case, k, err)
+
+
+@pytest.mark.parametrize("case,kw", [("rand64", {}), ("odd24x31", {}), ("odd24x31", {"direct_nodes": 0})])
+def test_mixed_precision_matches_reference(case, kw):
+    fx = load_fixture(case)
+    print("case", case, kw, flush=True)
     k = int(fx["steps"][-1])
     g = gpu_from_fixture(fx, "mixed")
+    g.set_mg_config(**kw)
     g.step_forward_quasistatic(float(fx["dt"]), k)
     ge = group_errors(g.get_fields(), fx["planes_%d" % k])
     print(case, "mixed errors", {a: "%.1e" % b for a, b in ge.items()}, g.last_solve())
@@ -156,8 +173,9 @@ def test_nan_source_reports_failure():
 @pytest.mark.parametrize("form", ["fp64", "mixed"])
 def test_tiled_kernels_match_per_colour_kernels(form):
     """The LDS-tiled multi-sweep kernels apply the same smoother, transfers
-    and colour order as the one-kernel-per-colour path; a V-cycle from the
-    same state agrees to rounding (FMA contraction may differ)."""
+    and colour order as the one-kernel-per-colour path; a step from the same
+    state by V-cycles (direct_nodes = 0: the default solves this grid without
+    them) agrees to rounding (FMA contraction may differ)."""
     print("case tiled-vs-colour", form, flush=True)
     p = simple_shear(256, u_bdry=2e-3)
     from stategen import random_state
@@ -168,7 +186,7 @@ def test_tiled_kernels_match_per_colour_kernels(form):
         g.set_fields(planes)
         g.set_vel(vel)
         g.time = 1.2
-        g.set_mg_config(kernels=kernels, nu1=2, nu2=2)
+        g.set_mg_config(kernels=kernels, nu1=2, nu2=2, direct_nodes=0)
         g.advection_step(0.5)
         g.mg_setup(p["viscosity"] / 0.5)
         src = None
@@ -176,13 +194,15 @@ def test_tiled_kernels_match_per_colour_kernels(form):
         out.append((g.get_vel(), g.get_fields(), g.last_solve()))
     (va, fa, ia), (vb, fb, ib) = out
     print(form, ia, ib)
-    assert ia["cycles"] == ib["cycles"]
+    assert ia["cycles"] == ib["cycles"] > 1
     assert np.max(np.abs(va - vb)) <= 1e-12 * np.max(np.abs(vb))
     assert max(field_errors(fa, fb)) < 1e-12
 
 
-@pytest.mark.parametrize("form", ["fp64", "mixed"])
-def test_every_solve_meets_its_threshold(form):
+# the FP64 form solves this grid directly unless asked for V-cycles; the mixed
+# form runs V-cycles anyway
+@pytest.mark.parametrize("form,kw", [("fp64", {}), ("fp64", {"direct_nodes": 0}), ("mixed", {})])
+def test_every_solve_meets_its_threshold(form, kw):
     """A warm-started run whose predictor decays to zero cycles before the
     first convergence test (elastic loading from rest, as in the 1024^2
     benchmark): after every step the FP64 residual of the projection, taken
@@ -192,13 +212,13 @@ def test_every_solve_meets_its_threshold(form):
     previous step's value exactly)."""
     from stz_amd.initial import simple_shear_state
     from stz_amd.problems import T_END
-    print("case threshold", form, flush=True)
+    print("case threshold", form, kw, flush=True)
     p = simple_shear(128)
     g = ShearSim(p, form)
     g.set_fields(simple_shear_state(p, 600.0, 25.0, 3.0, seed=1))
     g.set_vel(np.zeros((p["n"] + 1, p["m"], 2)))
     g.time = 0.0
-    g.set_mg_config(nu1=2, nu2=2, tol_mult=1e-4)
+    g.set_mg_config(nu1=2, nu2=2, tol_mult=1e-4, **kw)
     zero_first, prev = 0, None
     for k in range(120):
         g.step_forward_quasistatic(T_END / 5000, 1)
