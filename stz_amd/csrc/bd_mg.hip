@@ -1086,7 +1086,9 @@ template <class Src> __device__ int rap_kind(const Src &src, int cm, int cn, int
 __device__ __forceinline__ bool regular(int I, int fm) { return I >= 1 && 2 * I + 2 + ((fm & 1) == 0) < fm; }
 
 // Every row's stencil: a row whose fine rows were all interior rows takes
-// the shared interior stencil (its product is not formed), one whose fine
+// the shared interior stencil (its product is not formed; next to the far edge
+// of an even-sided level, where the weights differ, it is not quite that
+// product, which the preconditioner bears), one whose fine
 // rows were all outside rows takes the shared outside stencil, near the
 // level's edges, where the prolongation weights differ, if its product equals
 // it bit for bit; the others store their own product.  The shared stencils
