@@ -227,14 +227,15 @@ __global__ void __launch_bounds__(kInvThreads) direct_inverse_kernel(int M, int 
 
 // the same over the members of an ensemble (batch.h); members whose slot
 // flag is clear return at once
-template <typename T>
+template <typename T, int SPLIT>
 __global__ void __launch_bounds__(kModeThreads) direct_mode_batch_kernel(const DirectEntry<T> *E, const int *map,
-                                                                         int split, const EnsState *St) {
+                                                                         const EnsState *St) {
     const int2 el = batch_slot(map, blockIdx.x);
     const DirectEntry<T> &x = E[el.x];
     if (St && !St[x.member].active) return;
-    const int k = el.y / split, rb = el.y % split, each = kRowBlocks / split;
-    direct_mode_body(x.M, x.Nn, x.D, x.b, k, rb * each, (rb + 1) * each);
+    constexpr int each = kRowBlocks / SPLIT;
+    const int k = el.y / SPLIT, rb = el.y % SPLIT * each;
+    direct_mode_body(x.M, x.Nn, x.D, x.b, k, rb, rb + each);
 }
 template <typename T>
 __global__ void __launch_bounds__(kInvThreads) direct_inverse_batch_kernel(const DirectEntry<T> *E, const int *map,
@@ -245,8 +246,8 @@ __global__ void __launch_bounds__(kInvThreads) direct_inverse_batch_kernel(const
     direct_inverse_body(x.M, x.Nn, x.D, x.z, el.y);
 }
 
-// Workgroups per mode (a divisor of kRowBlocks) of a batch's mode launch of
-// `modes` modes in all.  Each stages and transforms the whole source, which a
+// Workgroups per mode (4, 2 or 1) of a batch's mode launch of `modes` modes
+// in all.  Each stages and transforms the whole source, which a
 // workgroup of its own for each row block repeats; on the other hand a few
 // modes leave most CUs idle and run their row blocks one after the other.
 // So the split stays within the workgroups that are resident at once (two a
@@ -279,8 +280,10 @@ template <typename T> int mg_direct_set_lds_limit(size_t bytes) {
     if (bytes <= set) return STZ_OK;
     STZ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&direct_mode_kernel<T>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
-    STZ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&direct_mode_batch_kernel<T>),
-                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    for (auto kernel : {&direct_mode_batch_kernel<T, 1>, &direct_mode_batch_kernel<T, 2>,
+                        &direct_mode_batch_kernel<T, 4>})
+        STZ_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(kernel),
+                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
     set = bytes;
     return STZ_OK;
 }
@@ -289,8 +292,9 @@ template <typename T>
 int batch_direct(const DirectEntry<T> *E, const int *mode_map, int mode_total, int split, const int *inv_map,
                  int inv_total, int ne, size_t lds, const EnsState *St, hipStream_t st) {
     if (ne == 0) return STZ_OK;
-    hipLaunchKernelGGL(direct_mode_batch_kernel<T>, dim3(mode_total), dim3(kModeThreads), lds, st, E, mode_map,
-                       split, St);
+    auto *kernel = split == 4 ? &direct_mode_batch_kernel<T, 4>
+                              : (split == 2 ? &direct_mode_batch_kernel<T, 2> : &direct_mode_batch_kernel<T, 1>);
+    hipLaunchKernelGGL(kernel, dim3(mode_total), dim3(kModeThreads), lds, st, E, mode_map, St);
     hipLaunchKernelGGL(direct_inverse_batch_kernel<T>, dim3(inv_total), dim3(kInvThreads), 0, st, E, inv_map, ne,
                        St);
     STZ_HIP(hipGetLastError());
